@@ -85,7 +85,10 @@ enum rcm_param {
   RCM_PARAM_TIMEOUT_MS = 2,  /* device watchdog, default 20000 */
   RCM_PARAM_SORT = 3,        /* 0 auto, 1 LDS radix sort, 2 segment-rank sort */
   RCM_PARAM_DIGIT_BITS = 4,  /* radix digit width of the current variant (read-only: set the variant) */
-  RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit):
+  RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit). Until it is set (and while
+                                WORKERS, SORT, STRICT, PROFILE, CLAIM_FILTER and BATCH_CAP keep their defaults),
+                                matrices of up to 65,536 rows (in a large set or a serving lane more), each of at
+                                most 64 entries, are ordered by one workgroup each, whatever the variant:
                                 0 = 256 threads, 2048 adjacency slots, 256 parents, 4-bit digits (serving
                                     lanes)
                                 1 = 512 threads, 2048 slots, 256 parents, 4-bit digits (rcm_ctx default)

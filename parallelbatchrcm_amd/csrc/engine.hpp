@@ -63,6 +63,7 @@ struct alignas(128) Control {
   uint32_t nbatches;  // batch records used by the finished run
   uint32_t placed;    // nodes placed by the finished run
   uint32_t diag[9];   // first error: site, batch, begin, end, slots, offset, count, first child id, children
+  int32_t start, sweeps, passes;  // one-workgroup engine: start used, start-search sweeps, passes over the matrix
 };
 static_assert(offsetof(Control, progress) == 128 && offsetof(Control, done) == 256, "one line each");
 

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "engine_many.hpp"
+#include "engine_solo.hpp"
 #include "hip_exec.hpp"
 #include "level_cm.hpp"
 #include "rcm_gpu_batch_abi.h"
@@ -89,6 +90,24 @@ constexpr int kLevelThreads = 256;
 constexpr int kLevelDigit = 8;
 using GeoSmall = Var<0>::G;  // the many-matrix helpers' default
 constexpr int kDigit = 4;
+// The one-workgroup engine (engine_solo.hpp): 1024 threads over chunks of 4096 slots.
+using SoloG = SoloGeo<1024, 4096, kSoloMaxN>;
+// A matrix goes through it when it fits and has at most `limit` rows. One workgroup takes 0.5-0.7 entries per ns where
+// the levels are wide, the batch engine 11 over the whole GPU, but 5-10 us a level however narrow: start search and
+// order on MI355X, one workgroup against the batch engine, 0.84 against 3.3 ms for a 100 x 100 grid, 2.6 against 4.0
+// ms for a 40k-point geometric graph, but 3.9 against 3.5 ms for a 48^3 stencil (110k rows). Up to kSoloAlone rows one
+// workgroup wins whatever the shape; beyond, only beside enough other matrices: a set of `total` rows keeps the batch
+// engine busy for total / 11 entries' time, so a matrix of total / kSoloShare rows ends on its one workgroup before
+// the batch engine would have ended the set.
+constexpr int32_t kSoloAlone = 1 << 16;
+constexpr int64_t kSoloShare = 16;
+// In a serving lane the other lanes' groups are that company (a 48-request burst of up to 100k rows: 11.7 ms with one
+// workgroup for each, 23.6 ms with the larger ones left to the batch engine, 27.3 ms with all of them).
+constexpr int64_t kSoloLaneTotal = (int64_t)kSoloShare << 17;
+bool solo_fits(int32_t n, uint32_t maxrow, int64_t total) {
+  return n <= std::min<int64_t>(kSoloMaxN, std::max<int64_t>(kSoloAlone, total / kSoloShare)) &&
+         maxrow <= (uint32_t)kSoloMaxRow;
+}
 
 // lev: a CM run that also records BFS levels (a speculated start-search sweep); plain-BFS runs always do.
 template <int V>
@@ -286,6 +305,7 @@ struct rcm_ctx {
   int64_t variant = kDefaultCtxVariant;
   int64_t strict = 0;
   int64_t profile = 0;
+  bool engine_set = false;   // RCM_PARAM_VARIANT was set (or tuned): the batch engine runs every matrix
   int64_t batch_cap = 0;     // RCM_PARAM_BATCH_CAP: batch records a run may use (0 = n + 1, all it can need)
   int64_t speculate = kDefaultSpeculate;  // RCM_PARAM_SPECULATE
   uint64_t* prof = nullptr;  // kProfSlots words
@@ -391,11 +411,46 @@ int run_level(rcm_ctx* c, int32_t start, bool bfs) {
   return RCM_OK;
 }
 
+// Whether the loaded matrix goes through the one-workgroup engine: it fits, and no parameter of the batch engine was
+// chosen.
+bool ctx_solo(const rcm_ctx* c) {
+  return !c->engine_set && c->workers == 0 && !c->strict && !c->profile && c->sort_mode == 0 && c->batch_cap == 0 &&
+         c->claim_filter == kDefaultClaimFilter && solo_fits(c->n, c->maxdeg, c->n);
+}
+
+// One launch of the one-workgroup engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl.
+int ctx_run_solo(rcm_ctx* c, int32_t mode, int32_t start) {
+  const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
+  RCM_HIP(hipEventRecord(c->ev[0], c->stream));
+  hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
+                     (uint64_t)c->timeout_ms * 100000ull, c->ctl);
+  RCM_HIP(hipGetLastError());
+  RCM_HIP(hipEventRecord(c->ev[2], c->stream));
+  RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+  RCM_HIP(hipEventRecord(c->ev[3], c->stream));
+  const int rc = wait_stream(c, c->ev[3], c->timeout_ms + 10000);
+  if (rc) return rc;
+  float ms = 0.f;
+  RCM_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[2]));
+  const Control& h = *c->h_ctl;
+  c->timing.init_kernel_ms = 0.0;
+  c->timing.run_kernel_ms = ms;
+  c->timing.workers = 1;
+  c->timing.batches = (int32_t)h.nbatches;
+  c->timing.placed = (int32_t)h.placed;
+  c->timing.error_site = 0;
+  for (int i = 0; i < 8; ++i) c->timing.error_info[i] = 0;
+  if (h.error == ERR_TIMEOUT) return RCM_ETIMEOUT;
+  if ((int32_t)h.placed != c->n) return RCM_ENOTCONNECTED;
+  return RCM_OK;
+}
+
 // One engine run from `start` (CM order, or plain BFS order with levels when bfs; a CM run also records the
 // levels when `levels`).
 int run_engine(rcm_ctx* c, int32_t start, bool bfs, bool levels = false) {
   if (!c->rp) return RCM_ENOTLOADED;
   if (start < 0 || start >= c->n) return RCM_EINVAL;
+  if (!bfs && !levels && ctx_solo(c)) return ctx_run_solo(c, SOLO_RUN, start);
   if (c->variant == kLevelVariant) return run_level(c, start, bfs);
   RunArgs a{};
   a.row_ptr = c->rp;
@@ -587,6 +642,16 @@ struct rcm_batch {
   uint32_t* helpers = nullptr;  // count words: workgroups helping each matrix
   int32_t *blk_order = nullptr, *blk_active = nullptr;  // helper-kernel block maps of `order` / a sub-list
   int32_t nblk_order = 0;
+  // The loaded set split by engine: matrices for the one-workgroup engine, and the rest (with its block map), both
+  // largest first. Used while batch_solo() holds; otherwise every matrix is the batch engine's.
+  bool engine_set = false;  // a parameter of the batch engine was chosen
+  bool lane = false;        // a serving lane: its workgroup count is not a choice of engine
+  std::vector<int32_t> solo, rest;
+  int32_t *d_solo = nullptr, *d_rest = nullptr, *blk_rest = nullptr;
+  std::vector<int32_t> blk_rest_h;
+  int64_t rest_rows = 0;
+  uint32_t* solo_next = nullptr;
+  int solo_resident = 0;  // co-resident workgroups of the one-workgroup engine
   ManyControl* g = nullptr;
   // pinned host mirrors
   ManyControl* h_g = nullptr;  // the launch control of the last launch (its abort word: the watchdog fired)
@@ -621,7 +686,7 @@ int32_t build_blk(const rcm_batch* b, const int32_t* list, int32_t count, std::v
 // Byte layout of a loaded set in the arena: every buffer 256-byte aligned.
 struct BatchLayout {
   size_t rp, ci, perm, level, aux, qinfo, claim, bstat, brange, ctl, jobs, order, starts, active, tail, nnz,
-      scratch, helpers, blk_order, blk_active, g, total;
+      scratch, helpers, blk_order, blk_active, solo, rest, blk_rest, g, total;
 };
 BatchLayout batch_layout(size_t rp_end, size_t ci_end, size_t N, size_t C) {
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
@@ -648,7 +713,10 @@ BatchLayout batch_layout(size_t rp_end, size_t ci_end, size_t N, size_t C) {
   put(L.helpers, 4 * C);
   put(L.blk_order, 4 * (C + 1));
   put(L.blk_active, 4 * (C + 1));
-  put(L.g, sizeof(ManyControl));
+  put(L.solo, 4 * C);
+  put(L.rest, 4 * C);
+  put(L.blk_rest, 4 * (C + 1));
+  put(L.g, sizeof(ManyControl) + 256);  // and the one-workgroup launches' list position, on a line of its own
   L.total = o;
   return L;
 }
@@ -745,6 +813,29 @@ void enqueue_many(rcm_batch* b, const int32_t* d_list, const int32_t* d_blk, int
   ManyArgs mm = m;
   void* args[] = {&mm};
   (void)hipLaunchKernel(kern, dim3(batch_workers(b)), dim3(kVarThreads[b->variant]), args, 0, b->stream);
+}
+
+// Whether the set's small matrices go through the one-workgroup engine: no parameter of the batch engine was chosen.
+bool batch_solo(const rcm_batch* b) {
+  return !b->engine_set && (b->lane || b->workers == 0) && b->sort_mode == 0 && b->claim_filter == kDefaultClaimFilter &&
+         !b->solo.empty();
+}
+
+// The one-workgroup engine over the set's small matrices, one workgroup each at a time.
+void enqueue_solo(rcm_batch* b, int32_t mode) {
+  SoloManyArgs m{};
+  m.jobs = b->jobs;
+  m.list = b->d_solo;
+  m.starts = b->d_starts;
+  m.next = b->solo_next;
+  m.count = (int32_t)b->solo.size();
+  m.mode = mode;
+  m.speculate = (int32_t)b->speculate;
+  m.budget_ticks = (uint64_t)b->timeout_ms * 100000ull;
+  const int grid = std::max(1, std::min(m.count, b->workers > 0 ? std::min((int)b->workers, b->solo_resident)
+                                                                : b->solo_resident));
+  hipLaunchKernelGGL(k_solo_reset, dim3(1), dim3(64), 0, b->stream, m.next);
+  hipLaunchKernelGGL(k_solo_many<SoloG>, dim3((unsigned)grid), dim3(SoloG::T), 0, b->stream, m);
 }
 
 // Per-matrix status from the control blocks of the last launch (jobs listed in `order`). A matrix the launch
@@ -854,7 +945,7 @@ struct rcm_server {
 namespace {
 
 // One lane: reorder a group of requests with the lane's many-matrix context.
-bool solo_fits(const rcm_server* s, int lane, const ServerJob& j) {
+bool lane_solo_fits(const rcm_server* s, int lane, const ServerJob& j) {
   return s->solo[(size_t)lane] && j.n >= kServeLargeN && j.n <= kServeSoloN && j.nnz <= kServeSoloNnz;
 }
 
@@ -898,7 +989,7 @@ void run_solo(rcm_server* s, int lane, ServerJob& j) {
 }
 
 void run_group(rcm_server* s, int lane, std::vector<std::shared_ptr<ServerJob>>& grp) {
-  if (grp.size() == 1 && solo_fits(s, lane, *grp[0])) {
+  if (grp.size() == 1 && lane_solo_fits(s, lane, *grp[0])) {
     run_solo(s, lane, *grp[0]);
     return;
   }
@@ -1045,7 +1136,7 @@ void lane_loop(rcm_server* s, int lane) {
       const bool large = s->pending.front()->n >= kServeLargeN;
       const size_t share = (s->pending.size() + (size_t)s->lanes - 1) / (size_t)s->lanes;
       // a large request that fits the lane's single-matrix context is ordered alone through it
-      const size_t cap = solo_fits(s, lane, *s->pending.front())
+      const size_t cap = lane_solo_fits(s, lane, *s->pending.front())
                              ? 1
                              : std::min<size_t>((size_t)s->cfg.slots, std::max<size_t>(1, share));
       GroupSize gs;
@@ -1356,7 +1447,11 @@ int rcm_ctx_set_param(rcm_ctx* c, int param, int64_t v) {
     case RCM_PARAM_CLAIM_FILTER: if (v < 0 || v > 2) return RCM_EINVAL; c->claim_filter = v; return RCM_OK;
     case RCM_PARAM_DIGIT_BITS:  // part of the variant
       return v == (c->variant == kLevelVariant ? kLevelDigit : kVarDigit[c->variant]) ? RCM_OK : RCM_EINVAL;
-    case RCM_PARAM_VARIANT: if (v < 0 || v > kLevelVariant) return RCM_EINVAL; c->variant = v; return RCM_OK;
+    case RCM_PARAM_VARIANT:
+      if (v < 0 || v > kLevelVariant) return RCM_EINVAL;
+      c->variant = v;
+      c->engine_set = true;
+      return RCM_OK;
     case RCM_PARAM_STRICT: c->strict = v ? 1 : 0; return RCM_OK;
     case RCM_PARAM_PROFILE: if (v < 0 || v > 2) return RCM_EINVAL; c->profile = v; return RCM_OK;
     case RCM_PARAM_BATCH_CAP: if (v < 0) return RCM_EINVAL; c->batch_cap = v; return RCM_OK;
@@ -1470,6 +1565,12 @@ int rcm_ctx_find_start(rcm_ctx* c, int32_t* start_out, int32_t* iterations_out) 
   if (n == 1) {
     cur = 0;
     iters = 1;
+  } else if (ctx_solo(c)) {
+    c->have_perm = false;
+    const int rc = ctx_run_solo(c, SOLO_SEARCH, -1);
+    if (rc) return rc;
+    cur = c->h_ctl->start;
+    iters = c->h_ctl->sweeps;
   } else {
     uint32_t lastdist = 0;
     const int32_t w = std::min<int32_t>(32, n - 1);
@@ -1512,7 +1613,14 @@ int rcm_ctx_order(rcm_ctx* c, int32_t start_node, uint32_t flags, int32_t* start
   c->have_perm = false;
   int32_t cur = start_node, iters = 0, passes = 0;
   bool ordered = false;
-  if (start_node < 0 && n == 1) {
+  if (ctx_solo(c)) {
+    const int rc = ctx_run_solo(c, SOLO_ORDER, start_node);
+    if (rc) return rc;
+    cur = c->h_ctl->start;
+    iters = c->h_ctl->sweeps;
+    passes = c->h_ctl->passes;
+    ordered = true;
+  } else if (start_node < 0 && n == 1) {
     cur = 0;
     iters = 1;
   } else if (start_node < 0) {
@@ -1677,6 +1785,12 @@ int rcm_batch_create(int device, rcm_batch** out) {
          hipSuccess;
     b->max_res[v] = std::max(1, per_cu) * prop.multiProcessorCount;
   }
+  if (ok) {
+    int per_cu = 0;
+    ok = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<void*>(&k_solo_many<SoloG>), SoloG::T,
+                                                      0) == hipSuccess;
+    b->solo_resident = std::max(1, per_cu) * prop.multiProcessorCount;
+  }
   if (!ok) {
     rcm_batch_destroy(b);
     return RCM_EDEVICE;
@@ -1717,6 +1831,7 @@ int rcm_batch_set_param(rcm_batch* b, int param, int64_t v) {
     case RCM_PARAM_VARIANT:
       if (v < 0 || v >= kVariants) return RCM_EINVAL;
       b->variant = v;
+      b->engine_set = true;
       batch_drop_graphs(b);  // captured graphs hold the old launch parameters
       b->max_resident = b->max_res[v];
       return RCM_OK;
@@ -1776,7 +1891,13 @@ int rcm_batch_load(rcm_batch* b, int32_t count, const int32_t* n, const int64_t*
   b->helpers = reinterpret_cast<uint32_t*>(base + L.helpers);
   b->blk_order = reinterpret_cast<int32_t*>(base + L.blk_order);
   b->blk_active = reinterpret_cast<int32_t*>(base + L.blk_active);
+  b->d_solo = reinterpret_cast<int32_t*>(base + L.solo);
+  b->d_rest = reinterpret_cast<int32_t*>(base + L.rest);
+  b->blk_rest = reinterpret_cast<int32_t*>(base + L.blk_rest);
   b->g = reinterpret_cast<ManyControl*>(base + L.g);
+  b->solo_next = reinterpret_cast<uint32_t*>(base + L.g + 128);
+  b->solo.clear();
+  b->rest.clear();
   b->count = count;
   b->n.assign(n, n + count);
   b->nnz.assign(nnz, nnz + count);
@@ -1842,11 +1963,56 @@ int rcm_batch_load(rcm_batch* b, int32_t count, const int32_t* n, const int64_t*
   b->timing.total_n = tot;
   b->timing.total_nnz = totnnz;
   b->timing.load_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  if (rc) batch_reset(b);
-  return rc;
+  if (rc) {
+    batch_reset(b);
+    return rc;
+  }
+  b->rest_rows = 0;
+  for (int32_t k : b->order) {
+    if (solo_fits(n[k], b->maxrow[k], b->lane ? std::max(tot, kSoloLaneTotal) : tot)) {
+      b->solo.push_back(k);
+    } else {
+      b->rest.push_back(k);
+      b->rest_rows += n[k];
+    }
+  }
+  (void)build_blk(b, b->rest.data(), (int32_t)b->rest.size(), b->blk_rest_h);
+  if (!b->solo.empty())
+    RCM_HIP(hipMemcpyAsync(b->d_solo, b->solo.data(), b->solo.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                           b->stream));
+  if (!b->rest.empty()) {
+    RCM_HIP(hipMemcpyAsync(b->d_rest, b->rest.data(), b->rest.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                           b->stream));
+    RCM_HIP(hipMemcpyAsync(b->blk_rest, b->blk_rest_h.data(), b->blk_rest_h.size() * sizeof(int32_t),
+                           hipMemcpyHostToDevice, b->stream));
+  }
+  RCM_HIP(hipStreamSynchronize(b->stream));
+  b->timing.load_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+  return RCM_OK;
 }
 
 namespace {
+// One launch of the one-workgroup engine over the set's small matrices (SOLO_SEARCH or SOLO_ORDER), then back on the
+// host: starts, sweeps and status of each.
+int batch_solo_pass(rcm_batch* b, int32_t mode, const std::vector<int32_t>& given, int32_t* cur, int32_t* iters,
+                    int32_t* status) {
+  const int32_t C = b->count;
+  RCM_HIP(hipMemcpyAsync(b->d_starts, given.data(), (size_t)C * sizeof(int32_t), hipMemcpyHostToDevice, b->stream));
+  enqueue_solo(b, mode);
+  RCM_HIP(hipGetLastError());
+  RCM_HIP(hipMemcpyAsync(b->h_ctl, b->ctl, (size_t)C * sizeof(Control), hipMemcpyDeviceToHost, b->stream));
+  RCM_HIP(hipEventRecord(b->ev[3], b->stream));
+  const int wr = batch_wait(b, b->ev[3]);
+  if (wr) return wr;
+  *b->h_g = ManyControl{};  // the batch engine's abort word: not this launch's
+  (void)collect_status(b, b->solo.data(), (int32_t)b->solo.size(), status, nullptr);
+  for (int32_t k : b->solo) {
+    cur[k] = b->h_ctl[k].start;
+    iters[k] = b->h_ctl[k].sweeps;
+  }
+  return RCM_OK;
+}
+
 // One launch over `list` (plain-BFS sweeps when bfs, else CM runs, which record levels when `levels`) from
 // cur[], then back on the host: every control block, and for each listed matrix the last w = min(32, n-1)
 // queue entries (node, level, row length) at h_tail[i * 96]. Per-matrix status of the listed matrices goes to
@@ -1886,7 +2052,15 @@ int rcm_batch_find_start(rcm_batch* b, int32_t* start_out, int32_t* iterations_o
   const int32_t C = b->count;
   std::vector<int32_t> cur(C), iters(C, 0), active, status(C, RCM_OK);
   std::vector<uint32_t> lastdist(C, 0);
-  for (int32_t k : b->order) {
+  int sweeps = 0;
+  const bool solo = batch_solo(b);
+  if (solo) {
+    ++sweeps;
+    const int r = batch_solo_pass(b, SOLO_SEARCH, std::vector<int32_t>((size_t)C, -1), cur.data(), iters.data(),
+                                  status.data());
+    if (r) return r;
+  }
+  for (int32_t k : solo ? b->rest : b->order) {
     if (b->n[k] == 1) {
       cur[k] = 0;
       iters[k] = 1;
@@ -1895,7 +2069,6 @@ int rcm_batch_find_start(rcm_batch* b, int32_t* start_out, int32_t* iterations_o
       active.push_back(k);
     }
   }
-  int sweeps = 0;
   while (!active.empty()) {
     ++sweeps;
     const int r = batch_pass(b, active, cur, true, false, status.data());
@@ -1956,6 +2129,15 @@ int rcm_batch_order(rcm_batch* b, const int32_t* start_in, uint32_t flags, int32
     }
   }
   int launches = 0;
+  if (batch_solo(b)) {
+    std::vector<int32_t> given((size_t)C, -1);
+    if (start_in)
+      for (int32_t k = 0; k < C; ++k) given[k] = std::max(start_in[k], -1);
+    ++launches;
+    const int r = batch_solo_pass(b, SOLO_ORDER, given, cur.data(), iters.data(), status.data());
+    if (r) return r;
+    for (int32_t k : b->solo) need[k] = kDone;
+  }
   std::vector<int32_t> plain, cm;
   for (;;) {
     plain.clear();
@@ -2031,8 +2213,15 @@ int rcm_batch_run(rcm_batch* b, const int32_t* start, uint32_t flags, int32_t* s
   const bool rev = (flags & RCM_FLAG_REVERSE) != 0;
   RCM_HIP(hipMemcpyAsync(b->d_starts, start, (size_t)C * sizeof(int32_t), hipMemcpyHostToDevice, b->stream));
   RCM_HIP(hipEventRecord(b->ev[0], b->stream));
+  const bool solo = batch_solo(b);
   auto enqueue_run = [&]() {
-    enqueue_many(b, b->d_order, b->blk_order, b->nblk_order, C, false, false, b->total_n);
+    if (solo) {
+      enqueue_solo(b, SOLO_RUN);
+      enqueue_many(b, b->d_rest, b->blk_rest, b->blk_rest_h.back(), (int32_t)b->rest.size(), false, false,
+                   b->rest_rows);
+    } else {
+      enqueue_many(b, b->d_order, b->blk_order, b->nblk_order, C, false, false, b->total_n);
+    }
     if (rev)
       hipLaunchKernelGGL(k_reverse_many, dim3((unsigned)b->nblk_order), dim3(256), 0, b->stream, b->jobs, b->d_order,
                          C, b->blk_order);
@@ -2061,7 +2250,8 @@ int rcm_batch_run(rcm_batch* b, const int32_t* start, uint32_t flags, int32_t* s
   float ms = 0.f;
   RCM_HIP(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));
   b->timing.run_ms = ms;
-  b->timing.workers = batch_workers(b);
+  b->timing.workers = solo && b->rest.empty() ? std::min((int)b->solo.size(), b->solo_resident) : batch_workers(b);
+  if (solo && b->rest.empty()) *b->h_g = ManyControl{};  // the batch engine did not run: no abort word of its own
   int64_t nb = 0;
   std::vector<int32_t> st((size_t)C, RCM_OK);
   const int rc = collect_status(b, b->order.data(), C, st.data(), &nb);
@@ -2217,6 +2407,8 @@ int rcm_server_create(int device, const rcm_server_config* cfg, rcm_server** out
     if (rc) break;
     s->batch.push_back(b);
     rcm_batch_set_param(b, RCM_PARAM_VARIANT, 0);  // lanes were measured with variant 0 (256 threads)
+    b->engine_set = false;                         // ... for the requests that do not fit the one-workgroup engine
+    b->lane = true;
     // twice the lane's share by default: idle workgroups leave a launch (k_reorder_many), so a lane whose group
     // needs fewer gives its slots back; measured on the 400-request stream, 4 lanes: capacity 4.0x one-at-a-time
     // with 128 workgroups per lane, 4.4x with 256 or 384, 3.9x with 512
@@ -2416,9 +2608,11 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
   if (start < 0 || start >= c->n) return RCM_EINVAL;
   RCM_HIP(hipSetDevice(c->device));
   const int64_t keep_v = c->variant, keep_w = c->workers;
+  const bool keep_set = c->engine_set;
   rcm_tune_result best{};
   best.best_ms = 1e300;
   int count = 0;
+  c->engine_set = true;
   for (int v = 0; v < kVariants; ++v) {
     std::vector<int> ws = tune_workers(c->max_resident[v]);
     if (v == 0) ws.insert(ws.begin(), 0);  // 0 = automatic: the default configuration
@@ -2431,6 +2625,7 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
         if (rc) {
           c->variant = keep_v;
           c->workers = keep_w;
+          c->engine_set = keep_set;
           return rc;
         }
         t.push_back(c->timing.run_kernel_ms);
@@ -2464,13 +2659,47 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
     } else if (rc != RCM_ECAPACITY) {
       c->variant = keep_v;
       c->workers = keep_w;
+      c->engine_set = keep_set;
       return rc;
     }
   }
   c->variant = best.variant;
   c->workers = best.workers;
-  best.candidates = count;
   best.threads = variant_threads(best.variant);
+  // the automatic choice, where that is the one-workgroup engine
+  const int64_t best_w = c->workers;
+  c->workers = 0;
+  c->engine_set = false;
+  bool automatic = false;
+  if (ctx_solo(c)) {
+    std::vector<double> t;
+    int rc = RCM_OK;
+    for (int r = 0; r < repeats && rc == RCM_OK; ++r) {
+      rc = run_engine(c, start, false);
+      t.push_back(c->timing.run_kernel_ms);
+    }
+    if (rc) {
+      c->variant = keep_v;
+      c->workers = keep_w;
+      c->engine_set = keep_set;
+      return rc;
+    }
+    ++count;
+    const double ms = median_of(t);
+    if (ms < best.best_ms) {
+      automatic = true;
+      best.best_ms = ms;
+      best.variant = (int32_t)kDefaultCtxVariant;
+      best.workers = 1;
+      best.threads = SoloG::T;
+      c->variant = kDefaultCtxVariant;
+    }
+  }
+  if (!automatic) {
+    c->workers = best_w;
+    c->engine_set = true;
+  }
+  best.candidates = count;
   c->have_perm = false;  // the tuning runs overwrote the last order
   *out = best;
   return RCM_OK;
@@ -2480,6 +2709,7 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
   if (!b || !start || !out || repeats < 1) return RCM_EINVAL;
   if (b->count == 0) return RCM_ENOTLOADED;
   const int64_t keep_v = b->variant, keep_w = b->workers;
+  const bool keep_set = b->engine_set;
   rcm_tune_result best{};
   best.best_ms = 1e300;
   int count = 0;
@@ -2496,6 +2726,7 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
         if (rc == RCM_EDEVICE || rc == RCM_ETIMEOUT || rc == RCM_EINVAL || rc == RCM_ENOTLOADED) {
           rcm_batch_set_param(b, RCM_PARAM_VARIANT, keep_v);
           rcm_batch_set_param(b, RCM_PARAM_WORKERS, keep_w);
+          b->engine_set = keep_set;
           return rc;
         }
         t.push_back(b->timing.run_ms);
@@ -2540,8 +2771,32 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
   }
   rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, best_h);
   best.helper_nodes = (int32_t)best_h;
-  best.candidates = count;
   best.threads = kVarThreads[best.variant];
+  // the automatic choice, where that sends matrices to the one-workgroup engine (the rest runs the chosen variant)
+  const int64_t best_w = b->workers;
+  rcm_batch_set_param(b, RCM_PARAM_WORKERS, 0);
+  b->engine_set = false;
+  bool automatic = false;
+  if (batch_solo(b)) {
+    std::vector<double> t;
+    for (int r = 0; r < repeats; ++r) {
+      const int run = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
+      if (run == RCM_EDEVICE || run == RCM_ETIMEOUT || run == RCM_EINVAL || run == RCM_ENOTLOADED) return run;
+      t.push_back(b->timing.run_ms);
+    }
+    ++count;
+    const double ms = median_of(t);
+    if (ms < best.best_ms) {
+      automatic = true;
+      best.best_ms = ms;
+      best.workers = b->timing.workers;
+    }
+  }
+  if (!automatic) {
+    rcm_batch_set_param(b, RCM_PARAM_WORKERS, best_w);
+    b->engine_set = true;
+  }
+  best.candidates = count;
   b->have_perm = false;
   *out = best;
   return RCM_OK;
@@ -2599,7 +2854,18 @@ int rcm_gpu_batch_noalloc(int32_t n, int64_t nnz, const int32_t* d_row_ptr, cons
   a.claim_filter = kDefaultClaimFilter;
 
   int32_t start = start_node;
-  if (start < 0) {  // SimplePeripheral::findPeripheral (src/simple_peripheral.cpp:92-141)
+  const bool solo = solo_fits(n, vflags[1], n);
+  if (solo) {  // start search and order in one launch of one workgroup
+    const SoloJob J{d_row_ptr, d_col_idx, d_perm_out, a.qinfo, n};
+    hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, nullptr, J, (int32_t)SOLO_ORDER, start,
+                       (int32_t)kDefaultSpeculate, a.budget_ticks, a.ctl);
+    RCM_HIP(hipGetLastError());
+    Control h{};
+    RCM_HIP(hipMemcpy(&h, a.ctl, sizeof(Control), hipMemcpyDeviceToHost));
+    if (h.error == ERR_TIMEOUT) return RCM_ETIMEOUT;
+    if ((int32_t)h.placed != n) return RCM_ENOTCONNECTED;
+    start = h.start;
+  } else if (start < 0) {  // SimplePeripheral::findPeripheral (src/simple_peripheral.cpp:92-141)
     int32_t* level = reinterpret_cast<int32_t*>(base + L.level);
     start = n / 2;
     if (n == 1) {
@@ -2622,8 +2888,10 @@ int rcm_gpu_batch_noalloc(int32_t n, int64_t nnz, const int32_t* d_row_ptr, cons
       }
     }
   }
-  int rc = noalloc_run(D, a, start, false);
-  if (rc) return rc;
+  if (!solo) {
+    const int rc = noalloc_run(D, a, start, false);
+    if (rc) return rc;
+  }
   if (bandwidth_out && (flags & RCM_FLAG_BANDWIDTH)) {  // computeBandwidth (src/main.cpp:143-184)
     int32_t* inv = reinterpret_cast<int32_t*>(a.claim);  // the claims are no longer needed
     const int blocks = (n + 255) / 256;

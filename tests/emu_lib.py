@@ -21,7 +21,7 @@ def lib(engine: str = "block"):
     if engine not in _libs:
         subprocess.run(["make", "-s", "-C", EMU_DIR], check=True)
         L = C.CDLL(os.path.join(EMU_DIR, f"libemu_{engine}.so"))
-        if engine in ("many", "ops"):
+        if engine in ("many", "ops", "solo"):
             _libs[engine] = L
             return L
         L.emu_run.restype = C.c_int
@@ -202,3 +202,31 @@ def run_wg(mats, starts, workers=3, bfs=False):
                       1 if bfs else 0, perm.ctypes.data_as(I32P), lev.ctypes.data_as(I32P), info.ctypes.data_as(I32P))
     off = np.concatenate([[0], np.cumsum(n)])
     return rc, [perm[off[k]:off[k + 1]] for k in range(len(mats))], [lev[off[k]:off[k + 1]] for k in range(len(mats))], info
+
+
+def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.0):
+    """One workgroup per matrix (engine_solo.hpp). mats: list of (rp, ci); mode 0 = order from starts[k], 1 = start
+    search, 2 = start search (where starts[k] < 0) and order. Returns ([perm], info[count, 6]) with info = error,
+    placed, steps, start, sweeps, passes."""
+    L = lib("solo")
+    if not hasattr(L, "_solo_ready"):
+        I64P = C.POINTER(C.c_int64)
+        L.emu_run_solo.restype = C.c_int
+        L.emu_run_solo.argtypes = [C.c_int32, I32P, I64P, I64P, I32P, I32P, I32P, C.c_int32, C.c_int32, C.c_int32,
+                                   C.c_int32, I32P, I32P, C.c_double]
+        L._solo_ready = True
+    n = np.array([len(rp) - 1 for rp, _ in mats], np.int32)
+    rp_off = np.concatenate([[0], np.cumsum([len(rp) for rp, _ in mats])[:-1]]).astype(np.int64)
+    ci_off = np.concatenate([[0], np.cumsum([len(ci) for _, ci in mats])[:-1]]).astype(np.int64)
+    rpc = np.ascontiguousarray(np.concatenate([rp for rp, _ in mats]), np.int32)
+    cic = np.ascontiguousarray(np.concatenate([ci for _, ci in mats] + [np.zeros(1, np.int32)]), np.int32)
+    st = np.ascontiguousarray(starts, np.int32)
+    perm = np.full(int(n.sum()), -1, np.int32)
+    info = np.zeros((len(mats), 6), np.int32)
+    I64 = C.POINTER(C.c_int64)
+    rc = L.emu_run_solo(len(mats), n.ctypes.data_as(I32P), rp_off.ctypes.data_as(I64), ci_off.ctypes.data_as(I64),
+                        rpc.ctypes.data_as(I32P), cic.ctypes.data_as(I32P), st.ctypes.data_as(I32P), workers, mode,
+                        speculate, geo, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
+    assert rc == 0, "emulator rejected the arguments"
+    off = np.concatenate([[0], np.cumsum(n)])
+    return [perm[off[k]:off[k + 1]] for k in range(len(mats))], info

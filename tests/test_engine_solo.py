@@ -1,0 +1,127 @@
+"""The one-workgroup engine (csrc/engine_solo.hpp) against the oracle, bit for bit: on the CPU in the wave emulator,
+with a small geometry whose chunks (256 slots, 128 parents) and ring (64 entries) fill, split and overflow at small
+sizes, and with the library's; on the GPU through the entry points that choose it."""
+import numpy as np
+import pytest
+
+import graphs as G
+import oracle_lib as O
+import parallelbatchrcm_amd as P
+
+MAXROW = 64  # the longest row the engine takes
+
+
+def _stencil(kind, *dims, seed=11):
+    m, _ = P.workloads.permute_symmetric(getattr(P.workloads, kind)(*dims), seed)
+    return m.row_offsets, m.col_ids
+
+
+def _regular(n, deg, seed):
+    """Every row of exactly `deg` entries (self included): a random circulant graph."""
+    rng = np.random.default_rng(seed)
+    steps = rng.choice(np.arange(2, n // 2), (deg - 1) // 2 - 1, replace=False)
+    steps = np.concatenate([[1], steps])
+    off = np.concatenate([[0], steps, n - steps])
+    rows = np.sort((np.arange(n)[:, None] + off[None, :]) % n, axis=1)
+    return np.arange(0, n * rows.shape[1] + 1, rows.shape[1]).astype(np.int32), rows.reshape(-1).astype(np.int32)
+
+
+CASES = {
+    "path1": lambda: G.path(1),
+    "path2": lambda: G.path(2),
+    "path300": lambda: G.path(300),  # more levels than the level boundaries kept
+    "star64": lambda: G.star(MAXROW),  # the centre's row is the longest taken
+    "complete40": lambda: G.complete(40),
+    "random1500": lambda: G.random_connected(1500, 9000, seed=5),  # levels of several chunks, the ring overflows
+    "duplicates": lambda: G.with_duplicates(*G.random_connected(300, 500, seed=7), seed=3),
+    "unsorted": lambda: G.shuffle_rows(*G.random_connected(300, 900, seed=7), seed=8),
+    "grid24x20": lambda: _stencil("stencil2d", 24, 20),
+    "stencil11x9x13": lambda: _stencil("stencil3d", 11, 9, 13),
+    "rows63": lambda: _regular(700, 63, 1),  # chunks cut inside and at rows of nearly a slot group
+}
+
+
+@pytest.mark.parametrize("geo", [0, 1])
+def test_emulated_order_and_search(geo):
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    names = list(CASES) if geo == 0 else ["path2", "star64", "duplicates", "grid24x20"]
+    mats = [CASES[name]() for name in names]
+    for start in (lambda n: 0, lambda n: n - 1):
+        starts = [start(len(rp) - 1) for rp, _ in mats]
+        perms, info = E.run_solo(mats, starts, workers=3, geo=geo)
+        for k, (rp, ci) in enumerate(mats):
+            assert info[k, 0] == 0 and info[k, 1] == len(rp) - 1, k
+            assert np.array_equal(perms[k], O.cm(rp, ci, starts[k])), (names[k], starts[k])
+    for spec in (0, 2, 3) if geo == 0 else (3,):
+        perms, info = E.run_solo(mats, [-1] * len(mats), workers=3, mode=2, speculate=spec, geo=geo)
+        for k, (rp, ci) in enumerate(mats):
+            _, s, it, _ = O.peripheral(rp, ci)
+            assert (info[k, 3], info[k, 4]) == (s, it), (names[k], spec)
+            assert np.array_equal(perms[k], O.cm(rp, ci, s)), (names[k], spec)
+
+
+def test_emulated_directed_and_disconnected():
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    directed = G.directed_with_empty_rows(2000, 1500, 24, 2)
+    parts = G.from_edges(10, [(0, 1), (1, 2), (5, 6)])
+    perms, info = E.run_solo([directed, parts], [0, 0], workers=2, geo=0)
+    assert info[0, 0] == 0 and np.array_equal(perms[0], O.cm(*directed, 0))
+    assert info[1, 0] == 0 and info[1, 1] == 3 and perms[1][:3].tolist() == [0, 1, 2]
+
+
+def test_emulated_watchdog():
+    """A launch past its budget still gives every matrix a status."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    _, info = E.run_solo([CASES["grid24x20"](), G.path(9)], [0, 0], workers=1, geo=0, timeout_s=0.0)
+    assert (info[:, 0] == 1).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CASES) + ["rows63x9000", "rgg65536", "grid65537"])
+def test_gpu_single(name):
+    """rcm_ctx (search, order, run), at the largest matrix one workgroup takes alone and just beyond it."""
+    big = {"rows63x9000": lambda: _regular(9000, 63, 2), "grid65537": lambda: _stencil("stencil2d", 3, 21846),
+           "rgg65536": lambda: (lambda m: (m.row_offsets, m.col_ids))(P.workloads.config(3, scale=65536, seed=6))}
+    rp, ci = (CASES.get(name) or big[name])()
+    m = P.CSR(rp, ci)
+    _, s, it, _ = O.peripheral(rp, ci)
+    want = O.cm(rp, ci, s)
+    print("[case]", name, m.rows, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        assert c.order() == (s, it)
+        assert np.array_equal(c.perm(), want)
+        assert c.find_start() == s and c.timing().start_iterations == it
+        c.run(s, P.RCM_FLAG_REVERSE)
+        assert np.array_equal(c.perm(), want[::-1])
+        assert c.bandwidth() == O.bandwidth(rp, ci, want)
+
+
+@pytest.mark.gpu
+def test_gpu_set_with_rows_for_either_engine():
+    """A set of matrices for both engines (rows up to 64 and beyond), a disconnected one and one given start."""
+    mats = [f() for f in CASES.values()] + [G.star(MAXROW + 1), G.hub_graph(3000, 2000, seed=3),
+                                            G.from_edges(10, [(0, 1), (1, 2), (5, 6)])]
+    bs = P.BatchSet.from_matrices([P.CSR(*m) for m in mats])
+    given = np.full(len(mats), -1, np.int32)
+    given[4] = 7
+    print("[case] set", len(mats), flush=True)
+    with P.RcmBatch(timeout_ms=20000) as b:
+        b.load(bs)
+        starts, iters, st = b.order(given)
+        assert st[-1] == P.RCM_ENOTCONNECTED and not st[:-1].any()
+        perms = b.perms()
+        for k, (rp, ci) in enumerate(mats[:-1]):
+            s, it = (7, 0) if k == 4 else O.peripheral(rp, ci)[1:3]
+            assert (starts[k], iters[k]) == (s, it), k
+            assert np.array_equal(perms[k], O.cm(rp, ci, s)), k
+        st = b.run(starts)
+        assert st[-1] == P.RCM_ENOTCONNECTED and not st[:-1].any()
+        for k, p in enumerate(b.perms()[:-1]):
+            assert np.array_equal(p, perms[k]), k
