@@ -87,8 +87,9 @@ enum rcm_param {
   RCM_PARAM_DIGIT_BITS = 4,  /* radix digit width of the current variant (read-only: set the variant) */
   RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit). Until it is set (and while
                                 WORKERS, SORT, STRICT, PROFILE, CLAIM_FILTER and BATCH_CAP keep their defaults),
-                                matrices of up to 65,536 rows (in a large set or a serving lane more), each of at
-                                most 64 entries, are ordered by one workgroup each, whatever the variant:
+                                whatever the variant, matrices whose rows have at most 64 entries are ordered by
+                                one workgroup each up to 32,768 rows in a context, 65,536 in a set (in a large
+                                set or a serving lane more), and in a context beyond that by a team of 128:
                                 0 = 256 threads, 2048 adjacency slots, 256 parents, 4-bit digits (serving
                                     lanes)
                                 1 = 512 threads, 2048 slots, 256 parents, 4-bit digits (rcm_ctx default)

@@ -38,8 +38,7 @@ struct SoloGeo {
   static constexpr int W = T / kWave;
   static constexpr int EPT = S / T;
   static constexpr int NC = S / kWave;
-  static constexpr int H = S;  // hash words: a chunk has at most S distinct children
-  static constexpr int HB = __builtin_ctz((unsigned)S_);
+  static constexpr int HB = __builtin_ctz((unsigned)S_);  // S hash words: a chunk has at most S distinct children
   static_assert(S % T == 0 && NC <= kWave && (S & (S - 1)) == 0 && (R & (R - 1)) == 0 && B % 32 == 0, "geometry");
   static_assert((1 << kSoloDegBits) > kSoloMaxRow, "degrees fit their field");
   static_assert(S >= kSoloMaxRow && S <= 65536, "any one parent fits a chunk");
@@ -47,7 +46,7 @@ struct SoloGeo {
 
 template <class G>
 struct SoloSmem {
-  uint32_t tab[G::H];            // hash: the smallest slot claiming a child, kNoSlot when free
+  uint32_t tab[G::S];            // hash: the smallest slot claiming a child, kNoSlot when free
   uint32_t sc[G::S];             // per slot: the child while the chunk claims; then the owned children, packed
   uint32_t ckey[G::S + 2];       // packed children: parent << kSoloDegBits | degree; child o at o + 1, ~0 around them
   uint32_t crb[G::S];            // packed children: row begin
@@ -78,6 +77,74 @@ struct SoloJob {
 struct RowBounds {
   int32_t b, e;
 } __attribute__((packed, aligned(4)));
+
+// The place of packed child o of cnt, key ckey[o + 1], among its siblings: earlier ones of larger degree go behind it,
+// later ones of smaller degree before it. pos and dp (its place and degree prefix in packed order) are corrected. The
+// nearest kSib on either side are read together; few parents have more children.
+template <class K>
+__device__ __forceinline__ void packed_place(const K& ckey, uint32_t o, uint32_t cnt, uint32_t key, uint32_t& pos,
+                                             uint32_t& dp) {
+  constexpr int kSib = 3;
+  constexpr uint32_t dm = (1u << kSoloDegBits) - 1u;
+  uint32_t f[kSib], h[kSib];
+#pragma unroll
+  for (int u = 0; u < kSib; ++u) {
+    f[u] = ckey[o >= (uint32_t)u ? o - (uint32_t)u : 0u];
+    h[u] = ckey[min(o + 2u + (uint32_t)u, cnt + 1u)];
+  }
+#pragma unroll
+  for (int u = 0; u < kSib; ++u) {  // siblings are neighbours: beyond the last one the keys differ above dm
+    if ((f[u] ^ key) <= dm && f[u] > key) {
+      --pos;
+      dp -= f[u] & dm;
+    }
+    if ((h[u] ^ key) <= dm && h[u] < key) {
+      ++pos;
+      dp += h[u] & dm;
+    }
+  }
+  if ((f[kSib - 1] ^ key) <= dm)
+    for (uint32_t u = o - (uint32_t)kSib;; --u) {
+      const uint32_t x = ckey[u];
+      if ((x ^ key) > dm) break;
+      if (x > key) {
+        --pos;
+        dp -= x & dm;
+      }
+    }
+  if ((h[kSib - 1] ^ key) <= dm)
+    for (uint32_t u = o + 2u + (uint32_t)kSib;; ++u) {
+      const uint32_t x = ckey[u];
+      if ((x ^ key) > dm) break;
+      if (x < key) {
+        ++pos;
+        dp += x & dm;
+      }
+    }
+}
+
+// Claims in the table: a child's word holds the smallest of its slots. hash_try offers slot j the word h and returns what
+// held it; hash_settle goes on from there and returns the child's word. (A slot's sm.sc is stored before; slots of the
+// same child meet at one word, so the search ends: S words, at most S children.)
+template <class SM>
+__device__ __forceinline__ uint32_t hash_try(SM& sm, uint32_t h, uint32_t j) {
+  uint32_t old = kNoSlot;
+  (void)__hip_atomic_compare_exchange_strong(&sm.tab[h], &old, j, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+  return old;
+}
+template <class G, class SM>
+__device__ __forceinline__ uint32_t hash_settle(SM& sm, uint32_t h, uint32_t old, uint32_t child, uint32_t j) {
+  while (old != kNoSlot) {
+    if (sm.sc[old] == child) {  // taken by this child
+      (void)__hip_atomic_fetch_min(&sm.tab[h], j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      break;
+    }
+    h = (h + 1) & (uint32_t)(G::S - 1);
+    old = hash_try(sm, h, j);
+  }
+  return h;
+}
 
 // The queue and the chunk of one pass, the same in every thread.
 struct SoloState {
@@ -175,26 +242,10 @@ __device__ __forceinline__ bool solo_step(const SoloJob& J, SoloSmem<G>& sm, Sol
     __asm__ volatile("" ::: "memory");  // a slot's child is in LDS before the slot can be found in the table
     uint32_t old[KN];
 #pragma unroll
-    for (int k = 0; k < KN; ++k) {
-      old[k] = kNoSlot;
-      if (own[k])
-        (void)__hip_atomic_compare_exchange_strong(&sm.tab[hp[k]], &old[k], (uint32_t)((k * W + wv) * kWave + ln),
-                                                   __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
+    for (int k = 0; k < KN; ++k) old[k] = own[k] ? hash_try(sm, hp[k], (uint32_t)((k * W + wv) * kWave + ln)) : kNoSlot;
 #pragma unroll
-    for (int k = 0; k < KN; ++k) {
-      const uint32_t j = (uint32_t)((k * W + wv) * kWave + ln);
-      while (old[k] != kNoSlot) {  // taken: by this child, or look further
-        if (sm.sc[old[k]] == cc[k]) {
-          (void)__hip_atomic_fetch_min(&sm.tab[hp[k]], j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-          break;
-        }
-        hp[k] = (hp[k] + 1) & (uint32_t)(G::H - 1);
-        old[k] = kNoSlot;
-        (void)__hip_atomic_compare_exchange_strong(&sm.tab[hp[k]], &old[k], j, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-    }
+    for (int k = 0; k < KN; ++k)
+      hp[k] = hash_settle<G>(sm, hp[k], old[k], cc[k], (uint32_t)((k * W + wv) * kWave + ln));
 #pragma unroll
     for (int k = 0; k < KN; ++k) {
       rb[k] = (uint32_t)bd[k].b;
@@ -261,19 +312,7 @@ __device__ __forceinline__ bool solo_step(const SoloJob& J, SoloSmem<G>& sm, Sol
     uint32_t pos = o, dp = sm.cdx[o];
     const uint32_t rbo = sm.crb[o], child = sm.sc[o], key = sm.ckey[o + 1];
     constexpr uint32_t dm = (1u << kSoloDegBits) - 1u;
-    if (!bfs) {
-      uint32_t f = sm.ckey[o], g = sm.ckey[o + 2];
-      for (uint32_t u = o; (f ^ key) <= dm; f = sm.ckey[--u])  // earlier siblings of larger degree go behind it
-        if (f > key) {
-          --pos;
-          dp -= f & dm;
-        }
-      for (uint32_t u = o + 2; (g ^ key) <= dm; g = sm.ckey[++u])  // later siblings of smaller degree go before it
-        if (g < key) {
-          ++pos;
-          dp += g & dm;
-        }
-    }
+    if (!bfs) packed_place(sm.ckey, o, cnt, key, pos, dp);
     const int32_t p = q.tail + (int32_t)pos;
     J.perm[p] = (int32_t)child;
     if (direct) {
@@ -356,7 +395,7 @@ template <class G>
 __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, int32_t mode, int32_t start,
                                             int32_t speculate, uint64_t deadline, Control* ctl) {
   const int tid = threadIdx.x, ln = lane_id();
-  for (int i = tid; i < G::H; i += G::T) sm.tab[i] = kNoSlot;
+  for (int i = tid; i < G::S; i += G::T) sm.tab[i] = kNoSlot;
   for (int i = tid; i < G::S; i += G::T) sm.mark[i] = 0;
   // (the pass's first barrier orders these before their first use)
   const int32_t n = J.n;

@@ -21,6 +21,7 @@
 
 #include "engine_many.hpp"
 #include "engine_solo.hpp"
+#include "engine_team.hpp"
 #include "hip_exec.hpp"
 #include "level_cm.hpp"
 #include "rcm_gpu_batch_abi.h"
@@ -95,8 +96,8 @@ using SoloG = SoloGeo<1024, 4096, kSoloMaxN>;
 // A matrix goes through it when it fits and has at most `limit` rows. One workgroup takes 0.5-0.7 entries per ns where
 // the levels are wide, the batch engine 11 over the whole GPU, but 5-10 us a level however narrow: start search and
 // order on MI355X, one workgroup against the batch engine, 0.84 against 3.3 ms for a 100 x 100 grid, 2.6 against 4.0
-// ms for a 40k-point geometric graph, but 3.9 against 3.5 ms for a 48^3 stencil (110k rows). Up to kSoloAlone rows one
-// workgroup wins whatever the shape; beyond, only beside enough other matrices: a set of `total` rows keeps the batch
+// ms for a 40k-point geometric graph, but 3.9 against 3.5 ms for a 48^3 stencil (110k rows). In a set, up to kSoloAlone
+// rows one workgroup wins whatever the shape; beyond, only beside enough other matrices: `total` rows keep the batch
 // engine busy for total / 11 entries' time, so a matrix of total / kSoloShare rows ends on its one workgroup before
 // the batch engine would have ended the set.
 constexpr int32_t kSoloAlone = 1 << 16;
@@ -108,6 +109,26 @@ bool solo_fits(int32_t n, uint32_t maxrow, int64_t total) {
   return n <= std::min<int64_t>(kSoloMaxN, std::max<int64_t>(kSoloAlone, total / kSoloShare)) &&
          maxrow <= (uint32_t)kSoloMaxRow;
 }
+
+// The team engine (engine_team.hpp): up to kTeamMax workgroups on the matrix of a context, beyond kCtxSolo rows.
+using TeamG = TeamGeo<1024, 4096>;
+// Start search and order in ms, one workgroup against the team: 32k rows, 2D 1.67 / 2.56, 3D 1.25 / 1.16, geometric of
+// mean degree 13 2.19 / 2.00; 64k, 2.95 / 4.25, 2.42 / 1.46, 4.16 / 2.96; 128k, 5.09 / 6.9, 4.6 / 2.09, 8.2 / 4.3. The
+// wider the levels the more a team gives, the narrow ones its leader takes on its own at 1.5 times one workgroup's time.
+constexpr int32_t kCtxSolo = 1 << 15;
+// Parents a member is given, as a power of two: about 128 slots, at most 16 parents (8 to 32 are within 10% on 2D, 3D and
+// geometric graphs of 8k to 1M rows). Longer rows mean levels that grow faster, and a level is spread by the count of the
+// one before: with 16 parents of 63 entries each, a member's children overflow its region.
+int team_wide(int32_t n, int64_t nnz) {
+  int w = 4;
+  while (w > 1 && ((int64_t)n << (7 - w)) < nnz) --w;
+  return w;
+}
+// Slots of a level beyond which its leader shares it: alone 1.4 us + 1.2 ns a slot, as a team 4.3-5 us a level
+// (2000 to 3500 are within 3%).
+constexpr uint32_t kTeamAlone = 2700;
+// Entries of a stage region: whatever two chunks give, and four times a member's share of the matrix.
+int32_t team_cap(int32_t n) { return std::min(kTeamMaxCap, std::max<int32_t>(2 * TeamG::S, n / (kTeamMax / 4))); }
 
 // lev: a CM run that also records BFS levels (a speculated start-search sweep); plain-BFS runs always do.
 template <int V>
@@ -336,6 +357,12 @@ struct rcm_ctx {
   int max_resident[kVariants] = {};  // co-resident workgroups of each variant
   rcm_mx::DevArena lscratch;         // level-synchronous engine scratch
   uint32_t* h_word = nullptr;        // pinned readback word of that engine
+  // team engine: stages, then the members' words and the records (one allocation for regions of team_cap entries); the
+  // tag its launches have come to (0: the stages hold anything); the loaded matrix outgrew a region
+  uint64_t* team = nullptr;
+  int32_t team_cap = 0;
+  uint32_t team_tag = 0;
+  bool team_off = false;
   // last result
   bool have_perm = false;
   bool reversed = false;
@@ -364,6 +391,21 @@ int ensure_state(rcm_ctx* c, int32_t n) {
   c->cap = n;
   c->dirty = n + 1;  // fresh memory: clear every batch record before the first run
   return RCM_OK;
+}
+
+// The team engine's memory for n rows: allocated when a matrix first needs it, kept and grown.
+bool ensure_team(rcm_ctx* c, int32_t n) {
+  const int32_t cap = team_cap(n);
+  if (c->team && c->team_cap >= cap) return true;
+  dev_free(c->team);
+  c->team_cap = 0;
+  c->team_tag = 0;
+  if (dev_alloc(&c->team, (size_t)kTeamMax * ((size_t)cap * 4 + kTeamWordStride) + 4) != hipSuccess) {
+    (void)hipGetLastError();  // the batch engine runs the matrix
+    return false;
+  }
+  c->team_cap = cap;
+  return true;
 }
 
 int wait_stream(rcm_ctx* c, hipEvent_t ev, int64_t limit_ms) {
@@ -411,38 +453,80 @@ int run_level(rcm_ctx* c, int32_t start, bool bfs) {
   return RCM_OK;
 }
 
-// Whether the loaded matrix goes through the one-workgroup engine: it fits, and no parameter of the batch engine was
-// chosen.
-bool ctx_solo(const rcm_ctx* c) {
+// Whether a level engine (one workgroup, or a team) takes the loaded matrix: it fits, and no parameter of the batch
+// engine was chosen.
+bool ctx_quick(const rcm_ctx* c) {
   return !c->engine_set && c->workers == 0 && !c->strict && !c->profile && c->sort_mode == 0 && c->batch_cap == 0 &&
-         c->claim_filter == kDefaultClaimFilter && solo_fits(c->n, c->maxdeg, c->n);
+         c->claim_filter == kDefaultClaimFilter && c->maxdeg <= (uint32_t)kSoloMaxRow && c->n <= kTeamMaxN &&
+         !c->team_off;
 }
 
-// One launch of the one-workgroup engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl.
-int ctx_run_solo(rcm_ctx* c, int32_t mode, int32_t start) {
-  const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
-  RCM_HIP(hipEventRecord(c->ev[0], c->stream));
-  hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
-                     (uint64_t)c->timeout_ms * 100000ull, c->ctl);
-  RCM_HIP(hipGetLastError());
-  RCM_HIP(hipEventRecord(c->ev[2], c->stream));
-  RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
-  RCM_HIP(hipEventRecord(c->ev[3], c->stream));
-  const int rc = wait_stream(c, c->ev[3], c->timeout_ms + 10000);
-  if (rc) return rc;
-  float ms = 0.f;
-  RCM_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[2]));
-  const Control& h = *c->h_ctl;
-  c->timing.init_kernel_ms = 0.0;
-  c->timing.run_kernel_ms = ms;
-  c->timing.workers = 1;
-  c->timing.batches = (int32_t)h.nbatches;
-  c->timing.placed = (int32_t)h.placed;
-  c->timing.error_site = 0;
-  for (int i = 0; i < 8; ++i) c->timing.error_info[i] = 0;
-  if (h.error == ERR_TIMEOUT) return RCM_ETIMEOUT;
-  if ((int32_t)h.placed != c->n) return RCM_ENOTCONNECTED;
-  return RCM_OK;
+// One launch of the level engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl. False when
+// it takes the matrix no further (ctx_quick, no memory for a team, a stage region too small): the batch engine's.
+bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
+  if (!ctx_quick(c)) return false;
+  const bool team = c->n > kCtxSolo;
+  if (team && !ensure_team(c, c->n)) return false;
+  *rc = [&]() -> int {
+    TeamArgs a{};
+    const uint64_t budget = (uint64_t)c->timeout_ms * 100000ull;
+    RCM_HIP(hipEventRecord(c->ev[0], c->stream));
+    if (team) {
+      const size_t words = (size_t)kTeamMax * (size_t)c->team_cap * 2;
+      a.row_ptr = c->rp;
+      a.col_idx = c->ci;
+      a.perm = c->perm;
+      a.claim = c->claim;
+      a.stage[0] = c->team;
+      a.stage[1] = c->team + words;
+      a.words = c->team + 2 * words;
+      a.rec = a.words + kTeamMax * kTeamWordStride;
+      a.ctl = c->ctl;
+      a.n = c->n;
+      a.cap = c->team_cap;
+      a.members = kTeamMax;
+      a.mode = mode;
+      a.start = start;
+      a.speculate = (int32_t)std::min<int64_t>(c->speculate, INT32_MAX);
+      a.wide = team_wide(c->n, c->nnz);
+      a.alone = kTeamAlone;
+      a.tag0 = c->team_tag < (1u << 30) ? c->team_tag : 0;  // a launch raises it by less than 2^31
+      a.budget_ticks = budget;
+      c->team_tag = 0;  // until the launch is known to have ended well
+      hipLaunchKernelGGL(k_team_init, dim3(256), dim3(256), 0, c->stream, a);
+      RCM_HIP(hipEventRecord(c->ev[1], c->stream));
+      hipLaunchKernelGGL(k_team<TeamG>, dim3(kTeamMax), dim3(TeamG::T), 0, c->stream, a);
+    } else {
+      const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
+      hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
+                         budget, c->ctl);
+    }
+    RCM_HIP(hipGetLastError());
+    RCM_HIP(hipEventRecord(c->ev[2], c->stream));
+    RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+    RCM_HIP(hipEventRecord(c->ev[3], c->stream));
+    const int st = wait_stream(c, c->ev[3], c->timeout_ms + 10000);
+    if (st) return st;
+    float ms_init = 0.f, ms = 0.f;
+    if (team) RCM_HIP(hipEventElapsedTime(&ms_init, c->ev[0], c->ev[1]));
+    RCM_HIP(hipEventElapsedTime(&ms, c->ev[team ? 1 : 0], c->ev[2]));
+    const Control& h = *c->h_ctl;
+    if (team && h.error == ERR_NONE) c->team_tag = a.tag0 + h.nbatches + 1;
+    c->timing.init_kernel_ms = ms_init;
+    c->timing.run_kernel_ms = ms;
+    c->timing.workers = team ? kTeamMax : 1;
+    c->timing.batches = (int32_t)h.nbatches;
+    c->timing.placed = (int32_t)h.placed;
+    c->timing.error_site = 0;
+    for (int i = 0; i < 8; ++i) c->timing.error_info[i] = 0;
+    if (h.error == ERR_TIMEOUT) return RCM_ETIMEOUT;
+    if (h.error == ERR_CAPACITY) return RCM_ECAPACITY;
+    if ((int32_t)h.placed != c->n) return RCM_ENOTCONNECTED;
+    return RCM_OK;
+  }();
+  if (*rc != RCM_ECAPACITY) return true;
+  c->team_off = true;
+  return false;
 }
 
 // One engine run from `start` (CM order, or plain BFS order with levels when bfs; a CM run also records the
@@ -450,7 +534,8 @@ int ctx_run_solo(rcm_ctx* c, int32_t mode, int32_t start) {
 int run_engine(rcm_ctx* c, int32_t start, bool bfs, bool levels = false) {
   if (!c->rp) return RCM_ENOTLOADED;
   if (start < 0 || start >= c->n) return RCM_EINVAL;
-  if (!bfs && !levels && ctx_solo(c)) return ctx_run_solo(c, SOLO_RUN, start);
+  int quick = RCM_OK;
+  if (!bfs && !levels && ctx_run_quick(c, SOLO_RUN, start, &quick)) return quick;
   if (c->variant == kLevelVariant) return run_level(c, start, bfs);
   RunArgs a{};
   a.row_ptr = c->rp;
@@ -593,6 +678,7 @@ int load_common(rcm_ctx* c, int32_t n, int64_t nnz) {
   RCM_HIP(hipStreamSynchronize(c->stream));
   if (h[0] != 0) return RCM_EINVAL;
   c->maxdeg = h[1];
+  c->team_off = false;
   c->n = n;
   c->nnz = nnz;
   c->have_perm = false;
@@ -1428,6 +1514,7 @@ int rcm_ctx_destroy(rcm_ctx* c) {
   dev_free(c->scratch);
   dev_free(c->prof);
   dev_free(c->trace);
+  dev_free(c->team);
   if (c->h_ctl) (void)hipHostFree(c->h_ctl);
   if (c->h_word) (void)hipHostFree(c->h_word);
   c->lscratch.release();
@@ -1562,13 +1649,13 @@ int rcm_ctx_find_start(rcm_ctx* c, int32_t* start_out, int32_t* iterations_out) 
   const int32_t n = c->n;
   int32_t cur = n / 2;
   int32_t iters = 0;
+  int quick = RCM_OK;
+  c->have_perm = c->have_perm && n == 1;
   if (n == 1) {
     cur = 0;
     iters = 1;
-  } else if (ctx_solo(c)) {
-    c->have_perm = false;
-    const int rc = ctx_run_solo(c, SOLO_SEARCH, -1);
-    if (rc) return rc;
+  } else if (ctx_run_quick(c, SOLO_SEARCH, -1, &quick)) {
+    if (quick) return quick;
     cur = c->h_ctl->start;
     iters = c->h_ctl->sweeps;
   } else {
@@ -1613,9 +1700,9 @@ int rcm_ctx_order(rcm_ctx* c, int32_t start_node, uint32_t flags, int32_t* start
   c->have_perm = false;
   int32_t cur = start_node, iters = 0, passes = 0;
   bool ordered = false;
-  if (ctx_solo(c)) {
-    const int rc = ctx_run_solo(c, SOLO_ORDER, start_node);
-    if (rc) return rc;
+  int quick = RCM_OK;
+  if (ctx_run_quick(c, SOLO_ORDER, start_node, &quick)) {
+    if (quick) return quick;
     cur = c->h_ctl->start;
     iters = c->h_ctl->sweeps;
     passes = c->h_ctl->passes;
@@ -2450,7 +2537,7 @@ int rcm_server_create(int device, const rcm_server_config* cfg, rcm_server** out
     if (dev_alloc(&sc->ci, (size_t)kServeSoloNnz) == hipSuccess) sc->cap_ci = kServeSoloNnz;
     sc->own_csr = true;
     if (sc->cap_rp < (int64_t)kServeSoloN + 1 || sc->cap_ci < kServeSoloNnz ||
-        ensure_state(sc, kServeSoloN) != RCM_OK) {
+        ensure_state(sc, kServeSoloN) != RCM_OK || !ensure_team(sc, kServeSoloN)) {
       (void)hipGetLastError();
       rcm_ctx_destroy(sc);
       continue;
@@ -2666,17 +2753,19 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
   c->variant = best.variant;
   c->workers = best.workers;
   best.threads = variant_threads(best.variant);
-  // the automatic choice, where that is the one-workgroup engine
+  // the automatic choice, where that is a level engine
   const int64_t best_w = c->workers;
   c->workers = 0;
   c->engine_set = false;
   bool automatic = false;
-  if (ctx_solo(c)) {
+  if (ctx_quick(c)) {
     std::vector<double> t;
+    int32_t used = 0;
     int rc = RCM_OK;
     for (int r = 0; r < repeats && rc == RCM_OK; ++r) {
       rc = run_engine(c, start, false);
       t.push_back(c->timing.run_kernel_ms);
+      used = c->timing.workers;
     }
     if (rc) {
       c->variant = keep_v;
@@ -2690,8 +2779,8 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
       automatic = true;
       best.best_ms = ms;
       best.variant = (int32_t)kDefaultCtxVariant;
-      best.workers = 1;
-      best.threads = SoloG::T;
+      best.workers = used;
+      best.threads = ctx_quick(c) ? SoloG::T : variant_threads(kDefaultCtxVariant);
       c->variant = kDefaultCtxVariant;
     }
   }

@@ -5,7 +5,7 @@
 template <class T, class V>
 inline T __hip_atomic_fetch_or(T* p, V v, int, int) { return __atomic_fetch_or(p, (T)v, __ATOMIC_SEQ_CST); }
 #endif
-#include "engine_solo.hpp"
+#include "engine_team.hpp"
 
 #include <vector>
 
@@ -75,5 +75,50 @@ int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const i
                                                perm_cat, info, timeout_s)
              : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
                                                    speculate, perm_cat, info, timeout_s);
+}
+
+// Orders one matrix with a team of `workers` workgroups (engine_team.hpp; 64 threads, 256 slots). wide: parents per
+// member wanted, as a power of two. alone: slots of a level its leader takes on its own. cap: entries of a stage region.
+// tag0 0 starts from memory that holds anything. info = error, placed, levels, start, sweeps, passes.
+int emu_run_team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start, int32_t workers, int32_t mode,
+                 int32_t speculate, int32_t wide, int32_t alone, int32_t cap, uint32_t tag0, int32_t* perm,
+                 int32_t* info, double timeout_s) {
+  using G = TeamGeo<64, 256>;
+  int32_t maxrow = 1;
+  for (int32_t i = 0; i < n; ++i) maxrow = std::max(maxrow, rp[i + 1] - rp[i]);
+  if (maxrow > kSoloMaxRow || workers > kTeamMax) return -3;
+  std::vector<uint64_t> claim((size_t)n, 0x5A5A5A5A5A5A5A5Aull);
+  const uint64_t old = tag0 ? (uint64_t)tag0 << 32 : 0x5A5A5A5A5A5A5A5Aull;
+  std::vector<uint64_t> s0((size_t)kTeamMax * cap * 2, old), s1((size_t)kTeamMax * cap * 2, old),
+      words((size_t)kTeamMax * kTeamWordStride, old), rec(4, 0x5A5A5A5A5A5A5A5Aull);
+  Control ctl;
+  TeamArgs a{};
+  a.row_ptr = rp;
+  a.col_idx = ci;
+  a.perm = perm;
+  a.claim = claim.data();
+  a.stage[0] = s0.data();
+  a.stage[1] = s1.data();
+  a.words = words.data();
+  a.rec = rec.data();
+  a.ctl = &ctl;
+  a.n = n;
+  a.cap = cap;
+  a.members = workers;
+  a.mode = mode;
+  a.start = start;
+  a.speculate = speculate;
+  a.wide = wide;
+  a.alone = (uint32_t)alone;
+  a.tag0 = tag0;
+  a.budget_ticks = (uint64_t)(timeout_s * 1e8);
+  emu::launch(2, 64, false, k_team_init, a);
+  emu::emu_lds_bytes = sizeof(TeamSmem<G>);
+  emu::launch((unsigned)workers, G::T, true, k_team<G>, a);
+  emu::emu_lds_bytes = 256 * 1024;
+  const int32_t v[6] = {(int32_t)ctl.error, (int32_t)ctl.placed, (int32_t)ctl.nbatches, ctl.start,
+                        ctl.sweeps, ctl.passes};
+  std::memcpy(info, v, sizeof(v));
+  return 0;
 }
 }

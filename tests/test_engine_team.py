@@ -1,0 +1,109 @@
+"""The team engine (csrc/engine_team.hpp) against the oracle, bit for bit: on the CPU in the wave emulator, with a small
+geometry (64 threads, 256 slots); on the GPU through a context, from the smallest matrix it takes."""
+import numpy as np
+import pytest
+
+import graphs as G
+import oracle_lib as O
+import parallelbatchrcm_amd as P
+from test_engine_solo import CASES, _regular, _stencil
+
+SOLO = 1 << 15  # rows up to which a context leaves a matrix to one workgroup
+
+
+def _lopsided(mids, fertile, tail):
+    """A level of 60 * mids nodes whose first `fertile` have 60 children each and the others none, then a path: whoever
+    gets the first part of that level ends with far more than a share of the next."""
+    e = [(0, 1 + k) for k in range(13)]
+    e += [(1 + k % 13, 14 + k) for k in range(mids)]
+    order = [14 + k for j in range(13) for k in range(j, mids, 13)]  # the mids by queue position
+    base = 14 + mids
+    e += [(m, base + 60 * i + j) for i, m in enumerate(order) for j in range(60)]
+    leaves = base + 60 * mids
+    e += [(base + i, leaves + 60 * i + j) for i in range(fertile) for j in range(60)]
+    n = leaves + 60 * fertile
+    e += [(n - 1 + j, n + j) for j in range(tail)]
+    return G.from_edges(n + tail, e)
+
+
+@pytest.mark.parametrize("workers,wide,alone", [(1, 2, 50), (4, 1, 0), (3, 0, 100)])
+def test_emulated_order_and_search(workers, wide, alone):
+    """A leader alone, everything shared, and levels that change from one to the other; unused workgroups."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    kw = dict(workers=workers, wide=wide, alone=alone)
+    for name in ("path1", "path2", "star64", "duplicates", "unsorted", "grid24x20", "random1500"):
+        rp, ci = CASES[name]()
+        n = len(rp) - 1
+        perm, info = E.run_team(rp, ci, n - 1, tag0=0, **kw)
+        assert info[0] == 0 and info[1] == n and np.array_equal(perm, O.cm(rp, ci, n - 1)), name
+        _, s, it, _ = O.peripheral(rp, ci)
+        perm, info = E.run_team(rp, ci, -1, mode=2, speculate=3 if alone else 0, **kw)
+        assert (info[3], info[4]) == (s, it) and np.array_equal(perm, O.cm(rp, ci, s)), name
+
+
+def test_emulated_ends():
+    """Directed rows, a disconnected matrix, a stage region that is too small, and the watchdog."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    directed = G.directed_with_empty_rows(2000, 1500, 24, 2)
+    perm, info = E.run_team(*directed, 0)
+    assert info[0] == 0 and np.array_equal(perm, O.cm(*directed, 0))
+    perm, info = E.run_team(*G.from_edges(10, [(0, 1), (1, 2), (5, 6)]), 0)
+    assert info[0] == 0 and info[1] == 3 and perm[:3].tolist() == [0, 1, 2]
+    assert E.run_team(*CASES["random1500"](), 0, cap=40)[1][0] == 2
+    assert E.run_team(*CASES["grid24x20"](), 0, timeout_s=0.0)[1][0] == 1
+
+
+GPU_CASES = {
+    "grid32768": lambda: _stencil("stencil2d", 128, 256),  # one workgroup's
+    "grid32769": lambda: _stencil("stencil2d", 3, 10923),  # narrow: the leader's local levels throughout
+    "stencil33": lambda: _stencil("stencil3d", 33, 33, 33),
+    "past_bitmap": lambda: _stencil("stencil2d", 5, 52430),  # 262,150 rows: more than the leader's bitmap has bits
+    "random": lambda: G.random_connected(60000, 500000, seed=9),  # a few wide levels, of several chunks a member
+    "rows63": lambda: _regular(40000, 63, 3),
+    "directed": lambda: G.directed_with_empty_rows(50000, 40000, 24, 2),
+    "lopsided": lambda: _lopsided(780, 520, 3000),  # a stage region overflows: the batch engine takes over
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(GPU_CASES))
+def test_gpu_context(name):
+    rp, ci = GPU_CASES[name]()
+    m = P.CSR(rp, ci)
+    print("[case]", name, m.rows, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        if name == "directed":  # only from node 0 is every node reached
+            s = 0
+        else:
+            _, s, it, _ = O.peripheral(rp, ci)
+            assert c.order() == (s, it)
+            assert np.array_equal(c.perm(), O.cm(rp, ci, s))
+            assert c.find_start() == s and c.timing().start_iterations == it
+        for start in (s, 0):  # stages and tags of one launch under the next
+            c.run(start)
+            assert np.array_equal(c.perm(), O.cm(rp, ci, start))
+        team = c.timing().workers == 128
+        assert team == (name not in ("grid32768", "lopsided"))
+
+
+@pytest.mark.gpu
+def test_gpu_reload_and_refuse():
+    """A larger matrix after a smaller one (the memory grows), a disconnected one, and the smaller one again."""
+    small, big = GPU_CASES["stencil33"](), G.random_connected(300000, 300000, seed=4)
+    apart = G.from_edges(SOLO + 9, [(i, i + 1) for i in range(SOLO)])
+    with P.RcmContext(timeout_ms=20000) as c:
+        for rp, ci in (small, big, apart, small):
+            print("[case]", len(rp) - 1, flush=True)
+            c.load(P.CSR(rp, ci))
+            if rp is apart[0]:
+                with pytest.raises(P.RcmError) as e:
+                    c.order()
+                assert e.value.status == P.RCM_ENOTCONNECTED
+            else:
+                c.run(5)
+                assert np.array_equal(c.perm(), O.cm(rp, ci, 5))
