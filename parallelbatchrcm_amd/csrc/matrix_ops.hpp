@@ -397,25 +397,70 @@ __global__ __launch_bounds__(kT) void k_long_rows(const int32_t* rp, int32_t n, 
   long_len[r] = l > kShortRow ? (uint32_t)l : 0u;
 }
 
-// Each row of at most kShortRow entries sorted by column, stably (insertion sort; the entries of a row are in
-// input order after the row sort, so equal columns keep it).
+// A workgroup on kRowsPerGroup consecutive rows takes their entries kT at a time, whatever the rows' lengths, and finds
+// an entry's row by search in LDS: a hub row is shared by the group, and short rows load coalesced (against a thread a
+// row, links inserted in an R-MAT graph of 65k rows, 2M entries: 25 against 2682 us).
+struct RowGroup {
+  int32_t rp[kRowsPerGroup + 1];
+};
+__device__ __forceinline__ void row_group_load(RowGroup& sm, const int32_t* rp, int32_t n, int32_t x0) {
+  if (threadIdx.x <= (uint32_t)kRowsPerGroup) sm.rp[threadIdx.x] = rp[min(x0 + (int32_t)threadIdx.x, n)];
+  __syncthreads();
+}
+// The row (of the group) that holds entry k: the last that begins at or before it.
+__device__ __forceinline__ int row_group_find(const RowGroup& sm, int32_t k) {
+  int j = 0;
+#pragma unroll
+  for (int s = kRowsPerGroup / 2; s > 0; s >>= 1)
+    if (sm.rp[j + s] <= k) j += s;
+  return j;
+}
+
+struct SortSmem {
+  RowGroup g;
+  uint32_t at[kRowsPerGroup + 1];  // the short rows' entries before each row
+  uint32_t col[kRowsPerGroup * kShortRow];
+  uint32_t idx[kRowsPerGroup * kShortRow];
+};
+
+// Each row of at most kShortRow entries sorted by column, stably: the group's short rows in LDS, an entry's place the
+// count of entries that go before it. (The entries of a row are in input order after the row sort, so equal columns
+// keep it. One thread a row, by insertion in global memory, took 424 us for an R-MAT graph of 65k rows, 1M entries, and
+// 176 us for the 128^3 stencil's lower triangle; so 26 and 92 us.)
 __global__ __launch_bounds__(kT) void k_sort_short_rows(const int32_t* rp, int32_t n, uint64_t* keys,
                                                        uint32_t* idx) {
-  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (r >= n) return;
-  const int32_t b = rp[r], e = rp[r + 1];
-  if (e - b > kShortRow) return;
-  for (int32_t i = b + 1; i < e; ++i) {
-    const uint64_t k = keys[i];
-    const uint32_t v = idx[i];
-    int32_t j = i;
-    while (j > b && (uint32_t)keys[j - 1] > (uint32_t)k) {
-      keys[j] = keys[j - 1];
-      idx[j] = idx[j - 1];
-      --j;
+  RCM_LDS(SortSmem, sm);
+  const int32_t x0 = (int32_t)blockIdx.x * kRowsPerGroup;
+  row_group_load(sm.g, rp, n, x0);
+  if (threadIdx.x < (uint32_t)kWave) {
+    const int j = lane_id();
+    const int32_t l = sm.g.rp[j + 1] - sm.g.rp[j];
+    const uint32_t take = l <= kShortRow ? (uint32_t)l : 0u;
+    const uint32_t inc = rcm::wave_incl_scan(take);
+    sm.at[j] = inc - take;
+    if (j == kWave - 1) sm.at[kRowsPerGroup] = inc;
+  }
+  __syncthreads();
+  const int32_t e0 = sm.g.rp[0], e1 = sm.g.rp[kRowsPerGroup];
+  for (int32_t k = e0 + (int32_t)threadIdx.x; k < e1; k += kT) {
+    const int j = row_group_find(sm.g, k);
+    const uint32_t o = sm.at[j] + (uint32_t)(k - sm.g.rp[j]);
+    if (sm.at[j + 1] > sm.at[j]) {
+      sm.col[o] = (uint32_t)keys[k];
+      sm.idx[o] = idx[k];
     }
-    keys[j] = k;
-    idx[j] = v;
+  }
+  __syncthreads();
+  for (int32_t k = e0 + (int32_t)threadIdx.x; k < e1; k += kT) {
+    const int j = row_group_find(sm.g, k);
+    const uint32_t b = sm.at[j], e = sm.at[j + 1];
+    if (b == e) continue;
+    const uint32_t o = b + (uint32_t)(k - sm.g.rp[j]), c = sm.col[o];
+    uint32_t before = 0;
+    for (uint32_t q = b; q < e; ++q) before += (sm.col[q] < c || (sm.col[q] == c && q < o)) ? 1u : 0u;
+    const int32_t dst = sm.g.rp[j] + (int32_t)before;
+    keys[dst] = ((uint64_t)(uint32_t)(x0 + j) << 32) | c;
+    idx[dst] = sm.idx[o];
   }
 }
 
@@ -592,24 +637,23 @@ __global__ __launch_bounds__(kT) void k_sym_place_transposes(const uint64_t* tke
 
 // flag[0] = 1: an empty row; flag[1] = 1: an entry (r, c) without (c, r) (columns are sorted)
 __global__ __launch_bounds__(kT) void k_struct_checks(const int32_t* rp, const int32_t* ci, int32_t n, uint32_t* flag) {
-  const int64_t r = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (r >= n) return;
-  const int32_t a = rp[r], b = rp[r + 1];
-  if (a == b) flag[0] = 1u;
-  for (int32_t k = a; k < b; ++k) {
-    const int32_t c = ci[k];
+  RCM_LDS(RowGroup, sm);
+  const int32_t x0 = (int32_t)blockIdx.x * kRowsPerGroup;
+  row_group_load(sm, rp, n, x0);
+  const int t = (int)threadIdx.x;
+  if (t < kRowsPerGroup && t < n - x0 && sm.rp[t] == sm.rp[t + 1]) flag[0] = 1u;
+  const int32_t e1 = sm.rp[kRowsPerGroup];
+  for (int32_t k = sm.rp[0] + t; k < e1; k += kT) {
+    const int32_t r = x0 + row_group_find(sm, k), c = ci[k];
     int32_t lo = rp[c], hi = rp[c + 1];  // lower bound of r in row c
     while (lo < hi) {
       const int32_t mid = lo + ((hi - lo) >> 1);
-      if (ci[mid] < (int32_t)r)
+      if (ci[mid] < r)
         lo = mid + 1;
       else
         hi = mid;
     }
-    if (lo == rp[c + 1] || ci[lo] != (int32_t)r) {
-      flag[1] = 1u;
-      return;
-    }
+    if (lo == rp[c + 1] || ci[lo] != r) flag[1] = 1u;
   }
 }
 
@@ -651,17 +695,19 @@ __device__ __forceinline__ uint32_t cc_find_cached(uint32_t* parent, uint32_t x)
 // Concurrent union-find: the trees of u and v are hooked, the larger root under the smaller one, with a
 // device-coherent compare-and-swap, so each tree's root is its smallest node. Walks use cached loads; a CAS only
 // succeeds on a true root, and when it fails the walk restarts from the parent it returned, so the larger of the
-// two candidates strictly decreases and the loop ends. (Device-coherent walks measured slower: 5.7 against 4.2 ms
-// for the whole canonicalisation of the 128^3 stencil.)
+// two candidates strictly decreases and the loop ends. A root that a stale line still shows is found out by a coherent
+// load, not by the compare-and-swap: those meet at one word, a few ns each, and everybody's stale root is the same one
+// (all edges of the 128^3 stencil 194 us against 554, of an R-MAT graph with 1M edges 308 against 1431; with every walk
+// device-coherent 569 and 596).
 __device__ __forceinline__ void cc_link(uint32_t* parent, uint32_t u, uint32_t v) {
   uint32_t a = cc_find_cached(parent, u), b = cc_find_cached(parent, v);
   while (a != b) {
     const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
-    uint32_t expected = hi;
-    if (__hip_atomic_compare_exchange_strong(parent + hi, &expected, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT))
+    uint32_t up = ld_u32(parent + hi);
+    if (up == hi && __hip_atomic_compare_exchange_strong(parent + hi, &up, lo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT))
       break;
-    a = cc_find_cached(parent, expected);
+    a = cc_find_cached(parent, up);
     b = cc_find_cached(parent, lo);
   }
 }
@@ -669,13 +715,14 @@ __device__ __forceinline__ void cc_link(uint32_t* parent, uint32_t u, uint32_t v
 // Every edge (u, v), v < u, of each row (sorted columns: each undirected edge once, from its larger end), except
 // the row's first entry when it is below u: k_cc_init already made it u's parent.
 __global__ __launch_bounds__(kT) void k_cc_hook(const int32_t* rp, const int32_t* ci, int32_t n, uint32_t* parent) {
-  const int64_t u = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (u >= n) return;
-  const int32_t k0 = rp[u], k1 = rp[u + 1];
-  for (int32_t k = (k0 < k1 && ci[k0] < (int32_t)u) ? k0 + 1 : k0; k < k1; ++k) {
-    const uint32_t v = (uint32_t)ci[k];
-    if (v >= (uint32_t)u) break;
-    cc_link(parent, (uint32_t)u, v);
+  RCM_LDS(RowGroup, sm);
+  const int32_t x0 = (int32_t)blockIdx.x * kRowsPerGroup;
+  row_group_load(sm, rp, n, x0);
+  const int32_t e1 = sm.rp[kRowsPerGroup];
+  for (int32_t k = sm.rp[0] + (int32_t)threadIdx.x; k < e1; k += kT) {
+    const int j = row_group_find(sm, k);
+    const uint32_t u = (uint32_t)(x0 + j), v = (uint32_t)ci[k];
+    if (v < u && k > sm.rp[j]) cc_link(parent, u, v);
   }
 }
 
@@ -698,35 +745,57 @@ __global__ __launch_bounds__(kT) void k_link_lengths(const int32_t* rp, const ui
   }
 }
 
+struct LinkSmem {
+  RowGroup g;
+  int32_t rp2[kRowsPerGroup];
+  uint32_t link[kRowsPerGroup];  // bit 0: x - 1, bit 1: x + 1
+};
+
 // Row x with its link entries merged in column order (value 1): x - 1 if x is a component root, x + 1 if
-// x + 1 is one. Neither column is already present (the nodes lie in different components).
+// x + 1 is one. A column that a row already holds (structurally unsymmetric matrices only) keeps its place before the
+// link.
 template <class V>
 __global__ __launch_bounds__(kT) void k_link_insert(const int32_t* rp, const int32_t* ci, const V* vals,
                                                    const uint32_t* root, int32_t n, const int32_t* rp2,
                                                    int32_t* ci2, V* vals2) {
-  const int64_t x = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (x >= n) return;
-  int32_t extra[2];
-  int ne = 0;
-  if (x > 0 && root[x] == (uint32_t)x) extra[ne++] = (int32_t)x - 1;
-  if (x + 1 < n && root[x + 1] == (uint32_t)(x + 1)) extra[ne++] = (int32_t)x + 1;
-  int32_t o = rp2[x];
-  int e = 0;
-  for (int32_t k = rp[x]; k < rp[x + 1]; ++k) {
-    const int32_t c = ci[k];
-    while (e < ne && extra[e] < c) {
-      ci2[o] = extra[e++];
-      if (vals) vals2[o] = (V)1;
-      ++o;
+  RCM_LDS(LinkSmem, sm);
+  const int32_t x0 = (int32_t)blockIdx.x * kRowsPerGroup;
+  const int t = threadIdx.x;
+  if (t < kRowsPerGroup) {
+    const int32_t x = x0 + t;
+    uint32_t link = 0;
+    if (x < n) {
+      if (x > 0 && root[x] == (uint32_t)x) link |= 1u;
+      if (x + 1 < n && root[x + 1] == (uint32_t)(x + 1)) link |= 2u;
+      sm.rp2[t] = rp2[x];
     }
+    sm.link[t] = link;
+  }
+  row_group_load(sm.g, rp, n, x0);
+  const int32_t e1 = sm.g.rp[kRowsPerGroup];
+  for (int32_t k = sm.g.rp[0] + t; k < e1; k += kT) {
+    const int j = row_group_find(sm.g, k);
+    const int32_t c = ci[k], x = x0 + j;
+    const uint32_t link = sm.link[j];
+    const int32_t before = ((link & 1u) != 0 && c > x - 1 ? 1 : 0) + ((link & 2u) != 0 && c > x + 1 ? 1 : 0);
+    const int32_t o = sm.rp2[j] + (k - sm.g.rp[j]) + before;
     ci2[o] = c;
     if (vals) vals2[o] = vals[k];
-    ++o;
   }
-  while (e < ne) {
-    ci2[o] = extra[e++];
-    if (vals) vals2[o] = (V)1;
-    ++o;
+  if (t < 2 * kRowsPerGroup) {  // the links themselves, behind the row's entries up to their column
+    const int j = t >> 1;
+    const int32_t x = x0 + j, col = (t & 1) ? x + 1 : x - 1;
+    if ((sm.link[j] >> (t & 1)) & 1u) {
+      int32_t lo = sm.g.rp[j], hi = sm.g.rp[j + 1];
+      while (lo < hi) {
+        const int32_t mid = lo + ((hi - lo) >> 1);
+        if (ci[mid] <= col) lo = mid + 1;
+        else hi = mid;
+      }
+      const int32_t o = sm.rp2[j] + (lo - sm.g.rp[j]) + ((t & 1) && (sm.link[j] & 1u) ? 1 : 0);
+      ci2[o] = col;
+      if (vals) vals2[o] = (V)1;
+    }
   }
 }
 
@@ -917,7 +986,7 @@ int coo_to_csr(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r, 
   if (nnz > 0) x.run(k_coo_keys, groups(nnz, kT), r, c, nnz, rows, cols, keys, idx, flag);
   if (x.read_u32(flag)) return kOpsInvalid;
   // rows first: a stable sort on the row bits alone keeps each row's entries in input order; then every row
-  // by column, stably -- short rows by one thread each, long rows by a radix sort over (long-row ordinal,
+  // by column, stably -- short rows in LDS, long rows by a radix sort over (long-row ordinal,
   // column). Fewer passes over all entries than a sort on both words.
   radix_sort(x, keys, idx, keys2, idx2, nnz, 0, bits_of(rows > 0 ? (uint64_t)(rows - 1) : 0));
   if (nnz > 0) {
@@ -930,7 +999,7 @@ int coo_to_csr(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r, 
       x.run(k_long_rows, groups((int64_t)rows + 1, kT), (const int32_t*)out.rp, rows, long_len, long_cnt);
       scan_u32(x, long_len, long_len, (int64_t)rows + 1, tot);
       scan_u32(x, long_cnt, long_cnt, (int64_t)rows + 1, tot + 1);
-      x.run(k_sort_short_rows, groups(rows, kT), (const int32_t*)out.rp, rows, keys, idx);
+      x.run(k_sort_short_rows, groups(rows, kRowsPerGroup), (const int32_t*)out.rp, rows, keys, idx);
       const uint32_t long_entries = x.read_u32(tot), long_rows = x.read_u32(tot + 1);
       if (x.failed()) return kOpsDevice;
       if (long_rows > 0) {
@@ -967,7 +1036,7 @@ template <class X>
 int components(X& x, int32_t n, const int32_t* rp, const int32_t* ci, uint32_t* root) {
   x.run(k_cc_init, groups(n, kT), rp, ci, n, root);
   x.run(k_cc_finish, groups(n, kT), root, n);
-  x.run(k_cc_hook, groups(n, kT), rp, ci, n, root);
+  x.run(k_cc_hook, groups(n, kRowsPerGroup), rp, ci, n, root);
   x.run(k_cc_finish, groups(n, kT), root, n);
   return x.failed() ? kOpsDevice : kOpsOk;
 }
@@ -1067,7 +1136,7 @@ int canonicalise(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r
   if (symmetric_known) {
     x.run(k_empty_rows, groups(n, kT), (const int32_t*)a.rp, n, flag);
   } else if (!nonsym) {
-    x.run(k_struct_checks, groups(n, kT), (const int32_t*)a.rp, (const int32_t*)a.ci, n, flag);
+    x.run(k_struct_checks, groups(n, kRowsPerGroup), (const int32_t*)a.rp, (const int32_t*)a.ci, n, flag);
     nonsym = x.read_u32(flag + 1) != 0;
   }
   if (nonsym) {
@@ -1099,7 +1168,7 @@ int canonicalise(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r
   b.ci = x.template keep<int32_t>((size_t)nnz2);
   b.vals = vals ? x.template keep<V>((size_t)nnz2) : nullptr;
   if (x.failed()) return kOpsDevice;
-  x.run(k_link_insert<V>, groups(n, kT), (const int32_t*)a.rp, (const int32_t*)a.ci, (const V*)a.vals,
+  x.run(k_link_insert<V>, groups(n, kRowsPerGroup), (const int32_t*)a.rp, (const int32_t*)a.ci, (const V*)a.vals,
         (const uint32_t*)root, n, (const int32_t*)rp2, b.ci, b.vals);
   out = b;
   return x.failed() ? kOpsDevice : kOpsOk;
