@@ -13,6 +13,7 @@
 // Every kernel reads only inside the sizes it is given; malformed inputs are rejected by validation kernels
 // before any kernel that indexes by their values.
 #pragma once
+#include "bucket_csr.hpp"
 #include "device_common.hpp"
 
 namespace rcm_mx {
@@ -31,6 +32,7 @@ constexpr int kTile = kT * kItems;   // 4096
 constexpr int kBins = 256;           // 8-bit radix digits
 constexpr int kShortRow = 64;        // rows up to this length are ordered by rank counting in LDS
 constexpr int kRowsPerGroup = 64;    // rows per workgroup in that kernel (one per lane of wave 0)
+constexpr int kBucketDealers = 256;  // workgroups that count and deal entries to buckets
 
 static_assert(kT == kBins, "one thread per digit");
 
@@ -1028,6 +1030,78 @@ int coo_to_csr(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r, 
   return x.failed() ? kOpsDevice : kOpsOk;
 }
 
+// coo_to_csr, and with `mirror` the symmetrisation, by buckets of rows (bucket_csr.hpp). False, with nothing done, when
+// the entries do not fit it: a record's fields exceed a word, there would be too many buckets, or one would hold more
+// than a workgroup sorts (hub rows).
+template <class X, class V>
+bool bucket_csr(X& x, int32_t rows, int64_t nnz, const int32_t* r, const int32_t* c, const V* vals, bool mirror,
+                Csr<V>& out, bool* nonsym, int* rc) {
+  using G = typename X::Buckets;
+  if (rows < 1 || nnz <= 0 || nnz > INT32_MAX / 2) return false;
+  const int64_t most = mirror ? 2 * nnz : nnz;  // records
+  BucketJob J{};
+  J.r = r;
+  J.c = c;
+  J.nnz = nnz;
+  J.rows = rows;
+  J.mirror = mirror ? 1 : 0;
+  J.col_bits = bits_of((uint64_t)rows - 1);
+  J.idx_bits = bits_of((uint64_t)nnz - 1);
+  // half of a bucket's capacity on average: the rest is for rows that are not spread evenly
+  J.sh = G::ROWBITS;
+  while (J.sh > 0 && (most << J.sh) / rows > G::CAP / 2) --J.sh;
+  J.buckets = (int32_t)groups(rows, (int64_t)1 << J.sh);
+  if (J.sh + J.col_bits + J.idx_bits + 1 > 63 || J.buckets > G::MAXB) return false;
+  const int64_t wgs = std::min<int64_t>(kBucketDealers, groups(nnz, 4 * G::T));
+  J.per = groups(nnz, wgs);
+  const int64_t m = (int64_t)J.buckets * wgs;
+  uint32_t* table = x.template alloc<uint32_t>((size_t)m + 1);
+  uint32_t* base = x.template alloc<uint32_t>((size_t)J.buckets + 1);
+  uint32_t* kept = x.template alloc<uint32_t>((size_t)J.buckets + 1);
+  uint32_t* flag = x.template alloc<uint32_t>(3);  // largest bucket or ~0; then k_bucket_sort's words
+  *rc = kOpsDevice;
+  if (x.failed()) return true;
+  x.run(k_fill_u32, 1, flag, (int64_t)3, 0u);
+  x.run_wide(k_bucket_count<G>, wgs, G::T, J, table, flag);
+  scan_u32(x, table, table, m, table + m);
+  x.run(k_bucket_bases, groups((int64_t)J.buckets + 1, kT), (const uint32_t*)table, J.buckets, (uint32_t)wgs, base, flag);
+  uint32_t h[3];
+  x.read_words(h, flag, 1);
+  if (x.failed()) return true;
+  *rc = kOpsInvalid;
+  if (h[0] == ~0u) return true;
+  if (h[0] > (uint32_t)G::CAP) return false;
+  *rc = kOpsDevice;
+  uint64_t* rec = x.template alloc<uint64_t>((size_t)most);
+  out.rows = out.cols = rows;
+  out.rp = x.template keep<int32_t>((size_t)rows + 1);
+  out.ci = x.template keep<int32_t>((size_t)most);
+  out.vals = vals ? x.template keep<V>((size_t)most) : nullptr;
+  if (x.failed()) return true;
+  x.run_wide(k_bucket_deal<G>, wgs, G::T, J, (const uint32_t*)table, rec);
+  x.run_wide(k_bucket_sort<G, V>, J.buckets, G::T, J, (const uint32_t*)base, (const uint64_t*)rec, vals, out.rp, out.ci,
+             out.vals, kept, flag + 1);
+  x.read_words(h, flag + 1, 2);
+  uint32_t total = 0;
+  x.read_words(&total, base + J.buckets, 1);
+  if (x.failed()) return true;
+  *nonsym = h[0] != 0;
+  out.nnz = (int64_t)total - (int64_t)h[1];
+  if (h[1] > 0) {
+    Csr<V> b = out;
+    b.rp = x.template keep<int32_t>((size_t)rows + 1);
+    b.ci = x.template keep<int32_t>((size_t)out.nnz);
+    b.vals = vals ? x.template keep<V>((size_t)out.nnz) : nullptr;
+    if (x.failed()) return true;
+    scan_u32(x, kept, kept, (int64_t)J.buckets + 1, (uint32_t*)nullptr);
+    x.run(k_bucket_close<V>, J.buckets, J, (const uint32_t*)base, (const uint32_t*)kept, (const int32_t*)out.rp,
+          (const int32_t*)out.ci, (const V*)out.vals, b.rp, b.ci, b.vals);
+    out = b;
+  }
+  *rc = x.failed() ? kOpsDevice : kOpsOk;
+  return true;
+}
+
 // Components of a structurally symmetric matrix: root[v] = the smallest node of v's component. The forest starts
 // from each node's smallest lower neighbour, is flattened, and then every lower edge is hooked. (Sampled linking in
 // the Afforest scheme, two rounds of first and second row entries and then only rows outside node 0's tree, measured
@@ -1073,11 +1147,15 @@ int canonicalise(X& x, int32_t rows, int32_t cols, int64_t nnz, const int32_t* r
                  bool check_sym, Csr<V>& out, int64_t* links_out) {
   Csr<V> a;
   uint64_t* skeys = nullptr;
-  int rc = coo_to_csr(x, rows, cols, nnz, r, c, vals, a, &skeys);
-  if (rc) return rc;
+  int rc = kOpsOk;
   bool symmetric_known = false;  // the pair pass decided structural symmetry
   bool nonsym = false;           // the result is not structurally symmetric: the directed repair runs
-  if (check_sym && nnz > 0) {
+  const bool bucketed = rows == cols && bucket_csr(x, rows, nnz, r, c, vals, check_sym, a, &nonsym, &rc);
+  if (!bucketed) rc = coo_to_csr(x, rows, cols, nnz, r, c, vals, a, &skeys);
+  if (rc) return rc;
+  if (bucketed) {
+    symmetric_known = check_sym && !nonsym;
+  } else if (check_sym && nnz > 0) {
     uint32_t* tot = x.template alloc<uint32_t>(2);
     uint32_t* odd = x.template alloc<uint32_t>((size_t)nnz + 1);
     if (x.failed()) return kOpsDevice;

@@ -20,7 +20,13 @@ struct EmuExec {
   template <class K, class... A>
   void run(K kernel, int64_t grid, A... args) {
     if (bad || grid <= 0) return;
-    emu::launch((unsigned)grid, rcm_mx::kT, false, kernel, args...);
+    run_wide(kernel, grid, rcm_mx::kT, args...);
+  }
+  using Buckets = rcm_mx::BucketGeo<64, 512, 5, 128>;  // several buckets at the tests' sizes
+  template <class K, class... A>
+  void run_wide(K kernel, int64_t grid, int threads, A... args) {
+    if (bad || grid <= 0) return;
+    emu::launch((unsigned)grid, (unsigned)threads, false, kernel, args...);
   }
   template <class T>
   T* get(std::vector<void*>& list, size_t count) {
