@@ -25,6 +25,8 @@
 #define __host__
 #define __forceinline__ inline
 #define __launch_bounds__(x)
+#define __builtin_nontemporal_load(p) (*(p))
+#define __builtin_nontemporal_store(v, p) ((void)(*(p) = (v)))
 
 struct emu_dim3 { unsigned x = 1, y = 1, z = 1; };
 

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import emu_lib as E
+import matrix_ref as M
 import oracle_lib as O
 import parallelbatchrcm_amd as P
 
@@ -128,3 +129,38 @@ def test_gpu(name):
             return m.row_offsets, m.col_ids, m.data, links
 
         _check(name, run)
+
+
+def _permute_case(n):
+    """Rows of 0 to 66 entries in unsorted order, and groups of 64 rows that divide by the 8 XCDs or leave a rest."""
+    rng = np.random.default_rng(n)
+    ln = rng.integers(0, 9, n)
+    ln[rng.integers(0, n, 3)] = [63, 64, 66]
+    rp = np.concatenate([[0], np.cumsum(ln)]).astype(np.int32)
+    ci = rng.integers(0, n, rp[-1]).astype(np.int32)
+    return P.CSR(rp, ci, rng.standard_normal(ci.size)), rng.permutation(n).astype(np.int32)
+
+
+def _check_permuted(m, perm, rp, ci, v):
+    erp, eci, ev = M.permute_ref(m.row_offsets, m.col_ids, m.data, perm)
+    np.testing.assert_array_equal(rp, erp)
+    np.testing.assert_array_equal(ci, eci)
+    np.testing.assert_array_equal(v, ev)
+
+
+@pytest.mark.parametrize("n", [5, 64, 511, 513, 1088])
+def test_emulated_permute(n):
+    m, perm = _permute_case(n)
+    rc, rp, ci, v = E.permute(m.row_offsets, m.col_ids, m.data, perm)
+    assert rc == 0
+    _check_permuted(m, perm, rp, ci, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [5, 64, 511, 513, 1088, 70001])
+def test_gpu_permute(n):
+    print("[case] permute", n, flush=True)
+    m, perm = _permute_case(n)
+    with P.MatrixOps() as ops:
+        b = ops.permute(m, perm)
+    _check_permuted(m, perm, b.row_offsets, b.col_ids, b.data)
