@@ -89,7 +89,8 @@ enum rcm_param {
                                 WORKERS, SORT, STRICT, PROFILE, CLAIM_FILTER and BATCH_CAP keep their defaults),
                                 whatever the variant, matrices whose rows have at most 64 entries are ordered by
                                 one workgroup each up to 32,768 rows in a context, 65,536 in a set (in a large
-                                set or a serving lane more), and in a context beyond that by a team of 128:
+                                set or a serving lane more), and in a context beyond that by a team of 128; in a
+                                context, longer rows from 262,144 entries on by variant 4:
                                 0 = 256 threads, 2048 adjacency slots, 256 parents, 4-bit digits (serving
                                     lanes)
                                 1 = 512 threads, 2048 slots, 256 parents, 4-bit digits (rcm_ctx default)

@@ -420,11 +420,29 @@ int wait_stream(rcm_ctx* c, hipEvent_t ev, int64_t limit_ms) {
   }
 }
 
+// Whether no parameter of the batch engine was chosen.
+bool ctx_automatic(const rcm_ctx* c) {
+  return !c->engine_set && c->workers == 0 && !c->strict && !c->profile && c->sort_mode == 0 && c->batch_cap == 0 &&
+         c->claim_filter == kDefaultClaimFilter;
+}
+
+// The batch engine's variant for the loaded matrix. Of its own accord it runs matrices with rows beyond the level
+// engines; from kWideNnz entries on, variant 4's wider batches suit them: start search and order of linked R-MAT graphs on
+// MI355X, variant 1 and 4, 250k entries 1.00 and 0.92 ms, 1M 1.47 and 1.20, 8M 5.75 and 4.13; a random graph of 100k rows
+// of 100 entries 1.92 and 1.34; below, R-MAT of 100k entries 0.63 and 0.63, of 13k 0.54 and 0.57.
+constexpr int64_t kWideVariant = 4;
+constexpr int64_t kWideNnz = (int64_t)1 << 18;
+bool ctx_wide(const rcm_ctx* c) {
+  return ctx_automatic(c) && c->maxdeg > (uint32_t)kSoloMaxRow && c->nnz >= kWideNnz;
+}
+int64_t ctx_variant(const rcm_ctx* c) { return ctx_wide(c) ? kWideVariant : c->variant; }
+
 int workers_for(rcm_ctx* c) {
-  if (c->variant == kLevelVariant) return 0;
+  const int64_t variant = ctx_variant(c);
+  if (variant == kLevelVariant) return 0;
   int w = (int)c->workers;
-  if (w <= 0) w = c->n > 16384 ? 256 : 64;  // measured on MI355X: 128-256 is best from 65k to 2M nodes
-  return std::max(1, std::min(w, c->max_resident[c->variant]));
+  if (w <= 0) w = c->n > 16384 || ctx_wide(c) ? 256 : 64;  // measured on MI355X: 128-256 is best from 65k to 2M nodes
+  return std::max(1, std::min(w, c->max_resident[variant]));
 }
 
 int variant_threads(int64_t v) { return v == kLevelVariant ? kLevelThreads : kVarThreads[v]; }
@@ -456,9 +474,7 @@ int run_level(rcm_ctx* c, int32_t start, bool bfs) {
 // Whether a level engine (one workgroup, or a team) takes the loaded matrix: it fits, and no parameter of the batch
 // engine was chosen.
 bool ctx_quick(const rcm_ctx* c) {
-  return !c->engine_set && c->workers == 0 && !c->strict && !c->profile && c->sort_mode == 0 && c->batch_cap == 0 &&
-         c->claim_filter == kDefaultClaimFilter && c->maxdeg <= (uint32_t)kSoloMaxRow && c->n <= kTeamMaxN &&
-         !c->team_off;
+  return ctx_automatic(c) && c->maxdeg <= (uint32_t)kSoloMaxRow && c->n <= kTeamMaxN && !c->team_off;
 }
 
 // One launch of the level engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl. False when
@@ -575,9 +591,10 @@ int run_engine(rcm_ctx* c, int32_t start, bool bfs, bool levels = false) {
   RCM_HIP(hipEventRecord(c->ev[0], c->stream));
   hipLaunchKernelGGL(k_init, dim3(init_blocks), dim3(256), 0, c->stream, a, start, bclear);
   RCM_HIP(hipEventRecord(c->ev[1], c->stream));
-  void* kern = reorder_kernel((int)c->variant, c->strict != 0, bfs, prof, levels && !bfs);
+  const int variant = (int)ctx_variant(c);
+  void* kern = reorder_kernel(variant, c->strict != 0, bfs, prof, levels && !bfs);
   void* args[] = {&a};
-  RCM_HIP(hipLaunchKernel(kern, dim3(workers), dim3(kVarThreads[c->variant]), args, 0, c->stream));
+  RCM_HIP(hipLaunchKernel(kern, dim3(workers), dim3(kVarThreads[variant]), args, 0, c->stream));
   RCM_HIP(hipEventRecord(c->ev[2], c->stream));
   RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
   RCM_HIP(hipEventRecord(c->ev[3], c->stream));

@@ -107,3 +107,29 @@ def test_gpu_reload_and_refuse():
             else:
                 c.run(5)
                 assert np.array_equal(c.perm(), O.cm(rp, ci, 5))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entries", [(1 << 18) - 4, 1 << 18])
+def test_gpu_context_with_long_rows(entries):
+    """Rows beyond the level engines, either side of the count from which the batch engine's wider variant runs."""
+    n = 3000
+    rng = np.random.default_rng(2)
+    key = np.unique(rng.integers(0, n, 2 * entries) * n + rng.integers(0, n, 2 * entries))
+    a, b = key // n, key % n
+    up = a < b
+    a, b = a[up], b[up]
+    chain = b == a + 1  # joins every node
+    keep = np.concatenate([rng.permutation(np.flatnonzero(~chain))[:(entries - 2 * (n - 1) - n) // 2]])
+    a, b = np.concatenate([a[keep], np.arange(n - 1)]), np.concatenate([b[keep], np.arange(1, n)])
+    r = np.concatenate([a, b, np.arange(n)])
+    c = np.concatenate([b, a, np.arange(n)])
+    rp, ci, _ = O.convert(n, r.astype(np.int32), c.astype(np.int32), np.ones(r.size))
+    assert len(ci) == entries and (rp[1:] - rp[:-1]).max() > 64
+    print("[case]", entries, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(P.CSR(rp, ci))
+        _, s, it, _ = O.peripheral(rp, ci)
+        assert c.order() == (s, it)
+        assert np.array_equal(c.perm(), O.cm(rp, ci, s))
+        assert c.timing().workers == (256 if entries >= 1 << 18 else 64)
