@@ -408,6 +408,13 @@ bool ensure_team(rcm_ctx* c, int32_t n) {
   return true;
 }
 
+// Between two looks at an event, `ms` into the wait: a sleep takes 70 us however short, most of a small matrix's time, so
+// the first milliseconds only yield.
+void poll_pause(int64_t ms) {
+  if (ms < 8) std::this_thread::yield();
+  else std::this_thread::sleep_for(std::chrono::microseconds(20));
+}
+
 int wait_stream(rcm_ctx* c, hipEvent_t ev, int64_t limit_ms) {
   const auto t0 = std::chrono::steady_clock::now();
   for (;;) {
@@ -416,7 +423,7 @@ int wait_stream(rcm_ctx* c, hipEvent_t ev, int64_t limit_ms) {
     if (q != hipErrorNotReady) return RCM_EDEVICE;
     const auto ms = std::chrono::duration_cast<std::chrono::milliseconds>(std::chrono::steady_clock::now() - t0).count();
     if (ms > limit_ms) return RCM_ETIMEOUT;
-    std::this_thread::sleep_for(std::chrono::microseconds(20));
+    poll_pause(ms);
   }
 }
 
@@ -514,14 +521,17 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       hipLaunchKernelGGL(k_team<TeamG>, dim3(kTeamMax), dim3(TeamG::T), 0, c->stream, a);
     } else {
       const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
+      // the result goes to pinned host memory as the kernel ends: no copy after it
       hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
-                         budget, c->ctl);
+                         budget, c->h_ctl);
     }
     RCM_HIP(hipGetLastError());
     RCM_HIP(hipEventRecord(c->ev[2], c->stream));
-    RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
-    RCM_HIP(hipEventRecord(c->ev[3], c->stream));
-    const int st = wait_stream(c, c->ev[3], c->timeout_ms + 10000);
+    if (team) {
+      RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
+      RCM_HIP(hipEventRecord(c->ev[3], c->stream));
+    }
+    const int st = wait_stream(c, c->ev[team ? 3 : 2], c->timeout_ms + 10000);
     if (st) return st;
     float ms_init = 0.f, ms = 0.f;
     if (team) RCM_HIP(hipEventElapsedTime(&ms_init, c->ev[0], c->ev[1]));
@@ -971,7 +981,7 @@ int batch_wait(rcm_batch* b, hipEvent_t ev) {
     if (q != hipErrorNotReady) return RCM_EDEVICE;
     const auto ms = std::chrono::duration_cast<std::chrono::milliseconds>(std::chrono::steady_clock::now() - t0).count();
     if (ms > b->timeout_ms + 10000) return RCM_ETIMEOUT;
-    std::this_thread::sleep_for(std::chrono::microseconds(50));
+    poll_pause(ms);
   }
 }
 
