@@ -60,7 +60,7 @@ struct HipExec {
   uint32_t* h_word;  // pinned, kPinnedWords words
   bool bad = false;
 
-  using Buckets = BucketGeo<1024, 8192, 11, 8192>;  // 512 threads, 4096 records: 681 us against 634, more buckets to deal to
+  using Buckets = BucketGeo<512, 4096, 11, 16384, 1024, 7>;
 
   template <class K, class... A>
   void run(K kernel, int64_t grid, A... args) {

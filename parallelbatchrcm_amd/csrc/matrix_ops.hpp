@@ -32,7 +32,7 @@ constexpr int kTile = kT * kItems;   // 4096
 constexpr int kBins = 256;           // 8-bit radix digits
 constexpr int kShortRow = 64;        // rows up to this length are ordered by rank counting in LDS
 constexpr int kRowsPerGroup = 64;    // rows per workgroup in that kernel (one per lane of wave 0)
-constexpr int kBucketDealers = 256;  // workgroups that count and deal entries to buckets
+constexpr int kBucketDealers = 512;  // workgroups that count and deal entries to buckets
 
 static_assert(kT == kBins, "one thread per digit");
 
@@ -1097,20 +1097,21 @@ bool bucket_csr(X& x, int32_t rows, int64_t nnz, const int32_t* r, const int32_t
   J.sh = G::ROWBITS;
   while (J.sh > 0 && (most << J.sh) / rows > G::CAP / 2) --J.sh;
   J.buckets = (int32_t)groups(rows, (int64_t)1 << J.sh);
-  if (J.sh + J.col_bits + J.idx_bits + 1 > 63 || J.buckets > G::MAXB) return false;
-  const int64_t wgs = std::min<int64_t>(kBucketDealers, groups(nnz, 4 * G::T));
+  J.fb = J.buckets > G::COARSE ? G::FB : 0;
+  J.groups = (int32_t)groups(J.buckets, (int64_t)1 << J.fb);
+  if (J.fb + J.sh + J.col_bits + J.idx_bits + 1 > 63 || J.buckets > G::MAXB) return false;
+  const int64_t wgs = std::min<int64_t>(kBucketDealers, groups(nnz, 2 * G::TD));
   J.per = groups(nnz, wgs);
-  const int64_t m = (int64_t)J.buckets * wgs;
-  uint32_t* table = x.template alloc<uint32_t>((size_t)m + 1);
+  uint32_t* table = x.template alloc<uint32_t>((size_t)J.buckets * wgs);
+  uint32_t* group = x.template alloc<uint32_t>((size_t)J.groups * wgs);
   uint32_t* base = x.template alloc<uint32_t>((size_t)J.buckets + 1);
   uint32_t* kept = x.template alloc<uint32_t>((size_t)J.buckets + 1);
   uint32_t* flag = x.template alloc<uint32_t>(3);  // largest bucket or ~0; then k_bucket_sort's words
   *rc = kOpsDevice;
   if (x.failed()) return true;
   x.run(k_fill_u32, 1, flag, (int64_t)3, 0u);
-  x.run_wide(k_bucket_count<G>, wgs, G::T, J, table, flag);
-  scan_u32(x, table, table, m, table + m);
-  x.run(k_bucket_bases, groups((int64_t)J.buckets + 1, kT), (const uint32_t*)table, J.buckets, (uint32_t)wgs, base, flag);
+  x.run_wide(k_bucket_count<G>, wgs, G::TD, J, table, group, flag);
+  x.run(k_bucket_total, groups((int64_t)J.buckets + 1, kT), (const uint32_t*)table, J.buckets, (uint32_t)wgs, base, flag);
   uint32_t h[3];
   x.read_words(h, flag, 1);
   if (x.failed()) return true;
@@ -1119,14 +1120,28 @@ bool bucket_csr(X& x, int32_t rows, int64_t nnz, const int32_t* r, const int32_t
   if (h[0] > (uint32_t)G::CAP) return false;
   *rc = kOpsDevice;
   uint64_t* rec = x.template alloc<uint64_t>((size_t)most);
+  V* val = vals ? x.template alloc<V>((size_t)most) : nullptr;
+  uint64_t* rec2 = J.fb ? x.template alloc<uint64_t>((size_t)most) : nullptr;
+  V* val2 = J.fb && vals ? x.template alloc<V>((size_t)most) : nullptr;
   out.rows = out.cols = rows;
   out.rp = x.template keep<int32_t>((size_t)rows + 1);
   out.ci = x.template keep<int32_t>((size_t)most);
   out.vals = vals ? x.template keep<V>((size_t)most) : nullptr;
   if (x.failed()) return true;
-  x.run_wide(k_bucket_deal<G>, wgs, G::T, J, (const uint32_t*)table, rec);
-  x.run_wide(k_bucket_sort<G, V>, J.buckets, G::T, J, (const uint32_t*)base, (const uint64_t*)rec, vals, out.rp, out.ci,
-             out.vals, kept, flag + 1);
+  scan_u32(x, base, base, (int64_t)J.buckets + 1, (uint32_t*)nullptr);
+  scan_u32(x, group, group, (int64_t)J.groups * wgs, (uint32_t*)nullptr);
+  x.run_wide(k_bucket_deal<G, V>, wgs, G::TD, J, (const uint32_t*)group, vals, rec, val);
+  if (J.fb) {
+    // a workgroup a tile (16 tiles for 2: 140 us against 133); `kept` is free until the sort: the buckets' cursors
+    const int32_t each = (int32_t)std::min<int64_t>(64, groups(most, (int64_t)J.groups * G::TILE));
+    x.run(k_bucket_cursors, groups(J.buckets, kT), (const uint32_t*)base, J.buckets, kept);
+    x.run_wide(k_bucket_split<G, V>, (int64_t)J.groups * each, G::TD, J, (const uint32_t*)base, kept, each,
+               (const uint64_t*)rec, (const V*)val, rec2, val2);
+    rec = rec2;
+    val = val2;
+  }
+  x.run_wide(k_bucket_sort<G, V>, J.buckets, G::T, J, (const uint32_t*)base, (const uint64_t*)rec, (const V*)val, out.rp,
+             out.ci, out.vals, kept, flag + 1);
   x.read_words(h, flag + 1, 2);
   uint32_t total = 0;
   x.read_words(&total, base + J.buckets, 1);

@@ -22,7 +22,7 @@ struct EmuExec {
     if (bad || grid <= 0) return;
     run_wide(kernel, grid, rcm_mx::kT, args...);
   }
-  using Buckets = rcm_mx::BucketGeo<64, 512, 5, 128>;  // several buckets at the tests' sizes
+  using Buckets = rcm_mx::BucketGeo<64, 256, 5, 128, 64, 3>;  // several buckets and groups at the tests' sizes
   template <class K, class... A>
   void run_wide(K kernel, int64_t grid, int threads, A... args) {
     if (bad || grid <= 0) return;
