@@ -32,11 +32,18 @@
 #pragma once
 #include "engine_solo.hpp"
 
+// Where the tests hold a member up: between its word and its look at the others' (0 a meeting, 1 a redistribution), and
+// before a workgroup that joins reads the leader's record (2). Nothing here relies on members keeping pace.
+#ifndef RCM_TEAM_LINGER
+#define RCM_TEAM_LINGER(where, member, tag)
+#endif
+
 namespace rcm {
 
 constexpr int kTeamMax = 128;        // members: a lane polls the words of two neighbours
 constexpr int kTeamPer = kTeamMax / kWave;
 constexpr int kTeamWordStride = 16;  // a member's words lie on a 128-byte line of their own
+constexpr int kTeamSplitWord = 2;    // behind the two of the meetings
 constexpr int kTeamNodeBits = 24;    // of a node or count; with a degree or member count at most 32 bits
 constexpr int kTeamPartBits = 18;    // of a parent's index in its member's part
 constexpr int32_t kTeamLocalN = 1 << 18;  // the bitmap of the leader's local levels
@@ -64,8 +71,10 @@ struct TeamArgs {
   // parents of the levels of even and odd tags: kTeamMax regions of `cap` entries of two words, row begin | tag << 32 and
   // degree | node << 7 | tag << 32; no word holds a tag above tag0 at the launch (with tag0 0: anything)
   uint64_t* stage[2];
-  // per member, zero at the launch: tag << 32 | (the leader's: workgroups started) << 24 | parents, its claims of that
-  // level made; and tag << 32 | next members << 24 | children, its part of a redistribution
+  // per member, zero at the launch. Words 0 and 1, levels of even and odd tags: tag << 32 | (the leader's: workgroups
+  // started) << 24 | parents, its claims of that level made. A member may be through with the next level's claims before
+  // another has read its word of this one, so they alternate; it is not through with the meeting after that, which needs
+  // the other. Word 2: tag << 32 | next members << 24 | children, its part of a redistribution.
   uint64_t* words;
   uint64_t* rec;     // two records of two words: the state of a redistributed level for workgroups that join it
   Control* ctl;      // ticket, done and error zero at the launch
@@ -179,8 +188,9 @@ __device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, int which, uint
 }
 __device__ __forceinline__ uint32_t word_count(uint64_t w) { return (uint32_t)w & ((1u << kTeamNodeBits) - 1u); }
 
-// The meeting: every member has made its claims of the level. False when the launch is over. Wave 0 has sm.met set when
-// it passes the next barrier.
+// The meeting: every member has made its claims of the level. False when the launch is over, or the pass (the words are
+// those of a later one, sm.verdict is TEAM_PASSED): of a level without parents nobody waits for its members to read the
+// words. Wave 0 has sm.met set when it passes the next barrier.
 template <class G>
 __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
                                           uint64_t deadline) {
@@ -197,8 +207,9 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
   TeamWords r;
   if (wave_id() == 0) {
     if (lane_id() == 0)
-      st_sync(team_word(a, sm.g, 0), ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
-    const uint32_t v = team_poll(a, 0, lv.tag, lv.members, deadline, r);
+      st_sync(team_word(a, sm.g, (int)(lv.tag & 1u)), ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
+    RCM_TEAM_LINGER(0, sm.g, lv.tag);
+    const uint32_t v = team_poll(a, (int)(lv.tag & 1u), lv.tag, lv.members, deadline, r);
     if (lane_id() == 0) sm.verdict = v;
   }
   __syncthreads();
@@ -234,7 +245,8 @@ __device__ __forceinline__ uint32_t team_counts(const TeamArgs& a, TeamSmem<G>& 
                                                 uint64_t deadline) {
   if (wave_id() == 0) {
     TeamWords r;
-    const uint32_t v = team_poll(a, 1, tag, members, deadline, r);
+    RCM_TEAM_LINGER(1, sm.g, tag);
+    const uint32_t v = team_poll(a, kTeamSplitWord, tag, members, deadline, r);
     uint32_t c = 0;
 #pragma unroll
     for (int i = 0; i < kTeamPer; ++i) c += word_count(r.w[i]);
@@ -461,7 +473,7 @@ __device__ __forceinline__ void team_publish(const TeamArgs& a, TeamSmem<G>& sm,
     __builtin_amdgcn_s_waitcnt(0);  // the record is there before the word says so
   }
   if (lane_id() == 0)
-    st_sync(team_word(a, sm.g, 1),
+    st_sync(team_word(a, sm.g, kTeamSplitWord),
             ((uint64_t)lv.tag << 32) |
                 (uint64_t)(((uint32_t)want << kTeamNodeBits) | children));
 }
@@ -683,12 +695,13 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
     else ok = team_chunk<G, G::EPT>(a, sm, lv, here, deadline, nx);
     if (!ok) return TEAM_STOP;
   } else {
-    if (!team_meet<G>(a, sm, lv, here, deadline)) return TEAM_STOP;
+    if (!team_meet<G>(a, sm, lv, here, deadline)) return sm.verdict == TEAM_PASSED ? TEAM_PASSED : TEAM_STOP;
     __syncthreads();
     nx.split = team_split(a, lv.members, sm.met[1], sm.met[2], sm.met[3]);
     nx.marked = true;
     if (sm.met[3] == 0) return TEAM_STOP;
-    if (wave_uniform((uint32_t)wave_id()) == 0u && nx.split) team_publish<G>(a, sm, lv, sm.met[1], team_wanted(a, sm.met[1], sm.met[3]), 0u);
+    if (wave_uniform((uint32_t)wave_id()) == 0u && nx.split)
+      team_publish<G>(a, sm, lv, sm.met[1], team_wanted(a, sm.met[1], sm.met[3]), 0u);
   }
   const int32_t width = (int32_t)sm.met[1];
   __syncthreads();
@@ -723,7 +736,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, ui
     if (wave_id() == 0) {
       uint32_t v = TEAM_ON, tag = 0, gn = 0;
       for (uint32_t spin = 0;; ++spin) {
-        const uint64_t w = ld_sync(team_word(a, 0, 1));
+        const uint64_t w = ld_sync(team_word(a, 0, kTeamSplitWord));
         tag = wave_uniform((uint32_t)(w >> 32));
         gn = wave_uniform((uint32_t)w >> kTeamNodeBits);
         if (tag > seen && (int32_t)gn > sm.g) break;
@@ -733,6 +746,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, ui
         }
         __builtin_amdgcn_s_sleep(4);
       }
+      RCM_TEAM_LINGER(2, sm.g, tag);
       if (lane_id() == 0) {
         sm.verdict = v;
         sm.np = tag;

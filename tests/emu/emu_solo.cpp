@@ -5,6 +5,17 @@
 template <class T, class V>
 inline T __hip_atomic_fetch_or(T* p, V v, int, int) { return __atomic_fetch_or(p, (T)v, __ATOMIC_SEQ_CST); }
 #endif
+#include <unistd.h>
+// holds member emu_linger[1] (-1: all but the leader) up at place emu_linger[0], for a while, on levels of tag emu_linger[2]
+// modulo 5
+static int emu_linger[3] = {-1, -1, -1};
+#define RCM_TEAM_LINGER(where, member, tag)                                                                      \
+  do {                                                                                                           \
+    if (emu_linger[0] == (where) && (emu_linger[1] < 0 ? (member) > 0 : emu_linger[1] == (member)) &&            \
+        (int)((tag) % 5u) == emu_linger[2] && lane_id() == 0)                                                    \
+      usleep(20000);                                                                                             \
+    __builtin_amdgcn_s_waitcnt(0);                                                                               \
+  } while (0)
 #include "engine_team.hpp"
 
 #include <vector>
@@ -75,6 +86,12 @@ int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const i
                                                perm_cat, info, timeout_s)
              : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
                                                    speculate, perm_cat, info, timeout_s);
+}
+
+void emu_team_linger(int where, int member, int phase) {
+  emu_linger[0] = where;
+  emu_linger[1] = member;
+  emu_linger[2] = phase;
 }
 
 // Orders one matrix with a team of `workers` workgroups (engine_team.hpp; 64 threads, 256 slots). wide: parents per

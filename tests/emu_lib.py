@@ -233,8 +233,9 @@ def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.
 
 
 def run_team(rp, ci, start, workers=3, mode=0, speculate=3, wide=2, alone=0, cap=4096, tag0=1000,
-             timeout_s=120.0):
-    """A team of workgroups on one matrix (engine_team.hpp). Returns (perm, info) with info as run_solo's."""
+             linger=(-1, -1, -1), timeout_s=120.0):
+    """A team of workgroups on one matrix (engine_team.hpp). Returns (perm, info) with info as run_solo's. linger: where,
+    which member and on which levels one is held up (emu_team_linger)."""
     L = lib("solo")
     if not hasattr(L, "_team_ready"):
         L.emu_run_team.restype = C.c_int
@@ -246,6 +247,7 @@ def run_team(rp, ci, start, workers=3, mode=0, speculate=3, wide=2, alone=0, cap
     n = rp.shape[0] - 1
     perm = np.full(n, -1, np.int32)
     info = np.zeros(6, np.int32)
+    L.emu_team_linger(*linger)
     rc = L.emu_run_team(n, rp.ctypes.data_as(I32P), ci.ctypes.data_as(I32P), int(start), workers, mode, speculate, wide,
                         alone, cap, tag0, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
     assert rc == 0, "emulator rejected the arguments"

@@ -43,6 +43,22 @@ def test_emulated_order_and_search(workers, wide, alone):
         assert (info[3], info[4]) == (s, it) and np.array_equal(perm, O.cm(rp, ci, s)), name
 
 
+@pytest.mark.parametrize("where", [0, 1, 2])
+@pytest.mark.parametrize("member", [-1, 0, 1])
+def test_emulated_slow_member(where, member):
+    """A member that falls behind the others by several levels' time still reads the words meant for it."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    for name in ("star64", "grid24x20", "random1500"):
+        rp, ci = CASES[name]()
+        _, s, it, _ = O.peripheral(rp, ci)
+        for phase in (0, 3):
+            perm, info = E.run_team(rp, ci, -1, mode=2, workers=4, wide=1, linger=(where, member, phase), timeout_s=30)
+            assert info[0] == 0 and (info[3], info[4]) == (s, it), (name, phase)
+            assert np.array_equal(perm, O.cm(rp, ci, s)), (name, phase)
+
+
 def test_emulated_ends():
     """Directed rows, a disconnected matrix, a stage region that is too small, and the watchdog."""
     pytest.importorskip("emu_lib")
