@@ -500,9 +500,9 @@ def pmc_probe(runs: int, claim_filter: int = -1, variant: int = -1, workers: int
 
 
 def measured_traffic():
-    """HBM bytes per k_reorder launch on the 128^3 stencil from the committed rocprofv3 --pmc summary
-    (profiles/k_reorder_stencil3d_128_traffic.md, line 'traffic_bytes_per_launch: <int>'), or None."""
-    path = os.path.join(ROOT, "profiles", "k_reorder_stencil3d_128_traffic.md")
+    """HBM bytes per k_team launch on the 128^3 stencil from the committed rocprofv3 --pmc summary
+    (profiles/k_team_stencil3d_128_traffic.md, line 'traffic_bytes_per_launch: <int>'), or None."""
+    path = os.path.join(ROOT, "profiles", "k_team_stencil3d_128_traffic.md")
     try:
         for line in open(path):
             if line.startswith("traffic_bytes_per_launch:"):
@@ -623,8 +623,8 @@ def main() -> int:
                    "variant": tune.variant if tune is not None else 0},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(),
-                     "kernel": "k_reorder (persistent)", "kernel_ms": kern_ms, "alg_bytes": balg,
-                     "traffic_source": "profiles/k_reorder_stencil3d_128_traffic.md (the autotuned configuration)",
+                     "kernel": "k_team", "kernel_ms": kern_ms, "alg_bytes": balg,
+                     "traffic_source": "profiles/k_team_stencil3d_128_traffic.md (the autotuned configuration)",
                      "measured_copy_GBs": copy_gbs, "frac_of_measured_copy": achieved / copy_gbs},
         "kernel_nnz_per_s": nnz / (kern_ms * 1e-3),
         "kernel_ms_p50": float(np.percentile(kern, 50)),
