@@ -27,7 +27,7 @@
 //   that has not started, so a launch ends whatever else runs on the GPU; the workgroups a level does without watch
 //   the leader's word for the next redistribution.
 // Measured on MI355X, whole calls, the batch engine before and a team after: one order of the 128^3 stencil 4.09 and 2.29
-// ms (379 levels), start search and order of a geometric graph of 1M points 22.9 and 13.3 ms, of a 48^3 stencil 3.4 and
+// ms (379 levels), start search and order of a geometric graph of 1M points 22.9 and 13.3 to 14.2 ms, of a 48^3 stencil 3.4 and
 // 1.9 ms.
 #pragma once
 #include "engine_solo.hpp"
