@@ -266,7 +266,8 @@ __device__ __forceinline__ uint32_t bucket_lower(const SM& sm, uint32_t a, uint3
 
 // One bucket: sorted, the transposes of evenly stored pairs taken out, and written as rows from the bucket's first record
 // on (rp, ci, vout; with anything taken out these leave gaps, see k_bucket_close). kept[b]: its records that stay
-// (kept[buckets] = 0). out[0] = 1: an evenly stored pair is not symmetric; out[1]: records taken out.
+// (kept[buckets] = 0). out[0] = 1: an evenly stored pair is not symmetric; out[1]: records taken out; out[2]:
+// records.
 // Bound by LDS and the latency of its phases, which three workgroups on a compute unit cover for each other.
 template <class G, class V>
 __global__ __launch_bounds__(G::T) void k_bucket_sort(BucketJob J, const uint32_t* base, const uint64_t* rec,
@@ -419,6 +420,7 @@ __global__ __launch_bounds__(G::T) void k_bucket_sort(BucketJob J, const uint32_
     kept[blockIdx.x] = left;
     if ((int32_t)blockIdx.x == J.buckets - 1) {
       kept[J.buckets] = 0;
+      out[2] = b0 + m;
       rp[J.rows] = (int32_t)(b0 + left);
     }
   }

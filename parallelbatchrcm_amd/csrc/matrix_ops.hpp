@@ -1106,10 +1106,10 @@ bool bucket_csr(X& x, int32_t rows, int64_t nnz, const int32_t* r, const int32_t
   uint32_t* group = x.template alloc<uint32_t>((size_t)J.groups * wgs);
   uint32_t* base = x.template alloc<uint32_t>((size_t)J.buckets + 1);
   uint32_t* kept = x.template alloc<uint32_t>((size_t)J.buckets + 1);
-  uint32_t* flag = x.template alloc<uint32_t>(3);  // largest bucket or ~0; then k_bucket_sort's words
+  uint32_t* flag = x.template alloc<uint32_t>(4);  // largest bucket or ~0; then k_bucket_sort's words
   *rc = kOpsDevice;
   if (x.failed()) return true;
-  x.run(k_fill_u32, 1, flag, (int64_t)3, 0u);
+  x.run(k_fill_u32, 1, flag, (int64_t)4, 0u);
   x.run_wide(k_bucket_count<G>, wgs, G::TD, J, table, group, flag);
   x.run(k_bucket_total, groups((int64_t)J.buckets + 1, kT), (const uint32_t*)table, J.buckets, (uint32_t)wgs, base, flag);
   uint32_t h[3];
@@ -1142,12 +1142,10 @@ bool bucket_csr(X& x, int32_t rows, int64_t nnz, const int32_t* r, const int32_t
   }
   x.run_wide(k_bucket_sort<G, V>, J.buckets, G::T, J, (const uint32_t*)base, (const uint64_t*)rec, (const V*)val, out.rp,
              out.ci, out.vals, kept, flag + 1);
-  x.read_words(h, flag + 1, 2);
-  uint32_t total = 0;
-  x.read_words(&total, base + J.buckets, 1);
+  x.read_words(h, flag + 1, 3);
   if (x.failed()) return true;
   *nonsym = h[0] != 0;
-  out.nnz = (int64_t)total - (int64_t)h[1];
+  out.nnz = (int64_t)h[2] - (int64_t)h[1];
   if (h[1] > 0) {
     Csr<V> b = out;
     b.rp = x.template keep<int32_t>((size_t)rows + 1);
