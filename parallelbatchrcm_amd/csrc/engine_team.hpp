@@ -32,8 +32,8 @@
 #pragma once
 #include "engine_solo.hpp"
 
-// Where the tests hold a member up: between its word and its look at the others' (0 a meeting, 1 a redistribution), and
-// before a workgroup that joins reads the leader's record (2). Nothing here relies on members keeping pace.
+// Where the tests hold a member up: between its word and its look at the others' (0 a meeting, 1 a redistribution),
+// before a workgroup that joins reads the leader's record (2), and before a level's queue entries are stored (3). Nothing here relies on members keeping pace.
 #ifndef RCM_TEAM_LINGER
 #define RCM_TEAM_LINGER(where, member, tag)
 #endif
@@ -557,8 +557,18 @@ __device__ __forceinline__ bool team_place(const TeamArgs& a, TeamSmem<G>& sm, c
     if (tid == 0) team_fail(a, ERR_CAPACITY);
     return false;
   }
-  if (wv == 0 && last && nx.split) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), nx.placed + cnt);
+  // Readers of a redistribution's children look at their tags, so its word goes out first. A part without children, though,
+  // may be of the pass's last level: then the leader reads the queue as soon as it has the members' words, with no meeting
+  // before, and the word waits for the part's queue entries (of all its chunks).
+  const bool word = last && nx.split, barren = nx.placed + cnt == 0;
+  if (wv == 0 && word && !barren) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), nx.placed + cnt);
+  RCM_TEAM_LINGER(3, sm.g, lv.tag);
   if (tid < np) st_sync(&a.perm[q0 + tid], (int32_t)sm.node[tid]);
+  if (word && barren) {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (wv == 0) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), 0u);
+  }
   if (active) {
     const uint32_t xc = ic - vc, xd = id - vd;
 #pragma unroll
@@ -862,8 +872,8 @@ __device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, ui
     if (redo) continue;
     lastdist = (uint32_t)lev;
     // the node of least row length among the last min(32, n - 1) of the last level, later ones winning ties. The last
-    // level's members have stored its queue entries when the pass's last meeting, of no parents, is over; a leader on
-    // its own waits for its stores here.
+    // level's queue entries are there: its members' words of what ended the pass -- a meeting of no parents, or a
+    // redistribution of no children -- went out after them; a leader on its own waits for its stores here.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (wave_id() == 0) {

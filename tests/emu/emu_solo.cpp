@@ -72,35 +72,11 @@ int run(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* c
   }
   return 0;
 }
-}  // namespace
 
-extern "C" {
-// Orders `count` concatenated matrices, one workgroup each. geo: 0 = the geometry of small chunks (128 threads, 256
-// slots, a ring of 64 entries: chunks, their remainders and the ring's overflow at small sizes), 1 = the library's.
-// perm_cat: matrix k's order at sum_{i<k} n[i]; info[6 k ..] = error, placed, steps, start, sweeps, passes.
-int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* ci_off, const int32_t* rpc,
-                 const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate,
-                 int32_t geo, int32_t* perm_cat, int32_t* info, double timeout_s) {
-  if (count <= 0 || workers <= 0) return -1;
-  return geo ? run<SoloGeo<512, 2048, 1 << 16>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode, speculate,
-                                               perm_cat, info, timeout_s)
-             : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
-                                                   speculate, perm_cat, info, timeout_s);
-}
-
-void emu_team_linger(int where, int member, int phase) {
-  emu_linger[0] = where;
-  emu_linger[1] = member;
-  emu_linger[2] = phase;
-}
-
-// Orders one matrix with a team of `workers` workgroups (engine_team.hpp; 64 threads, 256 slots). wide: parents per
-// member wanted, as a power of two. alone: slots of a level its leader takes on its own. cap: entries of a stage region.
-// tag0 0 starts from memory that holds anything. info = error, placed, levels, start, sweeps, passes.
-int emu_run_team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start, int32_t workers, int32_t mode,
-                 int32_t speculate, int32_t wide, int32_t alone, int32_t cap, uint32_t tag0, int32_t* perm,
-                 int32_t* info, double timeout_s) {
-  using G = TeamGeo<64, 256>;
+template <class G>
+int team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start, int32_t workers, int32_t mode,
+         int32_t speculate, int32_t wide, int32_t alone, int32_t cap, uint32_t tag0, int32_t* perm, int32_t* info,
+         double timeout_s) {
   int32_t maxrow = 1;
   for (int32_t i = 0; i < n; ++i) maxrow = std::max(maxrow, rp[i + 1] - rp[i]);
   if (maxrow > kSoloMaxRow || workers > kTeamMax) return -3;
@@ -137,5 +113,39 @@ int emu_run_team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start,
                         ctl.sweeps, ctl.passes};
   std::memcpy(info, v, sizeof(v));
   return 0;
+}
+}  // namespace
+
+extern "C" {
+// Orders `count` concatenated matrices, one workgroup each. geo: 0 = the geometry of small chunks (128 threads, 256
+// slots, a ring of 64 entries: chunks, their remainders and the ring's overflow at small sizes), 1 = the library's.
+// perm_cat: matrix k's order at sum_{i<k} n[i]; info[6 k ..] = error, placed, steps, start, sweeps, passes.
+int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* ci_off, const int32_t* rpc,
+                 const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate,
+                 int32_t geo, int32_t* perm_cat, int32_t* info, double timeout_s) {
+  if (count <= 0 || workers <= 0) return -1;
+  return geo ? run<SoloGeo<512, 2048, 1 << 16>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode, speculate,
+                                               perm_cat, info, timeout_s)
+             : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
+                                                   speculate, perm_cat, info, timeout_s);
+}
+
+void emu_team_linger(int where, int member, int phase) {
+  emu_linger[0] = where;
+  emu_linger[1] = member;
+  emu_linger[2] = phase;
+}
+
+// Orders one matrix with a team of `workers` workgroups (engine_team.hpp). wide: parents per member wanted, as a power of
+// two. alone: slots of a level its leader takes on its own. cap: entries of a stage region. tag0 0 starts from memory that
+// holds anything. geo: 0 = workgroups of one wave (256 slots), 1 = of two waves (512 slots). info = error, placed, levels,
+// start, sweeps, passes.
+int emu_run_team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start, int32_t workers, int32_t mode,
+                 int32_t speculate, int32_t wide, int32_t alone, int32_t cap, uint32_t tag0, int32_t geo, int32_t* perm,
+                 int32_t* info, double timeout_s) {
+  return geo ? team<TeamGeo<128, 512>>(n, rp, ci, start, workers, mode, speculate, wide, alone, cap, tag0, perm, info,
+                                       timeout_s)
+             : team<TeamGeo<64, 256>>(n, rp, ci, start, workers, mode, speculate, wide, alone, cap, tag0, perm, info,
+                                      timeout_s);
 }
 }

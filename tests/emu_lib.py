@@ -233,14 +233,14 @@ def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.
 
 
 def run_team(rp, ci, start, workers=3, mode=0, speculate=3, wide=2, alone=0, cap=4096, tag0=1000,
-             linger=(-1, -1, -1), timeout_s=120.0):
+             linger=(-1, -1, -1), timeout_s=120.0, geo=0):
     """A team of workgroups on one matrix (engine_team.hpp). Returns (perm, info) with info as run_solo's. linger: where,
-    which member and on which levels one is held up (emu_team_linger)."""
+    which member and on which levels one is held up (emu_team_linger). geo: 0 = workgroups of one wave, 1 = of two."""
     L = lib("solo")
     if not hasattr(L, "_team_ready"):
         L.emu_run_team.restype = C.c_int
         L.emu_run_team.argtypes = [C.c_int32, I32P, I32P, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32,
-                                   C.c_int32, C.c_int32, C.c_uint32, I32P, I32P, C.c_double]
+                                   C.c_int32, C.c_int32, C.c_uint32, C.c_int32, I32P, I32P, C.c_double]
         L._team_ready = True
     rp = np.ascontiguousarray(rp, np.int32)
     ci = np.ascontiguousarray(ci, np.int32)
@@ -249,6 +249,6 @@ def run_team(rp, ci, start, workers=3, mode=0, speculate=3, wide=2, alone=0, cap
     info = np.zeros(6, np.int32)
     L.emu_team_linger(*linger)
     rc = L.emu_run_team(n, rp.ctypes.data_as(I32P), ci.ctypes.data_as(I32P), int(start), workers, mode, speculate, wide,
-                        alone, cap, tag0, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
+                        alone, cap, tag0, geo, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
     assert rc == 0, "emulator rejected the arguments"
     return perm, info

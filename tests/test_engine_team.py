@@ -59,6 +59,51 @@ def test_emulated_slow_member(where, member):
             assert np.array_equal(perm, O.cm(rp, ci, s)), (name, phase)
 
 
+def _narrow_end():
+    """A tree of 1, 10, 60 and 3 nodes by level, its root n / 2, where a search begins."""
+    e = [(0, 1 + k) for k in range(10)]
+    e += [(1 + k // 6, 11 + k) for k in range(60)]
+    e += [(11 + 7 * k, 71 + k) for k in range(3)]
+    swap = {0: 37, 37: 0}
+    return G.from_edges(74, [(swap.get(a, a), swap.get(b, b)) for a, b in e])
+
+
+@pytest.mark.parametrize("geo", [0, 1])
+@pytest.mark.parametrize("wide", [2, 3])
+def test_emulated_slow_queue_entries(geo, wide):
+    """A search reads the queue entries of a last level that is redistributed (narrow: few members would do), however late
+    its members store them."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    rp, ci = _narrow_end()
+    _, s, it, _ = O.peripheral(rp, ci)
+    for phase in (2, 4, 0, 1, 3):
+        perm, info = E.run_team(rp, ci, -1, mode=2, workers=4, wide=wide, linger=(3, -1, phase), geo=geo, timeout_s=30)
+        assert info[0] == 0 and (info[3], info[4]) == (s, it), phase
+        assert np.array_equal(perm, O.cm(rp, ci, s)), phase
+
+
+def test_emulated_several_waves():
+    """Workgroups of two waves: what one wave of a member leaves for the other, at the meetings, the redistributions and
+    in a part of several chunks; held up at each place."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    for name in ("star64", "duplicates", "grid24x20", "random1500"):
+        rp, ci = CASES[name]()
+        _, s, it, _ = O.peripheral(rp, ci)
+        for where in (-1, 0, 1, 2, 3):
+            perm, info = E.run_team(rp, ci, -1, mode=2, workers=3, wide=2, linger=(where, -1, 3), tag0=0, geo=1,
+                                    timeout_s=30)
+            assert info[0] == 0 and (info[3], info[4]) == (s, it), (name, where)
+            assert np.array_equal(perm, O.cm(rp, ci, s)), (name, where)
+    directed = G.directed_with_empty_rows(2000, 1500, 24, 2)
+    perm, info = E.run_team(*directed, 0, geo=1)
+    assert info[0] == 0 and np.array_equal(perm, O.cm(*directed, 0))
+    assert E.run_team(*CASES["random1500"](), 0, cap=40, geo=1)[1][0] == 2
+
+
 def test_emulated_ends():
     """Directed rows, a disconnected matrix, a stage region that is too small, and the watchdog."""
     pytest.importorskip("emu_lib")
