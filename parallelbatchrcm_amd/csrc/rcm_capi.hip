@@ -93,22 +93,28 @@ using GeoSmall = Var<0>::G;  // the many-matrix helpers' default
 constexpr int kDigit = 4;
 // The one-workgroup engine (engine_solo.hpp): 1024 threads over chunks of 4096 slots.
 using SoloG = SoloGeo<1024, 4096, kSoloMaxN>;
-// A matrix goes through it when it fits and has at most `limit` rows. One workgroup takes 0.5-0.7 entries per ns where
-// the levels are wide, the batch engine 11 over the whole GPU, but 5-10 us a level however narrow: start search and
-// order on MI355X, one workgroup against the batch engine, 0.84 against 3.3 ms for a 100 x 100 grid, 2.6 against 4.0
-// ms for a 40k-point geometric graph, but 3.9 against 3.5 ms for a 48^3 stencil (110k rows). In a set, up to kSoloAlone
-// rows one workgroup wins whatever the shape; beyond, only beside enough other matrices: `total` rows keep the batch
-// engine busy for total / 11 entries' time, so a matrix of total / kSoloShare rows ends on its one workgroup before
-// the batch engine would have ended the set.
-constexpr int32_t kSoloAlone = 1 << 16;
+// One workgroup takes 0.5-0.6 entries per ns where the levels are wide, the batch engine 11 over the whole GPU, but 5-10 us
+// a level however narrow. A set's matrices of up to kSoloAlone rows go through it: on MI355X, batch engine and one
+// workgroup, ms a run of a set of one, 3D stencil 91k rows 1.60 / 1.18, 125k 1.78 / 1.55, 166k 2.10 / 2.13, 262k 2.43 /
+// 3.36; geometric of mean degree 13 130k 3.55 / 2.95, 200k 4.48 / 4.40, 260k 5.43 / 6.21; 2D 250k 9.79 / 3.44; with four
+// such matrices the same within 6%. Larger ones only beside enough others: `total` rows keep the batch engine busy for
+// total / 11 entries' time, so a matrix of total / kSoloShare rows ends on its one workgroup before the batch engine would
+// have ended the set.
+constexpr int32_t kSoloAlone = 9 << 14;
 constexpr int64_t kSoloShare = 16;
-// In a serving lane the other lanes' groups are that company (a 48-request burst of up to 100k rows: 11.7 ms with one
-// workgroup for each, 23.6 ms with the larger ones left to the batch engine, 27.3 ms with all of them).
-constexpr int64_t kSoloLaneTotal = (int64_t)kSoloShare << 17;
-bool solo_fits(int32_t n, uint32_t maxrow, int64_t total) {
-  return n <= std::min<int64_t>(kSoloMaxN, std::max<int64_t>(kSoloAlone, total / kSoloShare)) &&
+// A serving lane, whose launches other lanes' run beside (a 48-request burst of up to 100k rows: 11.7 ms with one workgroup
+// for each, 23.6 ms with those above 65,536 rows left to the batch engine; one 3D stencil of 125k rows 4.88 and 4.85 ms).
+constexpr int32_t kSoloLane = 1 << 17;
+// rcm_gpu_batch_noalloc: one matrix at a time.
+constexpr int32_t kSoloNoAlloc = 1 << 16;
+bool solo_fits(int32_t n, uint32_t maxrow, int64_t total, int32_t alone) {
+  return n <= std::min<int64_t>(kSoloMaxN, std::max<int64_t>(alone, total / kSoloShare)) &&
          maxrow <= (uint32_t)kSoloMaxRow;
 }
+
+// Whether a row holds so large a part of the matrix that its levels are few and wide: R-MAT graphs of 2^13 to 2^20 rows have
+// one of n / 27 entries or more.
+bool has_hub(int32_t n, uint32_t maxrow) { return maxrow > (uint32_t)kSoloMaxRow && (int64_t)maxrow * 32 >= n; }
 
 // The team engine (engine_team.hpp): up to kTeamMax workgroups on the matrix of a context, beyond kCtxSolo rows.
 using TeamG = TeamGeo<1024, 4096>;
@@ -756,7 +762,8 @@ struct rcm_batch {
   int32_t *blk_order = nullptr, *blk_active = nullptr;  // helper-kernel block maps of `order` / a sub-list
   int32_t nblk_order = 0;
   // The loaded set split by engine: matrices for the one-workgroup engine, and the rest (with its block map), both
-  // largest first. Used while batch_solo() holds; otherwise every matrix is the batch engine's.
+  // largest first. Used while batch_solo() holds; otherwise every matrix is the batch engine's (and where a set does better
+  // that way, `solo` is empty).
   bool engine_set = false;  // a parameter of the batch engine was chosen
   bool lane = false;        // a serving lane: its workgroup count is not a choice of engine
   std::vector<int32_t> solo, rest;
@@ -932,6 +939,19 @@ void enqueue_many(rcm_batch* b, const int32_t* d_list, const int32_t* d_blk, int
 bool batch_solo(const rcm_batch* b) {
   return !b->engine_set && (b->lane || b->workers == 0) && b->sort_mode == 0 && b->claim_filter == kDefaultClaimFilter &&
          !b->solo.empty();
+}
+
+// Whether a set gains from its split. The engines run one after the other, and a matrix of the rest with many levels keeps
+// the batch engine busy for as long as its levels take, with the others or without: only beside kSoloShare times its rows,
+// or with a hub row (few levels), does the rest end early enough. MI355X, ms a run by the batch engine alone and by both:
+// 5, 30 and 60 matrices of up to 60k rows beside a 2D stencil of 152k rows 6.7 / 7.3, 6.8 / 7.9, 6.9 / 8.0; beside a
+// geometric graph of 150k 3.86 / 4.50, 3.86 / 4.96, 3.92 / 5.06; beside an R-MAT graph of 2^16 rows 1.27 / 1.09, 3.42 /
+// 1.58, 3.87 / 1.61, of 2^13 rows 1.27 / 0.87, 3.40 / 1.36, 3.83 / 1.42.
+bool solo_pays(const rcm_batch* b) {
+  const int64_t company = (b->total_n - b->rest_rows) / kSoloShare;
+  for (int32_t k : b->rest)
+    if (b->n[k] > company && !has_hub(b->n[k], b->maxrow[k])) return false;
+  return true;
 }
 
 // The one-workgroup engine over the set's small matrices, one workgroup each at a time.
@@ -2083,12 +2103,17 @@ int rcm_batch_load(rcm_batch* b, int32_t count, const int32_t* n, const int64_t*
   }
   b->rest_rows = 0;
   for (int32_t k : b->order) {
-    if (solo_fits(n[k], b->maxrow[k], b->lane ? std::max(tot, kSoloLaneTotal) : tot)) {
+    if (solo_fits(n[k], b->maxrow[k], tot, b->lane ? kSoloLane : kSoloAlone)) {
       b->solo.push_back(k);
     } else {
       b->rest.push_back(k);
       b->rest_rows += n[k];
     }
+  }
+  if (!b->lane && !solo_pays(b)) {
+    b->solo.clear();
+    b->rest = b->order;
+    b->rest_rows = tot;
   }
   (void)build_blk(b, b->rest.data(), (int32_t)b->rest.size(), b->blk_rest_h);
   if (!b->solo.empty())
@@ -2970,7 +2995,7 @@ int rcm_gpu_batch_noalloc(int32_t n, int64_t nnz, const int32_t* d_row_ptr, cons
   a.claim_filter = kDefaultClaimFilter;
 
   int32_t start = start_node;
-  const bool solo = solo_fits(n, vflags[1], n);
+  const bool solo = solo_fits(n, vflags[1], n, kSoloNoAlloc);
   if (solo) {  // start search and order in one launch of one workgroup
     const SoloJob J{d_row_ptr, d_col_idx, d_perm_out, a.qinfo, n};
     hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, nullptr, J, (int32_t)SOLO_ORDER, start,

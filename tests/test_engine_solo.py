@@ -125,3 +125,67 @@ def test_gpu_set_with_rows_for_either_engine():
         assert st[-1] == P.RCM_ENOTCONNECTED and not st[:-1].any()
         for k, p in enumerate(b.perms()[:-1]):
             assert np.array_equal(p, perms[k]), k
+
+
+# members of a set, and how many workgroups run it (None: the batch engine's)
+SETS = {
+    "alone": (lambda: [_stencil("stencil2d", 384, 384), CASES["path300"]()], 2),  # 147,456 rows
+    "too_large": (lambda: [_stencil("stencil2d", 3, 49153), CASES["path300"]()], None),  # 147,459
+    "hubs": (lambda: [_stencil("stencil2d", 60, 70), G.hub_graph(3000, 2000, seed=3), CASES["random1500"](),
+                      G.star(MAXROW + 1)], None),
+    "long_rows": (lambda: [CASES["grid24x20"](), _regular(3000, 81, 5)], None),  # no hub: all by the batch engine
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(SETS))
+def test_gpu_set_split(name):
+    """Sets on either side of the rules that split them between the engines: search and order, start search, and run,
+    whose graph is replayed between them."""
+    mats, workgroups = SETS[name][0](), SETS[name][1]
+    bs = P.BatchSet.from_matrices([P.CSR(*m) for m in mats])
+    want = []
+    for rp, ci in mats:
+        _, s, it, _ = O.peripheral(rp, ci)
+        want.append((s, it, O.cm(rp, ci, s)))
+    given = np.array([s if k % 2 else -1 for k, (s, _, _) in enumerate(want)], np.int32)
+    with P.RcmBatch(timeout_ms=20000, graph=True) as b:
+        b.load(bs)
+        for rep in range(3):
+            print("[case]", name, "repeat", rep, flush=True)
+            starts, iters, st = b.order(given if rep == 2 else None)
+            assert not st.any() and [int(x) for x in starts] == [s for s, _, _ in want]
+            assert [int(x) for x in iters] == [0 if rep == 2 and k % 2 else it for k, (_, it, _) in enumerate(want)]
+            for k, p in enumerate(b.perms()):
+                assert np.array_equal(p, want[k][2]), (rep, k)
+            starts, iters, st = b.find_start()
+            assert not st.any() and [(int(x), int(y)) for x, y in zip(starts, iters)] == [w[:2] for w in want]
+            for flags in (P.RCM_FLAG_STABLE, P.RCM_FLAG_REVERSE):
+                assert not b.run(starts, flags).any()
+                for k, p in enumerate(b.perms()):
+                    assert np.array_equal(p, want[k][2][::-1] if flags == P.RCM_FLAG_REVERSE else want[k][2]), (rep, k)
+        assert b.timing().graph_replays >= 4
+        assert b.timing().workers == workgroups if workgroups else b.timing().workers > len(mats)
+
+
+@pytest.mark.gpu
+def test_gpu_set_of_the_largest():
+    """Beside enough others a matrix of as many rows as the bitmap has bits goes to one workgroup; one row more, and all of
+    the set to the batch engine."""
+    big, more = _stencil("stencil3d", 64, 64, 64), _stencil("stencil2d", 5, 52429)
+    assert len(big[0]) - 1 == 1 << 18 and len(more[0]) - 1 == (1 << 18) + 1
+    want = []
+    for rp, ci in (big, more):
+        _, s, it, _ = O.peripheral(rp, ci)
+        want.append((s, it, O.cm(rp, ci, s)))
+    with P.RcmBatch(timeout_ms=20000) as b:
+        for mats in ([big] * 16, [big] * 15 + [more]):
+            b.load(P.BatchSet.from_matrices([P.CSR(*m) for m in mats]))
+            print("[case] set", len(mats), flush=True)
+            starts, iters, st = b.order()
+            assert not st.any()
+            for k, p in enumerate(b.perms()):
+                s, it, order = want[mats[k] is more]
+                assert (starts[k], iters[k]) == (s, it) and np.array_equal(p, order), k
+            assert not b.run(starts).any()
+            assert (b.timing().workers == 16) == (mats[-1] is big)
