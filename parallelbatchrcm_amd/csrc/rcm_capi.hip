@@ -440,13 +440,14 @@ bool ctx_automatic(const rcm_ctx* c) {
 }
 
 // The batch engine's variant for the loaded matrix. Of its own accord it runs matrices with rows beyond the level
-// engines; from kWideNnz entries on, variant 4's wider batches suit them: start search and order of linked R-MAT graphs on
-// MI355X, variant 1 and 4, 250k entries 1.00 and 0.92 ms, 1M 1.47 and 1.20, 8M 5.75 and 4.13; a random graph of 100k rows
-// of 100 entries 1.92 and 1.34; below, R-MAT of 100k entries 0.63 and 0.63, of 13k 0.54 and 0.57.
+// engines; from kWideNnz entries on, variant 4's wider batches suit those with a hub: start search and order of linked R-MAT
+// graphs on MI355X, variant 1 and 4, 250k entries 1.00 and 0.92 ms, 1M 1.47 and 1.20, 8M 5.75 and 4.13; below, R-MAT of 100k
+// entries 0.63 and 0.63, of 13k 0.54 and 0.57. Without one the levels may be narrow, and narrow levels lose: one order of a
+// 5^3-point stencil on 10 x 10 x 2000 nodes 11.0 and 15.1 ms, on 6 x 6 x 6000 29.7 and 43.6 (on 40^3 1.18 and 0.89).
 constexpr int64_t kWideVariant = 4;
 constexpr int64_t kWideNnz = (int64_t)1 << 18;
 bool ctx_wide(const rcm_ctx* c) {
-  return ctx_automatic(c) && c->maxdeg > (uint32_t)kSoloMaxRow && c->nnz >= kWideNnz;
+  return ctx_automatic(c) && has_hub(c->n, c->maxdeg) && c->nnz >= kWideNnz;
 }
 int64_t ctx_variant(const rcm_ctx* c) { return ctx_wide(c) ? kWideVariant : c->variant; }
 

@@ -194,3 +194,25 @@ def test_gpu_context_with_long_rows(entries):
         assert c.order() == (s, it)
         assert np.array_equal(c.perm(), O.cm(rp, ci, s))
         assert c.timing().workers == (256 if entries >= 1 << 18 else 64)
+
+
+@pytest.mark.gpu
+def test_gpu_context_with_long_rows_and_narrow_levels():
+    """Rows beyond the level engines, many entries, but no hub: the batch engine's default variant."""
+    a, b, c = np.meshgrid(np.arange(6), np.arange(6), np.arange(300), indexing="ij")
+    at = np.stack([a, b, c], -1).reshape(-1, 3)
+    off = np.stack(np.meshgrid(*[np.arange(-2, 3)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    to = at[:, None] + off[None]
+    inside = ((to >= 0) & (to < (6, 6, 300))).all(-1)
+    rp = np.concatenate([[0], np.cumsum(inside.sum(1))]).astype(np.int32)
+    ci = ((to[..., 0] * 6 + to[..., 1]) * 300 + to[..., 2])[inside].astype(np.int32)
+    assert len(ci) >= 1 << 18 and np.diff(rp).max() > 64
+    m, _ = P.workloads.permute_symmetric(P.CSR(rp, ci), 3)
+    rp, ci = m.row_offsets, m.col_ids
+    print("[case]", m.rows, len(ci), flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        _, s, it, _ = O.peripheral(rp, ci)
+        assert c.order() == (s, it)
+        assert np.array_equal(c.perm(), O.cm(rp, ci, s))
+        assert c.timing().workers == 64
