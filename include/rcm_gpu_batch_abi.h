@@ -85,12 +85,13 @@ enum rcm_param {
   RCM_PARAM_TIMEOUT_MS = 2,  /* device watchdog, default 20000 */
   RCM_PARAM_SORT = 3,        /* 0 auto, 1 LDS radix sort, 2 segment-rank sort */
   RCM_PARAM_DIGIT_BITS = 4,  /* radix digit width of the current variant (read-only: set the variant) */
-  RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit). Until it is set (and while
-                                WORKERS, SORT, STRICT, PROFILE, CLAIM_FILTER and BATCH_CAP keep their defaults),
-                                whatever the variant, matrices whose rows have at most 64 entries are ordered by
-                                one workgroup each up to 32,768 rows in a context, 65,536 in a set (in a large
-                                set or a serving lane more), and in a context beyond that by a team of 128; in a
-                                context, longer rows from 262,144 entries on by variant 4:
+  RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit). While it has its default (as
+                                WORKERS, SORT, STRICT, PROFILE, CLAIM_FILTER and BATCH_CAP do), matrices whose
+                                rows have at most 64 entries are ordered by one workgroup each up to 32,768 rows
+                                in a context, 147,456 in a set, 131,072 in a serving lane (in a large set or
+                                group more), and in a context beyond that by a team of 128; in a context,
+                                matrices with a hub row from 262,144 entries on by variant 4. The default's own
+                                engine for every matrix: set WORKERS too.
                                 0 = 256 threads, 2048 adjacency slots, 256 parents, 4-bit digits (serving
                                     lanes)
                                 1 = 512 threads, 2048 slots, 256 parents, 4-bit digits (rcm_ctx default)

@@ -332,7 +332,7 @@ struct rcm_ctx {
   int64_t variant = kDefaultCtxVariant;
   int64_t strict = 0;
   int64_t profile = 0;
-  bool engine_set = false;   // RCM_PARAM_VARIANT was set (or tuned): the batch engine runs every matrix
+  bool engine_set = false;   // RCM_PARAM_VARIANT is not the default (or was tuned): its engine runs every matrix
   int64_t batch_cap = 0;     // RCM_PARAM_BATCH_CAP: batch records a run may use (0 = n + 1, all it can need)
   int64_t speculate = kDefaultSpeculate;  // RCM_PARAM_SPECULATE
   uint64_t* prof = nullptr;  // kProfSlots words
@@ -1585,7 +1585,7 @@ int rcm_ctx_set_param(rcm_ctx* c, int param, int64_t v) {
     case RCM_PARAM_VARIANT:
       if (v < 0 || v > kLevelVariant) return RCM_EINVAL;
       c->variant = v;
-      c->engine_set = true;
+      c->engine_set = v != kDefaultCtxVariant;  // a caller that puts back what it read finds the engines as they were
       return RCM_OK;
     case RCM_PARAM_STRICT: c->strict = v ? 1 : 0; return RCM_OK;
     case RCM_PARAM_PROFILE: if (v < 0 || v > 2) return RCM_EINVAL; c->profile = v; return RCM_OK;
@@ -1966,7 +1966,7 @@ int rcm_batch_set_param(rcm_batch* b, int param, int64_t v) {
     case RCM_PARAM_VARIANT:
       if (v < 0 || v >= kVariants) return RCM_EINVAL;
       b->variant = v;
-      b->engine_set = true;
+      b->engine_set = v != kDefaultBatchVariant;
       batch_drop_graphs(b);  // captured graphs hold the old launch parameters
       b->max_resident = b->max_res[v];
       return RCM_OK;

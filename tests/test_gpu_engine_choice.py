@@ -1,0 +1,65 @@
+"""GPU: which engine a context and a set run is a matter of their parameters alone: putting one back to the value that was
+read brings the automatic choice back, and with WORKERS set the default variant's batch engine runs every matrix."""
+import numpy as np
+import pytest
+
+import graphs as G
+import oracle_lib as O
+import parallelbatchrcm_amd as P
+from test_engine_solo import CASES
+
+pytestmark = pytest.mark.gpu
+
+
+def _say(*a):
+    print("[case]", *a, flush=True)
+
+
+def _want(rp, ci):
+    _, s, it, _ = O.peripheral(rp, ci)
+    return s, it, O.cm(rp, ci, s)
+
+
+@pytest.mark.parametrize("workers", [0, 64])
+def test_context(workers):
+    """Every short-row case by the level engine, and by the default variant of the batch engine."""
+    with P.RcmContext(timeout_ms=20000, workers=workers) as c:
+        for name in CASES:
+            rp, ci = CASES[name]()
+            _say(name, workers)
+            s, it, order = _want(rp, ci)
+            c.load(P.CSR(rp, ci))
+            assert c.order() == (s, it) and np.array_equal(c.perm(), order), name
+            assert c.find_start() == s, name
+            c.run(s)
+            assert np.array_equal(c.perm(), order), name
+            assert c.timing().workers == (workers or 1), name
+
+
+@pytest.mark.parametrize("name,value", [("variant", 3), ("claim_filter", 0), ("sort", 2), ("workers", 32), ("strict", 1)])
+def test_context_parameter_put_back(name, value):
+    rp, ci = CASES["random1500"]()
+    s, _, order = _want(rp, ci)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(P.CSR(rp, ci))
+        keep = c.get_param(name)
+        for v, workers in ((value, 32 if name == "workers" else 64), (keep, 1)):
+            c.set_param(name, v)
+            _say(name, v)
+            c.run(s)
+            assert np.array_equal(c.perm(), order) and c.timing().workers == workers, v
+
+
+def test_set_variant_put_back():
+    mats = [CASES["grid24x20"](), CASES["random1500"](), G.path(9)]
+    want = [_want(*m) for m in mats]
+    with P.RcmBatch(timeout_ms=20000) as b:
+        b.load(P.BatchSet.from_matrices([P.CSR(*m) for m in mats]))
+        few = []
+        for v in (3, 4):  # 4: the default
+            b.set_param("variant", v)
+            _say("variant", v)
+            assert not b.run([w[0] for w in want]).any()
+            assert all(np.array_equal(p, w[2]) for p, w in zip(b.perms(), want))
+            few.append(b.timing().workers == len(mats))
+        assert few == [False, True]
