@@ -2847,11 +2847,24 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
   return RCM_OK;
 }
 
+// A set's engine parameters while they are tuned: put back as they were unless the tuning is kept.
+struct BatchTuning {
+  rcm_batch* b;
+  int64_t variant = b->variant, workers = b->workers, helper_nodes = b->helper_nodes;
+  bool engine_set = b->engine_set, kept = false;
+  ~BatchTuning() {
+    if (kept) return;
+    (void)rcm_batch_set_param(b, RCM_PARAM_VARIANT, variant);
+    (void)rcm_batch_set_param(b, RCM_PARAM_WORKERS, workers);
+    (void)rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, helper_nodes);
+    b->engine_set = engine_set;
+  }
+};
+
 int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_tune_result* out) {
   if (!b || !start || !out || repeats < 1) return RCM_EINVAL;
   if (b->count == 0) return RCM_ENOTLOADED;
-  const int64_t keep_v = b->variant, keep_w = b->workers;
-  const bool keep_set = b->engine_set;
+  BatchTuning tuning{b};
   rcm_tune_result best{};
   best.best_ms = 1e300;
   int count = 0;
@@ -2865,12 +2878,7 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
       std::vector<double> t;
       for (int r = 0; r < repeats; ++r) {
         const int rc = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
-        if (rc == RCM_EDEVICE || rc == RCM_ETIMEOUT || rc == RCM_EINVAL || rc == RCM_ENOTLOADED) {
-          rcm_batch_set_param(b, RCM_PARAM_VARIANT, keep_v);
-          rcm_batch_set_param(b, RCM_PARAM_WORKERS, keep_w);
-          b->engine_set = keep_set;
-          return rc;
-        }
+        if (rc == RCM_EDEVICE || rc == RCM_ETIMEOUT || rc == RCM_EINVAL || rc == RCM_ENOTLOADED) return rc;
         t.push_back(b->timing.run_ms);
       }
       const double ms = median_of(t);
@@ -2886,10 +2894,9 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
   rcm_batch_set_param(b, RCM_PARAM_VARIANT, best.variant);
   rcm_batch_set_param(b, RCM_PARAM_WORKERS, best.workers);
   // then the helper cap, with the chosen engine
-  const int64_t keep_h = b->helper_nodes;
-  int64_t best_h = keep_h;
+  int64_t best_h = tuning.helper_nodes;
   for (int64_t h : {kDefaultHelperNodes, 4 * kDefaultHelperNodes, 16 * kDefaultHelperNodes}) {
-    if (h == keep_h) continue;  // timed above
+    if (h == tuning.helper_nodes) continue;  // timed above
     int rc = rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, h);
     std::vector<double> t;
     for (int r = 0; rc == RCM_OK && r < repeats; ++r) {
@@ -2899,10 +2906,7 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
       if (run == RCM_EDEVICE || run == RCM_ETIMEOUT || run == RCM_EINVAL || run == RCM_ENOTLOADED) rc = run;
       else t.push_back(b->timing.run_ms);
     }
-    if (rc != RCM_OK) {
-      rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, keep_h);
-      return rc;
-    }
+    if (rc != RCM_OK) return rc;
     if (t.empty()) continue;  // nothing timed: not a candidate
     ++count;
     const double ms = median_of(t);
@@ -2938,6 +2942,7 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
     rcm_batch_set_param(b, RCM_PARAM_WORKERS, best_w);
     b->engine_set = true;
   }
+  tuning.kept = true;
   best.candidates = count;
   b->have_perm = false;
   *out = best;

@@ -63,3 +63,22 @@ def test_set_variant_put_back():
             assert all(np.array_equal(p, w[2]) for p, w in zip(b.perms(), want))
             few.append(b.timing().workers == len(mats))
         assert few == [False, True]
+
+
+@pytest.mark.parametrize("bad", ["start", "time"])
+def test_set_after_a_failed_tuning(bad):
+    """A tuning that ends with an error leaves the engines as they were."""
+    mats = [P.workloads.config(3, scale=60000, seed=3)] * 2 + [P.CSR(*G.path(9))]
+    want = [_want(m.row_offsets, m.col_ids) for m in mats]
+    starts = [w[0] for w in want]
+    with P.RcmBatch(timeout_ms=20000) as b:
+        b.load(P.BatchSet.from_matrices(mats))
+        _say("tuning", bad)
+        if bad == "time":
+            b.set_param("timeout_ms", 1)
+        with pytest.raises(P.RcmError):
+            b.autotune([-1] * 3 if bad == "start" else starts)
+        b.set_param("timeout_ms", 20000)
+        assert not b.run(starts).any()
+        assert all(np.array_equal(p, w[2]) for p, w in zip(b.perms(), want))
+        assert b.timing().workers == len(mats)
