@@ -343,9 +343,9 @@ int rcm_selftest_copy_bandwidth(int device, int64_t bytes, int32_t reps, int32_t
                                 double* ms_out);
 
 /* ---- autotuner ---- */
-/* No reference counterpart. Times every candidate (engine variant x persistent workgroups, and for rcm_ctx the
- * level-synchronous variant 5; rcm_batch then also tries helper caps of 8192, 32768 and 131072 nodes) on the
- * loaded work
+/* No reference counterpart. Times the default parameters, then every candidate (engine variant x persistent
+ * workgroups, and for rcm_ctx the level-synchronous variant 5; rcm_batch then also tries helper caps of 8192, 32768
+ * and 131072 nodes) on the loaded work
  * (`repeats` runs each, median of the device time) and keeps the fastest in the context; the order never
  * depends on the choice. rcm_ctx_autotune runs the matrix from `start`; rcm_batch_autotune runs the whole
  * loaded set from start[k]. */
@@ -355,7 +355,7 @@ typedef struct rcm_tune_result {
   int32_t candidates;   /* configurations timed */
   int32_t threads;      /* block size of the chosen variant */
   double best_ms;       /* median device time of the choice */
-  double default_ms;    /* median device time of variant 0 with automatic workers */
+  double default_ms;    /* median device time of the default parameters */
   int32_t helper_nodes; /* rcm_batch_autotune: chosen RCM_PARAM_HELPER_NODES (0 from rcm_ctx_autotune) */
   int32_t reserved;
 } rcm_tune_result;

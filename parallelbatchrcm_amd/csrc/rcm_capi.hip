@@ -2742,105 +2742,77 @@ static double median_of(std::vector<double> v) {
   return v[v.size() / 2];
 }
 
+// A context's engine parameters while they are tuned: put back as they were unless the tuning is kept.
+struct CtxTuning {
+  rcm_ctx* c;
+  int64_t variant = c->variant, workers = c->workers;
+  bool engine_set = c->engine_set, kept = false;
+  ~CtxTuning() {
+    if (kept) return;
+    c->variant = variant;
+    c->workers = workers;
+    c->engine_set = engine_set;
+  }
+};
+
 int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result* out) {
   if (!c || !out || repeats < 1) return RCM_EINVAL;
   if (!c->rp || c->n == 0) return RCM_ENOTLOADED;
   if (start < 0 || start >= c->n) return RCM_EINVAL;
   RCM_HIP(hipSetDevice(c->device));
-  const int64_t keep_v = c->variant, keep_w = c->workers;
-  const bool keep_set = c->engine_set;
+  CtxTuning tuning{c};
   rcm_tune_result best{};
-  best.best_ms = 1e300;
   int count = 0;
+  std::vector<double> t;
+  const auto timed = [&]() -> int {  // the median of `repeats` runs of the current parameters goes behind t
+    t.clear();
+    for (int r = 0; r < repeats; ++r) {
+      const int rc = run_engine(c, start, false);
+      if (rc) return rc;
+      t.push_back(c->timing.run_kernel_ms);
+    }
+    ++count;
+    return RCM_OK;
+  };
+  // the default: a level engine where one takes the matrix
+  c->variant = kDefaultCtxVariant;
+  c->workers = 0;
+  c->engine_set = false;
+  if (const int rc = timed()) return rc;
+  bool automatic = ctx_quick(c);
+  best.default_ms = best.best_ms = median_of(t);
+  best.variant = (int32_t)(automatic ? c->variant : ctx_variant(c));
+  best.workers = c->timing.workers;
+  best.threads = automatic ? SoloG::T : variant_threads(best.variant);
+  const auto better = [&]() {
+    const double ms = median_of(t);
+    if (ms >= best.best_ms) return;
+    automatic = false;
+    best.best_ms = ms;
+    best.variant = (int32_t)c->variant;
+    best.workers = workers_for(c);
+    best.threads = variant_threads(c->variant);
+  };
   c->engine_set = true;
   for (int v = 0; v < kVariants; ++v) {
     std::vector<int> ws = tune_workers(c->max_resident[v]);
-    if (v == 0) ws.insert(ws.begin(), 0);  // 0 = automatic: the default configuration
+    if (v == 0) ws.insert(ws.begin(), 0);  // 0 = automatic
     for (int w : ws) {
       c->variant = v;
       c->workers = w;
-      std::vector<double> t;
-      for (int r = 0; r < repeats; ++r) {
-        const int rc = run_engine(c, start, false);
-        if (rc) {
-          c->variant = keep_v;
-          c->workers = keep_w;
-          c->engine_set = keep_set;
-          return rc;
-        }
-        t.push_back(c->timing.run_kernel_ms);
-      }
-      const double ms = median_of(t);
-      ++count;
-      if (v == 0 && w == 0) best.default_ms = ms;
-      if (ms < best.best_ms) {
-        best.best_ms = ms;
-        best.variant = v;
-        best.workers = workers_for(c);
-      }
+      if (const int rc = timed()) return rc;
+      better();
     }
   }
-  {  // the level-synchronous engine: one configuration
-    c->variant = kLevelVariant;
-    std::vector<double> t;
-    int rc = RCM_OK;
-    for (int r = 0; r < repeats && rc == RCM_OK; ++r) {
-      rc = run_engine(c, start, false);
-      t.push_back(c->timing.run_kernel_ms);
-    }
-    if (rc == RCM_OK) {  // a level too wide for 64-bit keys leaves it out
-      ++count;
-      const double ms = median_of(t);
-      if (ms < best.best_ms) {
-        best.best_ms = ms;
-        best.variant = kLevelVariant;
-        best.workers = 0;
-      }
-    } else if (rc != RCM_ECAPACITY) {
-      c->variant = keep_v;
-      c->workers = keep_w;
-      c->engine_set = keep_set;
-      return rc;
-    }
-  }
-  c->variant = best.variant;
-  c->workers = best.workers;
-  best.threads = variant_threads(best.variant);
-  // the automatic choice, where that is a level engine
-  const int64_t best_w = c->workers;
+  c->variant = kLevelVariant;  // the level-synchronous engine: one configuration
   c->workers = 0;
-  c->engine_set = false;
-  bool automatic = false;
-  if (ctx_quick(c)) {
-    std::vector<double> t;
-    int32_t used = 0;
-    int rc = RCM_OK;
-    for (int r = 0; r < repeats && rc == RCM_OK; ++r) {
-      rc = run_engine(c, start, false);
-      t.push_back(c->timing.run_kernel_ms);
-      used = c->timing.workers;
-    }
-    if (rc) {
-      c->variant = keep_v;
-      c->workers = keep_w;
-      c->engine_set = keep_set;
-      return rc;
-    }
-    ++count;
-    const double ms = median_of(t);
-    if (ms < best.best_ms) {
-      automatic = true;
-      best.best_ms = ms;
-      best.variant = (int32_t)kDefaultCtxVariant;
-      best.workers = used;
-      best.threads = ctx_quick(c) ? SoloG::T : variant_threads(kDefaultCtxVariant);
-      c->variant = kDefaultCtxVariant;
-    }
-  }
-  if (!automatic) {
-    c->workers = best_w;
-    c->engine_set = true;
-  }
+  const int rc = timed();
+  if (rc == RCM_OK) better();
+  else if (rc != RCM_ECAPACITY) return rc;  // a level too wide for 64-bit keys leaves it out
+  c->variant = automatic ? kDefaultCtxVariant : best.variant;
+  c->workers = automatic ? 0 : best.workers;
+  c->engine_set = !automatic;
+  tuning.kept = true;
   best.candidates = count;
   c->have_perm = false;  // the tuning runs overwrote the last order
   *out = best;
@@ -2866,82 +2838,79 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
   if (b->count == 0) return RCM_ENOTLOADED;
   BatchTuning tuning{b};
   rcm_tune_result best{};
-  best.best_ms = 1e300;
   int count = 0;
   std::vector<int32_t> st((size_t)b->count);
+  std::vector<double> t;
+  const auto timed = [&]() -> int {  // the median of `repeats` runs of the current parameters goes behind t
+    t.clear();
+    for (int r = 0; r < repeats; ++r) {
+      // per-matrix failures (a disconnected member) do not void the timing: every matrix was run; only launch-level
+      // failures end the tuning
+      const int rc = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
+      if (rc == RCM_EDEVICE || rc == RCM_ETIMEOUT || rc == RCM_EINVAL || rc == RCM_ENOTLOADED) return rc;
+      t.push_back(b->timing.run_ms);
+    }
+    ++count;
+    return RCM_OK;
+  };
+  // the default: matrices that fit it by the one-workgroup engine
+  rcm_batch_set_param(b, RCM_PARAM_VARIANT, kDefaultBatchVariant);
+  rcm_batch_set_param(b, RCM_PARAM_WORKERS, 0);
+  if (const int rc = timed()) return rc;
+  bool automatic = batch_solo(b);
+  best.default_ms = best.best_ms = median_of(t);
+  best.variant = (int32_t)b->variant;
+  best.workers = b->timing.workers;
+  int64_t best_h = tuning.helper_nodes;
+  double batch_ms = automatic ? std::numeric_limits<double>::infinity() : best.best_ms;  // of the batch engine alone
+  int64_t batch_v = b->variant, batch_w = batch_workers(b);
+  const auto better = [&]() {
+    const double ms = median_of(t);
+    if (ms < batch_ms) {
+      batch_ms = ms;
+      batch_v = b->variant;
+      batch_w = batch_workers(b);
+      best_h = b->helper_nodes;
+    }
+    if (ms >= best.best_ms) return;
+    automatic = false;
+    best.best_ms = ms;
+    best.variant = (int32_t)b->variant;
+    best.workers = batch_workers(b);
+  };
   for (int v = 0; v < kVariants; ++v) {
     std::vector<int> ws = tune_workers(b->max_res[v]);
     if (v == 0) ws.insert(ws.begin(), 0);
     for (int w : ws) {
       rcm_batch_set_param(b, RCM_PARAM_VARIANT, v);
       rcm_batch_set_param(b, RCM_PARAM_WORKERS, w);
-      std::vector<double> t;
-      for (int r = 0; r < repeats; ++r) {
-        const int rc = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
-        if (rc == RCM_EDEVICE || rc == RCM_ETIMEOUT || rc == RCM_EINVAL || rc == RCM_ENOTLOADED) return rc;
-        t.push_back(b->timing.run_ms);
-      }
-      const double ms = median_of(t);
-      ++count;
-      if (v == 0 && w == 0) best.default_ms = ms;
-      if (ms < best.best_ms) {
-        best.best_ms = ms;
-        best.variant = v;
-        best.workers = batch_workers(b);
-      }
+      b->engine_set = true;
+      if (const int rc = timed()) return rc;
+      better();
     }
   }
-  rcm_batch_set_param(b, RCM_PARAM_VARIANT, best.variant);
-  rcm_batch_set_param(b, RCM_PARAM_WORKERS, best.workers);
-  // then the helper cap, with the chosen engine
-  int64_t best_h = tuning.helper_nodes;
+  // then the helper cap, with the fastest of them
+  rcm_batch_set_param(b, RCM_PARAM_VARIANT, batch_v);
+  rcm_batch_set_param(b, RCM_PARAM_WORKERS, batch_w);
+  b->engine_set = true;
   for (int64_t h : {kDefaultHelperNodes, 4 * kDefaultHelperNodes, 16 * kDefaultHelperNodes}) {
     if (h == tuning.helper_nodes) continue;  // timed above
     int rc = rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, h);
-    std::vector<double> t;
-    for (int r = 0; rc == RCM_OK && r < repeats; ++r) {
-      // per-matrix failures (a disconnected member) do not void the timing: every matrix was run, as in the
-      // variant loop above; only launch-level failures end the tuning
-      const int run = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
-      if (run == RCM_EDEVICE || run == RCM_ETIMEOUT || run == RCM_EINVAL || run == RCM_ENOTLOADED) rc = run;
-      else t.push_back(b->timing.run_ms);
-    }
+    if (rc == RCM_OK) rc = timed();
     if (rc != RCM_OK) return rc;
-    if (t.empty()) continue;  // nothing timed: not a candidate
-    ++count;
-    const double ms = median_of(t);
-    if (ms < best.best_ms) {
-      best.best_ms = ms;
-      best_h = h;
-    }
+    better();
   }
+  if (automatic) {
+    batch_v = kDefaultBatchVariant;
+    batch_w = 0;
+    best_h = tuning.helper_nodes;
+  }
+  rcm_batch_set_param(b, RCM_PARAM_VARIANT, batch_v);
+  rcm_batch_set_param(b, RCM_PARAM_WORKERS, batch_w);
   rcm_batch_set_param(b, RCM_PARAM_HELPER_NODES, best_h);
+  b->engine_set = !automatic;
   best.helper_nodes = (int32_t)best_h;
   best.threads = kVarThreads[best.variant];
-  // the automatic choice, where that sends matrices to the one-workgroup engine (the rest runs the chosen variant)
-  const int64_t best_w = b->workers;
-  rcm_batch_set_param(b, RCM_PARAM_WORKERS, 0);
-  b->engine_set = false;
-  bool automatic = false;
-  if (batch_solo(b)) {
-    std::vector<double> t;
-    for (int r = 0; r < repeats; ++r) {
-      const int run = rcm_batch_run(b, start, RCM_FLAG_STABLE, st.data());
-      if (run == RCM_EDEVICE || run == RCM_ETIMEOUT || run == RCM_EINVAL || run == RCM_ENOTLOADED) return run;
-      t.push_back(b->timing.run_ms);
-    }
-    ++count;
-    const double ms = median_of(t);
-    if (ms < best.best_ms) {
-      automatic = true;
-      best.best_ms = ms;
-      best.workers = b->timing.workers;
-    }
-  }
-  if (!automatic) {
-    rcm_batch_set_param(b, RCM_PARAM_WORKERS, best_w);
-    b->engine_set = true;
-  }
   tuning.kept = true;
   best.candidates = count;
   b->have_perm = false;

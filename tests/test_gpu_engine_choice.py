@@ -82,3 +82,32 @@ def test_set_after_a_failed_tuning(bad):
         assert not b.run(starts).any()
         assert all(np.array_equal(p, w[2]) for p, w in zip(b.perms(), want))
         assert b.timing().workers == len(mats)
+
+
+@pytest.mark.parametrize("graph", ["level", "hub"])
+def test_tuning_times_the_default(graph):
+    """default_ms is what a context or set with nothing chosen takes, not a variant that no default call runs."""
+    m = P.workloads.config(3, scale=40000, seed=3) if graph == "level" else P.CSR(*G.hub_graph(5000, 9000, seed=1))
+    s, _, order = _want(m.row_offsets, m.col_ids)
+    _say(graph)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        times = []
+        for _ in range(9):
+            c.run(s)
+            times.append(c.timing().run_kernel_ms)
+        r = c.autotune(s, repeats=5)
+        assert 0 < r.best_ms <= r.default_ms and min(times) / 2 < r.default_ms < 2 * max(times)
+        assert r.workers > 0 or r.variant == 5
+        c.run(s)
+        assert np.array_equal(c.perm(), order)
+    with P.RcmBatch(timeout_ms=20000) as b:
+        b.load(P.BatchSet.from_matrices([m] * 3))
+        times = []
+        for _ in range(9):
+            assert not b.run([s] * 3).any()
+            times.append(b.timing().run_ms)
+        r = b.autotune([s] * 3, repeats=5)
+        assert 0 < r.best_ms <= r.default_ms and min(times) / 2 < r.default_ms < 2 * max(times)
+        assert not b.run([s] * 3).any()
+        assert all(np.array_equal(p, order) for p in b.perms())
