@@ -58,7 +58,8 @@ struct SoloSmem {
   uint16_t cpar[G::NC];          // per 64 slots: 1 + the parent of the first of them
   uint64_t cinfo[G::NC];         // per 64 slots: owned children | their degree sum << 32
   int32_t levstart[64];          // first queue position of the last 64 levels
-  uint32_t np, E, quit;          // of the chunk: parents, slots; the watchdog fired
+  uint32_t np, E, quit;          // of the chunk: parents, slots; the watchdog fired in the pass
+  uint32_t late;                 // it fired between two passes
   int32_t job, cur;
 };
 constexpr uint32_t kNoSlot = ~0u;
@@ -408,6 +409,12 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
   __syncthreads();
   expired = sm.quit != 0;
   while (!expired && (searching || mode != SOLO_SEARCH)) {
+    if (passes > 0) {  // a pass looks at the clock on every 64th step, and may have fewer
+      if (tid == 0) sm.late = wall_ticks() > deadline ? 1u : 0u;
+      __syncthreads();
+      expired = sm.late != 0;
+      if (expired) break;
+    }
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && mode == SOLO_ORDER && speculate > 0 && iters >= speculate;
     placed = solo_pass<G>(J, sm, cur, searching && !attempt, deadline, &lev, &steps);

@@ -82,6 +82,20 @@ def test_emulated_watchdog():
     assert (info[:, 0] == 1).all()
 
 
+# unsymmetric: the sweeps from nodes 2 and 3 find eccentricities 1 and 2 in turn, and no start is ever confirmed
+ENDLESS = (np.array([0, 3, 6, 9, 12], np.int32), np.array([1, 2, 3, 1, 2, 3, 0, 1, 3, 0, 1, 3], np.int32))
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+def test_emulated_endless_search(mode):
+    """A search that would go on for ever, of passes too short to look at the clock, ends by the watchdog."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    assert E.run_solo([ENDLESS], [-1], workers=1, mode=mode, timeout_s=0.2)[1][0, 0] == 1
+    assert E.run_team(*ENDLESS, -1, workers=2, mode=mode, timeout_s=0.2)[1][0] == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(CASES) + ["rows63x9000", "rgg65536", "grid65537"])
 def test_gpu_single(name):
