@@ -82,7 +82,8 @@ typedef struct rcm_ctx rcm_ctx;
 
 enum rcm_param {
   RCM_PARAM_WORKERS = 1,     /* persistent workgroups for one matrix (0 = autotuned) */
-  RCM_PARAM_TIMEOUT_MS = 2,  /* device watchdog, default 20000 */
+  RCM_PARAM_TIMEOUT_MS = 2,  /* device watchdog of each pass over a matrix (a sweep of a start search, an order),
+                                default 20000 */
   RCM_PARAM_SORT = 3,        /* 0 auto, 1 LDS radix sort, 2 segment-rank sort */
   RCM_PARAM_DIGIT_BITS = 4,  /* radix digit width of the current variant (read-only: set the variant) */
   RCM_PARAM_VARIANT = 5,     /* engine variant (block size, batch width, radix digit). While it has its default (as

@@ -38,6 +38,10 @@ template <class T>
 __device__ __forceinline__ void st_sync(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// A word of pinned host memory that the host looks at while the kernel runs.
+__device__ __forceinline__ void st_host(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <bool STRICT>
 __device__ __forceinline__ void publish_wait() {
   if constexpr (STRICT)

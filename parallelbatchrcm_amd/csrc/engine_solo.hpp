@@ -389,12 +389,38 @@ __device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, 
   return q.tail;
 }
 
+// The watchdog of a workgroup. Its budget is for one pass over each matrix, as where every sweep is a launch of its own: a
+// pass is to end within one budget, and the pass numbered p (from 1) of any matrix within p budgets of the launch.
+struct SoloClock {
+  uint64_t t0, budget;
+  uint32_t* beat;  // pinned, or null: changes as passes begin, so that the host does not give a long search up
+  uint32_t due;    // the largest p yet
+  __device__ __forceinline__ uint64_t deadline() const { return t0 + budget * due; }
+};
+// One thread, as a pass after the first begins. The host allows 10 s beyond the budget; before 10 ms it need not know (the
+// store to its memory takes 3 us, of a pass over a 100 x 100 grid's 290).
+__device__ __forceinline__ void pass_beat(uint32_t* beat, uint64_t t0) {
+  const uint64_t now = wall_ticks();
+  if (beat && now - t0 > 1000000u) st_host(beat, (uint32_t)now);
+}
+
+// Which passes of a search the watchdog counts. In a symmetric matrix every sweep is longer than the one before or confirms
+// it; in others the sweeps may repeat for ever, so one that does neither moves the deadline no further.
+struct SearchPasses {
+  uint32_t count = 1, longest = 0;
+  __device__ __forceinline__ void sweep(uint32_t lev, bool attempt) {  // the sweep after it is due, and an attempt's repeat
+    if (lev <= longest) return;
+    longest = lev;
+    count += attempt ? 2u : 1u;
+  }
+};
+
 // One matrix: the start search (SOLO_SEARCH), the order from `start` (SOLO_RUN), or both (SOLO_ORDER; `start` >= 0
 // skips the search). From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is first run as a CM pass: when its
 // eccentricity equals the previous sweep's it is the confirming sweep and the result. The results go to *ctl.
 template <class G>
 __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, int32_t mode, int32_t start,
-                                            int32_t speculate, uint64_t deadline, Control* ctl) {
+                                            int32_t speculate, SoloClock& clk, Control* ctl) {
   const int tid = threadIdx.x, ln = lane_id();
   for (int i = tid; i < G::S; i += G::T) sm.tab[i] = kNoSlot;
   for (int i = tid; i < G::S; i += G::T) sm.mark[i] = 0;
@@ -404,28 +430,33 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
   int32_t cur = start >= 0 ? start : n > 1 ? n / 2 : 0;
   int32_t iters = start < 0 && n == 1 ? 1 : 0, passes = 0, placed = n, lev = 0;
   uint32_t steps = 0, lastdist = 0;
-  bool expired = wall_ticks() > deadline;  // thread 0's word counts, below
+  SearchPasses due;
+  bool expired = wall_ticks() > clk.deadline();  // thread 0's word counts, below
   if (tid == 0) sm.quit = expired ? 1u : 0u;
   __syncthreads();
   expired = sm.quit != 0;
   while (!expired && (searching || mode != SOLO_SEARCH)) {
+    clk.due = max(clk.due, due.count);
     if (passes > 0) {  // a pass looks at the clock on every 64th step, and may have fewer
-      if (tid == 0) sm.late = wall_ticks() > deadline ? 1u : 0u;
+      if (tid == 0) sm.late = wall_ticks() > clk.deadline() ? 1u : 0u;
       __syncthreads();
       expired = sm.late != 0;
       if (expired) break;
     }
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && mode == SOLO_ORDER && speculate > 0 && iters >= speculate;
-    placed = solo_pass<G>(J, sm, cur, searching && !attempt, deadline, &lev, &steps);
+    if (passes > 0 && tid == 0) pass_beat(clk.beat, clk.t0);
+    placed = solo_pass<G>(J, sm, cur, searching && !attempt, min(clk.deadline(), wall_ticks() + clk.budget), &lev, &steps);
     ++passes;
     expired = sm.quit != 0;
     if (placed != n || expired || !searching) break;
     if ((uint32_t)lev == lastdist) {  // cur is the start
       if (attempt || mode == SOLO_SEARCH) break;
       searching = false;
+      ++due.count;
       continue;
     }
+    due.sweep((uint32_t)lev, attempt);
     redo = attempt;  // a failed attempt is followed by the plain sweep from the same start
     if (redo) continue;
     lastdist = (uint32_t)lev;
@@ -462,10 +493,11 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
 // One matrix in one launch.
 template <class G>
 __global__ __launch_bounds__(G::T) void k_solo(SoloJob J, int32_t mode, int32_t start, int32_t speculate,
-                                               uint64_t budget_ticks, Control* ctl) {
+                                               uint64_t budget_ticks, uint32_t* beat, Control* ctl) {
   using SM = SoloSmem<G>;
   RCM_LDS(SM, sm);
-  solo_matrix<G>(J, sm, mode, start, speculate, wall_ticks() + budget_ticks, ctl);
+  SoloClock clk{wall_ticks(), budget_ticks, beat, 1u};
+  solo_matrix<G>(J, sm, mode, start, speculate, clk, ctl);
 }
 
 // Many matrices: workgroups take the jobs of the list in its order (largest first). A workgroup past the watchdog
@@ -480,6 +512,7 @@ struct SoloManyArgs {
   int32_t mode;
   int32_t speculate;
   uint64_t budget_ticks;
+  uint32_t* beat;
 };
 
 __global__ void k_solo_reset(uint32_t* next) {
@@ -490,7 +523,7 @@ template <class G>
 __global__ __launch_bounds__(G::T) void k_solo_many(SoloManyArgs m) {
   using SM = SoloSmem<G>;
   RCM_LDS(SM, sm);
-  const uint64_t deadline = wall_ticks() + m.budget_ticks;
+  SoloClock clk{wall_ticks(), m.budget_ticks, m.beat, 1u};
   for (;;) {
     if (threadIdx.x == 0) {
       const uint32_t x = atomic_add_u32(m.next, 1u);
@@ -501,7 +534,7 @@ __global__ __launch_bounds__(G::T) void k_solo_many(SoloManyArgs m) {
     if (j < 0) break;
     const JobDesc& D = m.jobs[j];
     const SoloJob J{D.row_ptr, D.col_idx, D.perm, D.qinfo, D.n};
-    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, deadline, D.ctl);  // ends with a barrier
+    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, clk, D.ctl);  // ends with a barrier
   }
 }
 

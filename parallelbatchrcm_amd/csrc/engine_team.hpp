@@ -86,6 +86,7 @@ struct TeamArgs {
   uint32_t alone;    // slots beyond which the leader shares its next local level
   uint32_t tag0;     // the first level's tag is tag0 + 1
   uint64_t budget_ticks;
+  uint32_t* beat;    // as SoloClock's
 };
 
 template <class G>
@@ -137,11 +138,21 @@ __device__ __forceinline__ void team_fail(const TeamArgs& a, uint32_t err) {
   st_sync(&a.ctl->done, 1u);
 }
 
+// The watchdog (as SoloClock): the leader says in ctl->passes how many passes are due; who runs out of time looks there.
+struct TeamClock {
+  uint64_t t0, deadline;
+};
+__device__ __forceinline__ bool team_late(const TeamArgs& a, TeamClock& clk) {
+  if (wall_ticks() <= clk.deadline) return false;
+  clk.deadline = max(clk.deadline, clk.t0 + a.budget_ticks * (uint64_t)(uint32_t)ld_sync(&a.ctl->passes));
+  return wall_ticks() > clk.deadline;
+}
+
 // One wave: whether to give up waiting (the launch is over, or the watchdog fires). Looked at on every 16th poll.
-__device__ __forceinline__ bool team_stop(const TeamArgs& a, uint64_t deadline, uint32_t spin) {
+__device__ __forceinline__ bool team_stop(const TeamArgs& a, TeamClock& clk, uint32_t spin) {
   if (spin % 16u != 15u) return false;
   if (wave_uniform(ld_sync(&a.ctl->done))) return true;
-  if (wave_uniform(wall_ticks() > deadline ? 1u : 0u)) {
+  if (wave_uniform(team_late(a, clk) ? 1u : 0u)) {
     if (lane_id() == 0) team_fail(a, ERR_TIMEOUT);
     return true;
   }
@@ -171,7 +182,7 @@ struct TeamWords {
   uint64_t w[kTeamPer];
 };
 __device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, int which, uint32_t tag, int32_t members,
-                                              uint64_t deadline, TeamWords& r) {
+                                              TeamClock& clk, TeamWords& r) {
   const int l0 = lane_id() * kTeamPer;
   for (uint32_t spin = 0;; ++spin) {
     bool early = false, late = false;
@@ -183,7 +194,7 @@ __device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, int which, uint
     }
     if (ballot(late)) return TEAM_PASSED;
     if (!ballot(early)) return TEAM_ON;
-    if (team_stop(a, deadline, spin)) return TEAM_STOP;
+    if (team_stop(a, clk, spin)) return TEAM_STOP;
   }
 }
 __device__ __forceinline__ uint32_t word_count(uint64_t w) { return (uint32_t)w & ((1u << kTeamNodeBits) - 1u); }
@@ -193,7 +204,7 @@ __device__ __forceinline__ uint32_t word_count(uint64_t w) { return (uint32_t)w 
 // words. Wave 0 has sm.met set when it passes the next barrier.
 template <class G>
 __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
-                                          uint64_t deadline) {
+                                          TeamClock& clk) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (lv.members == 1) {
@@ -209,7 +220,7 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
     if (lane_id() == 0)
       st_sync(team_word(a, sm.g, (int)(lv.tag & 1u)), ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
     RCM_TEAM_LINGER(0, sm.g, lv.tag);
-    const uint32_t v = team_poll(a, (int)(lv.tag & 1u), lv.tag, lv.members, deadline, r);
+    const uint32_t v = team_poll(a, (int)(lv.tag & 1u), lv.tag, lv.members, clk, r);
     if (lane_id() == 0) sm.verdict = v;
   }
   __syncthreads();
@@ -242,11 +253,11 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
 // and the leader's sm.gnext. TEAM_PASSED when that is over for this workgroup (the others have gone on without it).
 template <class G>
 __device__ __forceinline__ uint32_t team_counts(const TeamArgs& a, TeamSmem<G>& sm, uint32_t tag, int32_t members,
-                                                uint64_t deadline) {
+                                                TeamClock& clk) {
   if (wave_id() == 0) {
     TeamWords r;
     RCM_TEAM_LINGER(1, sm.g, tag);
-    const uint32_t v = team_poll(a, kTeamSplitWord, tag, members, deadline, r);
+    const uint32_t v = team_poll(a, kTeamSplitWord, tag, members, clk, r);
     uint32_t c = 0;
 #pragma unroll
     for (int i = 0; i < kTeamPer; ++i) c += word_count(r.w[i]);
@@ -299,7 +310,7 @@ __device__ __forceinline__ void team_mark(TeamSmem<G>& sm, uint32_t i, uint32_t 
 // sm.np and sm.E tell how many parents and slots. Ends with a barrier. False when the launch is over.
 template <class G>
 __device__ __forceinline__ bool team_take(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, int32_t c0,
-                                          uint64_t deadline) {
+                                          TeamClock& clk) {
   constexpr int T = G::T, S = G::S, W = G::W;
   const int tid = threadIdx.x;
   const int32_t avail = min(lv.cnt - c0, (int32_t)T);
@@ -316,7 +327,7 @@ __device__ __forceinline__ bool team_take(const TeamArgs& a, TeamSmem<G>& sm, co
     const uint64_t* e = a.stage[lv.tag & 1u] + 2 * ((size_t)(lv.region + lo) * (size_t)a.cap + (size_t)((uint32_t)p - first));
     uint64_t e0 = ld_sync(e), e1 = ld_sync(e + 1);
     for (uint32_t spin = 0; (uint32_t)(e0 >> 32) != lv.tag || (uint32_t)(e1 >> 32) != lv.tag; ++spin) {
-      if (spin % 16u == 15u && (ld_sync(&a.ctl->done) || wall_ticks() > deadline)) {
+      if (spin % 16u == 15u && (ld_sync(&a.ctl->done) || team_late(a, clk))) {
         sm.lost = 1;
         break;
       }
@@ -624,18 +635,18 @@ __device__ __forceinline__ bool team_chunk_local(const TeamArgs& a, TeamSmem<G>&
 }
 template <class G, int KN>
 __device__ __forceinline__ bool team_chunk(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
-                                           uint64_t deadline, TeamNext& nx) {
+                                           TeamClock& clk, TeamNext& nx) {
   TeamSlots<KN> s;
   team_expand<G, KN>(a, sm, 0, lv.E, s);
   team_claim<G, KN>(a, lv, lv.E, s);
-  if (!team_meet<G>(a, sm, lv, here, deadline)) return false;
+  if (!team_meet<G>(a, sm, lv, here, clk)) return false;
   return team_place<G, KN, false>(a, sm, lv, 0, lv.cnt, lv.E, s, true, true, nx);
 }
 
 // The part when it is more than one chunk: the claims of all of them, the meeting, then the children of each.
 template <class G>
 __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, int32_t np0,
-                                            uint32_t E0, uint32_t here, uint64_t deadline, TeamNext& nx) {
+                                            uint32_t E0, uint32_t here, TeamClock& clk, TeamNext& nx) {
   constexpr int KN = G::EPT;
   TeamSlots<KN> s;
   int32_t np = np0;
@@ -646,14 +657,14 @@ __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, 
     c0 += np;
     if (c0 >= lv.cnt) break;
     __syncthreads();
-    if (!team_take<G>(a, sm, lv, c0, deadline)) return false;
+    if (!team_take<G>(a, sm, lv, c0, clk)) return false;
     np = (int32_t)sm.np;
     e = wave_uniform(sm.E);
   }
-  if (!team_meet<G>(a, sm, lv, here, deadline)) return false;
+  if (!team_meet<G>(a, sm, lv, here, clk)) return false;
   for (int32_t c0 = 0; c0 < lv.cnt;) {
     __syncthreads();
-    if (!team_take<G>(a, sm, lv, c0, deadline)) return false;
+    if (!team_take<G>(a, sm, lv, c0, clk)) return false;
     np = (int32_t)sm.np;
     e = wave_uniform(sm.E);
     team_expand<G, KN>(a, sm, c0, e, s);
@@ -680,7 +691,7 @@ __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, 
 // or this workgroup is not a member of the next level. here: thread 0 of the leader, the workgroups started.
 template <class G>
 __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& sm, TeamLevel& lv, uint32_t here,
-                                               uint64_t deadline) {
+                                               TeamClock& clk) {
   TeamNext nx{0, 0, false, false};
   bool ok = true;
   if (lv.local && lv.cnt > 0 && !lv.marked) {  // too wide for one chunk: through the claim words from here on
@@ -695,17 +706,17 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
   } else if (lv.cnt > 0) {
     int32_t np = lv.cnt;
     if (!lv.marked) {
-      if (!team_take<G>(a, sm, lv, 0, deadline)) return TEAM_STOP;
+      if (!team_take<G>(a, sm, lv, 0, clk)) return TEAM_STOP;
       np = (int32_t)sm.np;
       lv.E = wave_uniform(sm.E);
     }
-    if (np < lv.cnt) ok = team_chunks<G>(a, sm, lv, np, lv.E, here, deadline, nx);
-    else if (lv.E <= (uint32_t)G::T) ok = team_chunk<G, 1>(a, sm, lv, here, deadline, nx);
-    else if (lv.E <= 2u * G::T) ok = team_chunk<G, 2>(a, sm, lv, here, deadline, nx);
-    else ok = team_chunk<G, G::EPT>(a, sm, lv, here, deadline, nx);
+    if (np < lv.cnt) ok = team_chunks<G>(a, sm, lv, np, lv.E, here, clk, nx);
+    else if (lv.E <= (uint32_t)G::T) ok = team_chunk<G, 1>(a, sm, lv, here, clk, nx);
+    else if (lv.E <= 2u * G::T) ok = team_chunk<G, 2>(a, sm, lv, here, clk, nx);
+    else ok = team_chunk<G, G::EPT>(a, sm, lv, here, clk, nx);
     if (!ok) return TEAM_STOP;
   } else {
-    if (!team_meet<G>(a, sm, lv, here, deadline)) return sm.verdict == TEAM_PASSED ? TEAM_PASSED : TEAM_STOP;
+    if (!team_meet<G>(a, sm, lv, here, clk)) return sm.verdict == TEAM_PASSED ? TEAM_PASSED : TEAM_STOP;
     __syncthreads();
     nx.split = team_split(a, lv.members, sm.met[1], sm.met[2], sm.met[3]);
     nx.marked = true;
@@ -720,7 +731,7 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
   const uint32_t tag = lv.tag++;
   lv.base += 1ull << 32;
   if (nx.split) {
-    const uint32_t v = team_counts<G>(a, sm, tag, lv.members, deadline);
+    const uint32_t v = team_counts<G>(a, sm, tag, lv.members, clk);
     if (v != TEAM_ON) return v;
     const int32_t m = (int32_t)sm.mnext, gn = (int32_t)sm.gnext;
     if (m == 0 || gn <= sm.g) return TEAM_PASSED;
@@ -740,7 +751,7 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
 
 // A workgroup that does not lead: watches the leader's word and takes part in the levels it is counted in.
 template <class G>
-__device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, uint64_t deadline) {
+__device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, TeamClock& clk) {
   uint32_t seen = a.tag0;
   for (;;) {
     if (wave_id() == 0) {
@@ -750,7 +761,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, ui
         tag = wave_uniform((uint32_t)(w >> 32));
         gn = wave_uniform((uint32_t)w >> kTeamNodeBits);
         if (tag > seen && (int32_t)gn > sm.g) break;
-        if (team_stop(a, deadline, spin)) {
+        if (team_stop(a, clk, spin)) {
           v = TEAM_STOP;
           break;
         }
@@ -776,14 +787,14 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, ui
     lv.base = r1;
     const int32_t regions = (int32_t)wave_uniform((uint32_t)(r0 >> 32));
     __syncthreads();
-    uint32_t v = team_counts<G>(a, sm, seen, regions, deadline);
+    uint32_t v = team_counts<G>(a, sm, seen, regions, clk);
     if (v == TEAM_ON) {
       const int32_t m = (int32_t)sm.mnext;
       if (m > 0) {
         team_even<G>(sm, lv, m, gn, regions);
         do {
           seen = lv.tag;
-          v = team_level<G>(a, sm, lv, 0u, deadline);
+          v = team_level<G>(a, sm, lv, 0u, clk);
         } while (v == TEAM_ON);
         // the leader's word of a redistribution after `seen` may count this workgroup again only later
       }
@@ -797,7 +808,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, ui
 // position. *stop when the launch is over.
 template <class G>
 __device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm, int32_t start, bool bfs, uint32_t epoch,
-                                             uint64_t deadline, uint32_t* tag, int32_t* levels, int32_t* last,
+                                             TeamClock& clk, uint32_t* tag, int32_t* levels, int32_t* last,
                                              bool* stop) {
   const int tid = threadIdx.x;
   const uint32_t rb = (uint32_t)a.row_ptr[start], d = (uint32_t)a.row_ptr[start + 1] - rb;
@@ -820,13 +831,13 @@ __device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm,
     // here = 0 when the watchdog fires (a leader on its own waits for nobody, so it looks at the clock here)
     if (tid == 0) {
       if (here < (uint32_t)a.members) here = min(ld_sync(&a.ctl->ticket), (uint32_t)a.members);
-      if (lv.tag % 64u == 0u && wall_ticks() > deadline) {
+      if (lv.tag % 64u == 0u && team_late(a, clk)) {
         team_fail(a, ERR_TIMEOUT);
         here = 0;
       }
     }
     const int32_t pos = lv.pos;
-    const uint32_t v = team_level<G>(a, sm, lv, here, deadline);
+    const uint32_t v = team_level<G>(a, sm, lv, here, clk);
     if (v == TEAM_STOP) {
       *stop = true;
       break;
@@ -844,14 +855,16 @@ __device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm,
 
 // The leader: the search and order of solo_matrix (engine_solo.hpp), a pass at a time.
 template <class G>
-__device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, uint64_t deadline) {
+__device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, TeamClock& clk) {
   const int tid = threadIdx.x, ln = lane_id();
   const int32_t n = a.n;
   constexpr uint32_t kEpochs = 255;  // passes until the claims must be cleared again
+  const uint64_t launch = clk.t0;
   bool searching = a.mode != SOLO_RUN && a.start < 0 && n > 1, redo = false, stop = false;
   int32_t cur = a.start >= 0 ? a.start : n > 1 ? n / 2 : 0;
   int32_t iters = a.start < 0 && n == 1 ? 1 : 0, passes = 0, placed = n, lev = 0, last = 0;
   uint32_t tag = a.tag0, lastdist = 0, left = kEpochs;
+  SearchPasses due;
   while (searching || a.mode != SOLO_SEARCH) {
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && a.mode == SOLO_ORDER && a.speculate > 0 && iters >= a.speculate;
@@ -860,14 +873,22 @@ __device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, ui
       left = kEpochs;
     }
     --left;
-    placed = team_pass<G>(a, sm, cur, searching && !attempt, left, deadline, &tag, &lev, &last, &stop);
+    clk.deadline = min(launch + a.budget_ticks * due.count, wall_ticks() + a.budget_ticks);
+    clk.t0 = clk.deadline - a.budget_ticks * due.count;  // its own word moves the leader's deadline no further
+    if (tid == 0) {
+      st_sync(&a.ctl->passes, (int32_t)due.count);
+      if (passes > 0) pass_beat(a.beat, launch);
+    }
+    placed = team_pass<G>(a, sm, cur, searching && !attempt, left, clk, &tag, &lev, &last, &stop);
     ++passes;
     if (placed != n || stop || !searching) break;
     if ((uint32_t)lev == lastdist) {  // cur is the start
       if (attempt || a.mode == SOLO_SEARCH) break;
       searching = false;
+      ++due.count;
       continue;
     }
+    due.sweep((uint32_t)lev, attempt);
     redo = attempt;  // a failed attempt is followed by the plain sweep from the same start
     if (redo) continue;
     lastdist = (uint32_t)lev;
@@ -906,7 +927,8 @@ __global__ __launch_bounds__(G::T) void k_team(TeamArgs a) {
   using SM = TeamSmem<G>;
   RCM_LDS(SM, sm);
   const int tid = threadIdx.x;
-  const uint64_t deadline = wall_ticks() + a.budget_ticks;
+  const uint64_t now = wall_ticks();
+  TeamClock clk{now, now + a.budget_ticks};
   if (tid == 0) {
     sm.g = (int32_t)atomic_add_u32(&a.ctl->ticket, 1u);
     sm.ckey[0] = ~0u;
@@ -919,9 +941,9 @@ __global__ __launch_bounds__(G::T) void k_team(TeamArgs a) {
   __syncthreads();
   if (sm.g >= a.members) return;
   if (sm.g == 0)
-    team_lead<G>(a, sm, deadline);
+    team_lead<G>(a, sm, clk);
   else
-    team_help<G>(a, sm, deadline);
+    team_help<G>(a, sm, clk);
 }
 
 // Clears what a launch starts from: claims, the members' words, the control block; with tag0 0 the stages too (fresh

@@ -359,6 +359,7 @@ struct rcm_ctx {
   Control* ctl = nullptr;
   uint32_t* scratch = nullptr;  // 16 words: validation flags, bandwidth
   Control* h_ctl = nullptr;     // pinned
+  uint32_t* h_beat = nullptr;   // pinned, behind it: changes with every pass of a search
   int32_t dirty = 0;  // batch records [0, dirty) may hold values from earlier runs
   int max_resident[kVariants] = {};  // co-resident workgroups of each variant
   rcm_mx::DevArena lscratch;         // level-synchronous engine scratch
@@ -421,15 +422,25 @@ void poll_pause(int64_t ms) {
   else std::this_thread::sleep_for(std::chrono::microseconds(20));
 }
 
-int wait_stream(rcm_ctx* c, hipEvent_t ev, int64_t limit_ms) {
+// Waits for `ev`, for limit_ms at most; with `beat` (a pinned word that the device changes), for that long since its last
+// change.
+int wait_event(hipEvent_t ev, int64_t limit_ms, const uint32_t* beat = nullptr) {
   const auto t0 = std::chrono::steady_clock::now();
+  auto since = t0;
+  uint32_t seen = 0;
   for (;;) {
     const hipError_t q = hipEventQuery(ev);
     if (q == hipSuccess) return RCM_OK;
     if (q != hipErrorNotReady) return RCM_EDEVICE;
-    const auto ms = std::chrono::duration_cast<std::chrono::milliseconds>(std::chrono::steady_clock::now() - t0).count();
-    if (ms > limit_ms) return RCM_ETIMEOUT;
-    poll_pause(ms);
+    const auto now = std::chrono::steady_clock::now();
+    if (beat) {
+      const uint32_t b = __atomic_load_n(beat, __ATOMIC_RELAXED);
+      if (b != seen) since = now;
+      seen = b;
+    }
+    const auto ms = [&](auto from) { return std::chrono::duration_cast<std::chrono::milliseconds>(now - from).count(); };
+    if (ms(since) > limit_ms) return RCM_ETIMEOUT;
+    poll_pause(ms(t0));
   }
 }
 
@@ -500,6 +511,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
   *rc = [&]() -> int {
     TeamArgs a{};
     const uint64_t budget = (uint64_t)c->timeout_ms * 100000ull;
+    *c->h_beat = 0;
     RCM_HIP(hipEventRecord(c->ev[0], c->stream));
     if (team) {
       const size_t words = (size_t)kTeamMax * (size_t)c->team_cap * 2;
@@ -522,6 +534,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       a.alone = kTeamAlone;
       a.tag0 = c->team_tag < (1u << 30) ? c->team_tag : 0;  // a launch raises it by less than 2^31
       a.budget_ticks = budget;
+      a.beat = c->h_beat;
       c->team_tag = 0;  // until the launch is known to have ended well
       hipLaunchKernelGGL(k_team_init, dim3(256), dim3(256), 0, c->stream, a);
       RCM_HIP(hipEventRecord(c->ev[1], c->stream));
@@ -530,7 +543,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
       // the result goes to pinned host memory as the kernel ends: no copy after it
       hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
-                         budget, c->h_ctl);
+                         budget, c->h_beat, c->h_ctl);
     }
     RCM_HIP(hipGetLastError());
     RCM_HIP(hipEventRecord(c->ev[2], c->stream));
@@ -538,7 +551,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
       RCM_HIP(hipEventRecord(c->ev[3], c->stream));
     }
-    const int st = wait_stream(c, c->ev[team ? 3 : 2], c->timeout_ms + 10000);
+    const int st = wait_event(c->ev[team ? 3 : 2], c->timeout_ms + 10000, c->h_beat);
     if (st) return st;
     float ms_init = 0.f, ms = 0.f;
     if (team) RCM_HIP(hipEventElapsedTime(&ms_init, c->ev[0], c->ev[1]));
@@ -615,7 +628,7 @@ int run_engine(rcm_ctx* c, int32_t start, bool bfs, bool levels = false) {
   RCM_HIP(hipEventRecord(c->ev[2], c->stream));
   RCM_HIP(hipMemcpyAsync(c->h_ctl, c->ctl, sizeof(Control), hipMemcpyDeviceToHost, c->stream));
   RCM_HIP(hipEventRecord(c->ev[3], c->stream));
-  int rc = wait_stream(c, c->ev[3], c->timeout_ms + 10000);
+  int rc = wait_event(c->ev[3], c->timeout_ms + 10000);
   if (rc) return rc;
   float ms_init = 0.f, ms_run = 0.f;
   RCM_HIP(hipEventElapsedTime(&ms_init, c->ev[0], c->ev[1]));
@@ -776,6 +789,7 @@ struct rcm_batch {
   ManyControl* g = nullptr;
   // pinned host mirrors
   ManyControl* h_g = nullptr;  // the launch control of the last launch (its abort word: the watchdog fired)
+  uint32_t* h_beat = nullptr;  // behind it, on a line of its own: changes with every pass of the one-workgroup engine
   Control* h_ctl = nullptr;
   int32_t* h_tail = nullptr;
   // graph of the run launches (reset + reorder [+ reverse]), per reverse flag
@@ -966,6 +980,7 @@ void enqueue_solo(rcm_batch* b, int32_t mode) {
   m.mode = mode;
   m.speculate = (int32_t)b->speculate;
   m.budget_ticks = (uint64_t)b->timeout_ms * 100000ull;
+  m.beat = b->h_beat;
   const int grid = std::max(1, std::min(m.count, b->workers > 0 ? std::min((int)b->workers, b->solo_resident)
                                                                 : b->solo_resident));
   hipLaunchKernelGGL(k_solo_reset, dim3(1), dim3(64), 0, b->stream, m.next);
@@ -994,16 +1009,8 @@ int collect_status(rcm_batch* b, const int32_t* order, int32_t count, int32_t* s
   return worst;
 }
 
-int batch_wait(rcm_batch* b, hipEvent_t ev) {
-  const auto t0 = std::chrono::steady_clock::now();
-  for (;;) {
-    const hipError_t q = hipEventQuery(ev);
-    if (q == hipSuccess) return RCM_OK;
-    if (q != hipErrorNotReady) return RCM_EDEVICE;
-    const auto ms = std::chrono::duration_cast<std::chrono::milliseconds>(std::chrono::steady_clock::now() - t0).count();
-    if (ms > b->timeout_ms + 10000) return RCM_ETIMEOUT;
-    poll_pause(ms);
-  }
+int batch_wait(rcm_batch* b, hipEvent_t ev, const uint32_t* beat = nullptr) {
+  return wait_event(ev, b->timeout_ms + 10000, beat);
 }
 
 }  // namespace
@@ -1522,7 +1529,8 @@ int rcm_ctx_create(int device, rcm_ctx** out) {
   for (auto& e : c->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
   ok = ok && dev_alloc(&c->ctl, 1) == hipSuccess && dev_alloc(&c->scratch, 16) == hipSuccess &&
        dev_alloc(&c->prof, kProfSlots) == hipSuccess;
-  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), sizeof(Control), hipHostMallocDefault) == hipSuccess;
+  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&c->h_ctl), 2 * sizeof(Control), hipHostMallocDefault) == hipSuccess;
+  if (ok) c->h_beat = reinterpret_cast<uint32_t*>(c->h_ctl + 1);
   ok = ok && hipHostMalloc(reinterpret_cast<void**>(&c->h_word), rcm_mx::kPinnedWords * sizeof(uint32_t),
                             hipHostMallocDefault) == hipSuccess;
   hipDeviceProp_t prop;
@@ -1910,8 +1918,11 @@ int rcm_batch_create(int device, rcm_batch** out) {
   b->device = device;
   bool ok = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) == hipSuccess;
   for (auto& e : b->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
-  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&b->h_g), sizeof(ManyControl), hipHostMallocDefault) == hipSuccess;
-  if (ok) *b->h_g = ManyControl{};
+  ok = ok && hipHostMalloc(reinterpret_cast<void**>(&b->h_g), 256, hipHostMallocDefault) == hipSuccess;
+  if (ok) {
+    *b->h_g = ManyControl{};
+    b->h_beat = reinterpret_cast<uint32_t*>(b->h_g) + 32;
+  }
   hipDeviceProp_t prop;
   ok = ok && hipGetDeviceProperties(&prop, device) == hipSuccess;
   for (int v = 0; ok && v < kVariants; ++v) {
@@ -2138,11 +2149,12 @@ int batch_solo_pass(rcm_batch* b, int32_t mode, const std::vector<int32_t>& give
                     int32_t* status) {
   const int32_t C = b->count;
   RCM_HIP(hipMemcpyAsync(b->d_starts, given.data(), (size_t)C * sizeof(int32_t), hipMemcpyHostToDevice, b->stream));
+  *b->h_beat = 0;
   enqueue_solo(b, mode);
   RCM_HIP(hipGetLastError());
   RCM_HIP(hipMemcpyAsync(b->h_ctl, b->ctl, (size_t)C * sizeof(Control), hipMemcpyDeviceToHost, b->stream));
   RCM_HIP(hipEventRecord(b->ev[3], b->stream));
-  const int wr = batch_wait(b, b->ev[3]);
+  const int wr = batch_wait(b, b->ev[3], b->h_beat);
   if (wr) return wr;
   *b->h_g = ManyControl{};  // the batch engine's abort word: not this launch's
   (void)collect_status(b, b->solo.data(), (int32_t)b->solo.size(), status, nullptr);
@@ -2974,7 +2986,7 @@ int rcm_gpu_batch_noalloc(int32_t n, int64_t nnz, const int32_t* d_row_ptr, cons
   if (solo) {  // start search and order in one launch of one workgroup
     const SoloJob J{d_row_ptr, d_col_idx, d_perm_out, a.qinfo, n};
     hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, nullptr, J, (int32_t)SOLO_ORDER, start,
-                       (int32_t)kDefaultSpeculate, a.budget_ticks, a.ctl);
+                       (int32_t)kDefaultSpeculate, a.budget_ticks, nullptr, a.ctl);
     RCM_HIP(hipGetLastError());
     Control h{};
     RCM_HIP(hipMemcpy(&h, a.ctl, sizeof(Control), hipMemcpyDeviceToHost));

@@ -96,6 +96,61 @@ def test_emulated_endless_search(mode):
     assert E.run_team(*ENDLESS, -1, workers=2, mode=mode, timeout_s=0.2)[1][0] == 1
 
 
+@pytest.mark.parametrize("engine", ["solo", "team"])
+def test_emulated_watchdog_of_each_pass(engine):
+    """The budget is for each pass of a search, as where each is a launch of its own."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+    import time
+
+    def order(rp, ci, timeout_s):
+        if engine == "solo":
+            perms, info = E.run_solo([(rp, ci)], [-1], workers=1, mode=2, timeout_s=timeout_s)
+            return perms[0], info[0]
+        return E.run_team(rp, ci, -1, workers=2, mode=2, timeout_s=timeout_s, alone=1 << 20)
+
+    rp, ci = G.path(300)
+    _, s, it, _ = O.peripheral(rp, ci)
+    t0 = time.perf_counter()
+    order(rp, ci, 100.0)
+    total = time.perf_counter() - t0
+    perm, info = order(rp, ci, 0.6 * total)
+    assert info[5] >= 3  # passes of equal length but for the first, half as long: none takes 0.6 of them all
+    assert info[0] == 0 and (info[3], info[4]) == (s, it) and np.array_equal(perm, O.cm(rp, ci, s))
+    assert order(rp, ci, 0.1 * total)[1][0] == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [30000, 40000])
+def test_gpu_watchdog_of_each_pass(rows):
+    """The same for a context (one workgroup, a team) and a set: a timeout that every pass keeps but not all together."""
+    m = P.CSR(*G.path(rows))
+    endless = P.CSR(*ENDLESS)
+    print("[case]", rows, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c, P.RcmBatch(timeout_ms=20000) as b:
+        c.load(m)
+        c.run(0)
+        limit = int(1.4 * c.timing().run_kernel_ms)  # the whole search and order: 2.5 passes from an end
+        s, it = c.order()
+        want = c.perm()
+        c.set_param("timeout_ms", limit)
+        assert c.order() == (s, it) and np.array_equal(c.perm(), want)
+        assert c.find_start() == s
+        c.set_param("timeout_ms", max(1, limit // 4))
+        assert c.run_status(0) == P.RCM_ETIMEOUT
+        c.set_param("timeout_ms", 20)
+        c.load(endless)
+        with pytest.raises(P.RcmError) as e:
+            c.order()
+        assert e.value.status == P.RCM_ETIMEOUT
+        b.load(P.BatchSet.from_matrices([m, m, P.CSR(*G.path(9))]))
+        b.run([0, 0, 0])
+        b.set_param("timeout_ms", int(1.4 * b.timing().run_ms))
+        starts, iters, st = b.order()
+        assert not st.any() and (starts[0], iters[0]) == (s, it)
+        assert all(np.array_equal(p, want) for p in b.perms()[:2])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(CASES) + ["rows63x9000", "rgg65536", "grid65537"])
 def test_gpu_single(name):
