@@ -400,7 +400,7 @@ int ensure_state(rcm_ctx* c, int32_t n) {
   return RCM_OK;
 }
 
-// The team engine's memory for n rows: allocated when a matrix first needs it, kept and grown.
+// The team engine's memory for n rows: allocated when a matrix that needs it is loaded, kept and grown.
 bool ensure_team(rcm_ctx* c, int32_t n) {
   const int32_t cap = team_cap(n);
   if (c->team && c->team_cap >= cap) return true;
@@ -502,11 +502,14 @@ bool ctx_quick(const rcm_ctx* c) {
   return ctx_automatic(c) && c->maxdeg <= (uint32_t)kSoloMaxRow && c->n <= kTeamMaxN && !c->team_off;
 }
 
+// Whether that is a team.
+bool ctx_team(const rcm_ctx* c) { return ctx_quick(c) && c->n > kCtxSolo; }
+
 // One launch of the level engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl. False when
 // it takes the matrix no further (ctx_quick, no memory for a team, a stage region too small): the batch engine's.
 bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
   if (!ctx_quick(c)) return false;
-  const bool team = c->n > kCtxSolo;
+  const bool team = ctx_team(c);
   if (team && !ensure_team(c, c->n)) return false;
   *rc = [&]() -> int {
     TeamArgs a{};
@@ -729,6 +732,7 @@ int load_common(rcm_ctx* c, int32_t n, int64_t nnz) {
   c->n = n;
   c->nnz = nnz;
   c->have_perm = false;
+  if (ctx_team(c)) (void)ensure_team(c, n);  // tried again by a run; without it the batch engine runs the matrix
   return RCM_OK;
 }
 

@@ -153,6 +153,21 @@ def test_gpu_context(name):
 
 
 @pytest.mark.gpu
+def test_gpu_memory_at_load():
+    """A run allocates nothing: the team's memory is there when the matrix is loaded."""
+    import torch
+
+    with P.RcmContext(timeout_ms=20000) as c:
+        for name in ("stencil33", "past_bitmap"):
+            c.load(P.CSR(*GPU_CASES[name]()))
+            print("[case]", name, flush=True)
+            free = torch.cuda.mem_get_info()[0]
+            c.order()
+            assert c.timing().workers == 128
+            assert torch.cuda.mem_get_info()[0] == free
+
+
+@pytest.mark.gpu
 def test_gpu_reload_and_refuse():
     """A larger matrix after a smaller one (the memory grows), a disconnected one, and the smaller one again."""
     small, big = GPU_CASES["stencil33"](), G.random_connected(300000, 300000, seed=4)
