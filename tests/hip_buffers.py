@@ -38,6 +38,11 @@ class HipBuffers:
         assert self.L.hipMemcpy(a.ctypes.data_as(C.c_void_p), p, a.nbytes, 2) == 0  # device to host
         return a
 
+    def free_bytes(self):
+        free, total = C.c_size_t(), C.c_size_t()
+        assert self.L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
     def close(self):
         for p in self.bufs:
             self.L.hipFree(p)

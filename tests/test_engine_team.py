@@ -155,16 +155,16 @@ def test_gpu_context(name):
 @pytest.mark.gpu
 def test_gpu_memory_at_load():
     """A run allocates nothing: the team's memory is there when the matrix is loaded."""
-    import torch
+    from hip_buffers import HipBuffers
 
-    with P.RcmContext(timeout_ms=20000) as c:
+    with P.RcmContext(timeout_ms=20000) as c, HipBuffers() as hip:
         for name in ("stencil33", "past_bitmap"):
             c.load(P.CSR(*GPU_CASES[name]()))
             print("[case]", name, flush=True)
-            free = torch.cuda.mem_get_info()[0]
+            free = hip.free_bytes()
             c.order()
             assert c.timing().workers == 128
-            assert torch.cuda.mem_get_info()[0] == free
+            assert hip.free_bytes() == free
 
 
 @pytest.mark.gpu
