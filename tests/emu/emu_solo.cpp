@@ -124,8 +124,8 @@ int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const i
                  const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate,
                  int32_t geo, int32_t* perm_cat, int32_t* info, double timeout_s) {
   if (count <= 0 || workers <= 0) return -1;
-  return geo ? run<SoloGeo<512, 2048, 1 << 16>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode, speculate,
-                                               perm_cat, info, timeout_s)
+  return geo ? run<SoloGeo<1024, 4096, kSoloMaxN>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode, speculate,
+                                                 perm_cat, info, timeout_s)
              : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
                                                    speculate, perm_cat, info, timeout_s);
 }

@@ -62,6 +62,19 @@ def test_emulated_order_and_search(geo):
             assert np.array_equal(perms[k], O.cm(rp, ci, s)), (names[k], spec)
 
 
+def test_emulated_full_chunks():
+    """The library's geometry on levels wider than its chunks of 4096 slots."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    mats = [CASES[name]() for name in ("rows63", "random1500", "stencil11x9x13")]
+    perms, info = E.run_solo(mats, [-1] * len(mats), workers=2, mode=2, geo=1)
+    for k, (rp, ci) in enumerate(mats):
+        _, s, it, _ = O.peripheral(rp, ci)
+        assert info[k, 0] == 0 and (info[k, 3], info[k, 4]) == (s, it), k
+        assert np.array_equal(perms[k], O.cm(rp, ci, s)), k
+
+
 def test_emulated_directed_and_disconnected():
     pytest.importorskip("emu_lib")
     import emu_lib as E
