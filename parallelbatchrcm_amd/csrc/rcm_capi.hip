@@ -502,6 +502,9 @@ bool ctx_quick(const rcm_ctx* c) {
   return ctx_automatic(c) && c->maxdeg <= (uint32_t)kSoloMaxRow && c->n <= kTeamMaxN && !c->team_off;
 }
 
+// RCM_PARAM_SPECULATE as the level engines take it.
+int32_t sweep_number(int64_t speculate) { return (int32_t)std::min<int64_t>(speculate, INT32_MAX); }
+
 // Whether that is a team.
 bool ctx_team(const rcm_ctx* c) { return ctx_quick(c) && c->n > kCtxSolo; }
 
@@ -532,7 +535,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       a.members = kTeamMax;
       a.mode = mode;
       a.start = start;
-      a.speculate = (int32_t)std::min<int64_t>(c->speculate, INT32_MAX);
+      a.speculate = sweep_number(c->speculate);
       a.wide = team_wide(c->n, c->nnz);
       a.alone = kTeamAlone;
       a.tag0 = c->team_tag < (1u << 30) ? c->team_tag : 0;  // a launch raises it by less than 2^31
@@ -545,7 +548,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
     } else {
       const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
       // the result goes to pinned host memory as the kernel ends: no copy after it
-      hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, (int32_t)c->speculate,
+      hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, sweep_number(c->speculate),
                          budget, c->h_beat, c->h_ctl);
     }
     RCM_HIP(hipGetLastError());
@@ -982,7 +985,7 @@ void enqueue_solo(rcm_batch* b, int32_t mode) {
   m.next = b->solo_next;
   m.count = (int32_t)b->solo.size();
   m.mode = mode;
-  m.speculate = (int32_t)b->speculate;
+  m.speculate = sweep_number(b->speculate);
   m.budget_ticks = (uint64_t)b->timeout_ms * 100000ull;
   m.beat = b->h_beat;
   const int grid = std::max(1, std::min(m.count, b->workers > 0 ? std::min((int)b->workers, b->solo_resident)

@@ -111,3 +111,21 @@ def test_tuning_times_the_default(graph):
         assert 0 < r.best_ms <= r.default_ms and min(times) / 2 < r.default_ms < 2 * max(times)
         assert not b.run([s] * 3).any()
         assert all(np.array_equal(p, order) for p in b.perms())
+
+
+def test_speculate_beyond_32_bits():
+    """A sweep number that no search reaches means no speculation, however large."""
+    rp, ci = CASES["grid24x20"]()
+    _say("speculate")
+    with P.RcmContext(timeout_ms=20000) as c, P.RcmBatch(timeout_ms=20000) as b:
+        c.load(P.CSR(rp, ci))
+        b.load(P.BatchSet.from_matrices([P.CSR(rp, ci)]))
+        passes = []
+        for v in (0, (1 << 32) + 1, 1):
+            c.set_param("speculate", v)
+            b.set_param("speculate", v)
+            s, it = c.order()
+            assert np.array_equal(c.perm(), O.cm(rp, ci, s))
+            assert b.order()[0][0] == s and np.array_equal(b.perms()[0], c.perm())
+            passes.append(c.timing().order_passes)
+        assert passes[0] == passes[1] == it + 1 and passes[2] > it + 1
