@@ -407,7 +407,7 @@ __device__ __forceinline__ void pass_beat(uint32_t* beat, uint64_t t0) {
 // Which passes of a search the watchdog counts. In a symmetric matrix every sweep is longer than the one before or confirms
 // it; in others the sweeps may repeat for ever, so one that does neither moves the deadline no further.
 struct SearchPasses {
-  uint32_t count = 1, longest = 0;
+  uint32_t count, longest;  // 1 and 0 at first
   __device__ __forceinline__ void sweep(uint32_t lev, bool attempt) {  // the sweep after it is due, and an attempt's repeat
     if (lev <= longest) return;
     longest = lev;
@@ -430,7 +430,7 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
   int32_t cur = start >= 0 ? start : n > 1 ? n / 2 : 0;
   int32_t iters = start < 0 && n == 1 ? 1 : 0, passes = 0, placed = n, lev = 0;
   uint32_t steps = 0, lastdist = 0;
-  SearchPasses due;
+  SearchPasses due{1u, 0u};
   bool expired = wall_ticks() > clk.deadline();  // thread 0's word counts, below
   if (tid == 0) sm.quit = expired ? 1u : 0u;
   __syncthreads();

@@ -106,6 +106,8 @@ struct TeamSmem {
   uint32_t pre[kTeamMax + 1];  // redistribution: parents before each region
   uint32_t np, E;            // of a taken chunk: parents, slots
   uint32_t verdict, lost;
+  uint64_t launch, t0, deadline;  // the watchdog
+  SearchPasses due;          // thread 0 of the leader
   // of the meeting: parents of the members before, of all, of the largest part; workgroups started
   alignas(16) uint32_t met[4];
   uint32_t mnext, gnext;     // of a redistribution: parents of the next level, its members
@@ -138,21 +140,22 @@ __device__ __forceinline__ void team_fail(const TeamArgs& a, uint32_t err) {
   st_sync(&a.ctl->done, 1u);
 }
 
-// The watchdog (as SoloClock): the leader says in ctl->passes how many passes are due; who runs out of time looks there.
-struct TeamClock {
-  uint64_t t0, deadline;
-};
-__device__ __forceinline__ bool team_late(const TeamArgs& a, TeamClock& clk) {
-  if (wall_ticks() <= clk.deadline) return false;
-  clk.deadline = max(clk.deadline, clk.t0 + a.budget_ticks * (uint64_t)(uint32_t)ld_sync(&a.ctl->passes));
-  return wall_ticks() > clk.deadline;
+// The watchdog (as SoloClock, in LDS: registers are short here): the leader says in ctl->passes how many passes are due; who
+// runs out of time looks there.
+template <class SM>
+__device__ __forceinline__ bool team_late(const TeamArgs& a, SM& sm) {
+  if (wall_ticks() <= sm.deadline) return false;
+  const uint64_t due = (uint64_t)(uint32_t)ld_sync(&a.ctl->passes);
+  sm.deadline = max(sm.deadline, sm.t0 + a.budget_ticks * due);
+  return wall_ticks() > sm.deadline;
 }
 
 // One wave: whether to give up waiting (the launch is over, or the watchdog fires). Looked at on every 16th poll.
-__device__ __forceinline__ bool team_stop(const TeamArgs& a, TeamClock& clk, uint32_t spin) {
+template <class SM>
+__device__ __forceinline__ bool team_stop(const TeamArgs& a, SM& sm, uint32_t spin) {
   if (spin % 16u != 15u) return false;
   if (wave_uniform(ld_sync(&a.ctl->done))) return true;
-  if (wave_uniform(team_late(a, clk) ? 1u : 0u)) {
+  if (wave_uniform(team_late(a, sm) ? 1u : 0u)) {
     if (lane_id() == 0) team_fail(a, ERR_TIMEOUT);
     return true;
   }
@@ -166,14 +169,19 @@ __device__ __forceinline__ int32_t team_wanted(const TeamArgs& a, uint32_t width
 }
 
 // Whether the children of a level of `width` parents, the largest part `most`, are redistributed: the members are too few
-// for it, or a quarter of them would do, or one has twice its share. (The limits are flat: growth from 1, 2 or 3 times
-// the wanted part, imbalance of 2 or 3 above 2, 4 or 6 times it, 8 to 32 parents a part: within 10% of each other on
-// 2D, 3D and geometric graphs.)
-__device__ __forceinline__ bool team_split(const TeamArgs& a, int32_t members, uint32_t width, uint32_t most,
+// for it, or a quarter of them would do, or one has twice its share, or it is many times all levels before: then
+// its children may be as many times more, and most of them the first members', who claim first. (The limits are flat:
+// growth from 1, 2 or 3 times the wanted part, imbalance of 2 or 3 above 2, 4 or 6 times it, 8 to 32 parents a part: within
+// 10% of each other on 2D, 3D and geometric graphs, which outgrow what is behind them in their first levels only. Random
+// graphs of 33k and 100k rows of 33 entries took 280 and 480 us an order without the last rule, 94 and 185 with it; by the
+// batch engine 122 and 260.)
+constexpr uint32_t kTeamGrowth = 4;
+__device__ __forceinline__ bool team_split(const TeamArgs& a, const TeamLevel& lv, uint32_t width, uint32_t most,
                                            uint32_t here) {
-  const int32_t want = team_wanted(a, width, here);
+  const int32_t want = team_wanted(a, width, here), members = lv.members;
   return (want > members && most > 2u << a.wide) || 4 * want <= members ||
-         (most > 4u << a.wide && most * (uint32_t)members > 2u * width);
+         (most > 4u << a.wide && most * (uint32_t)members > 2u * width) ||
+         (want > 1 && width > kTeamGrowth * (uint32_t)lv.pos);
 }
 
 // The words `which` of the first `members` members, two neighbours to a lane, until every tag is at least `tag`.
@@ -181,8 +189,9 @@ __device__ __forceinline__ bool team_split(const TeamArgs& a, int32_t members, u
 struct TeamWords {
   uint64_t w[kTeamPer];
 };
-__device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, int which, uint32_t tag, int32_t members,
-                                              TeamClock& clk, TeamWords& r) {
+template <class SM>
+__device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, SM& sm, int which, uint32_t tag, int32_t members,
+                                              TeamWords& r) {
   const int l0 = lane_id() * kTeamPer;
   for (uint32_t spin = 0;; ++spin) {
     bool early = false, late = false;
@@ -194,7 +203,7 @@ __device__ __forceinline__ uint32_t team_poll(const TeamArgs& a, int which, uint
     }
     if (ballot(late)) return TEAM_PASSED;
     if (!ballot(early)) return TEAM_ON;
-    if (team_stop(a, clk, spin)) return TEAM_STOP;
+    if (team_stop(a, sm, spin)) return TEAM_STOP;
   }
 }
 __device__ __forceinline__ uint32_t word_count(uint64_t w) { return (uint32_t)w & ((1u << kTeamNodeBits) - 1u); }
@@ -203,8 +212,7 @@ __device__ __forceinline__ uint32_t word_count(uint64_t w) { return (uint32_t)w 
 // those of a later one, sm.verdict is TEAM_PASSED): of a level without parents nobody waits for its members to read the
 // words. Wave 0 has sm.met set when it passes the next barrier.
 template <class G>
-__device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
-                                          TeamClock& clk) {
+__device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here) {
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (lv.members == 1) {
@@ -220,7 +228,7 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
     if (lane_id() == 0)
       st_sync(team_word(a, sm.g, (int)(lv.tag & 1u)), ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
     RCM_TEAM_LINGER(0, sm.g, lv.tag);
-    const uint32_t v = team_poll(a, (int)(lv.tag & 1u), lv.tag, lv.members, clk, r);
+    const uint32_t v = team_poll(a, sm, (int)(lv.tag & 1u), lv.tag, lv.members, r);
     if (lane_id() == 0) sm.verdict = v;
   }
   __syncthreads();
@@ -252,12 +260,11 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
 // The children counts of a redistribution after the level `tag`, whose members are the first `members`: sm.pre, sm.mnext
 // and the leader's sm.gnext. TEAM_PASSED when that is over for this workgroup (the others have gone on without it).
 template <class G>
-__device__ __forceinline__ uint32_t team_counts(const TeamArgs& a, TeamSmem<G>& sm, uint32_t tag, int32_t members,
-                                                TeamClock& clk) {
+__device__ __forceinline__ uint32_t team_counts(const TeamArgs& a, TeamSmem<G>& sm, uint32_t tag, int32_t members) {
   if (wave_id() == 0) {
     TeamWords r;
     RCM_TEAM_LINGER(1, sm.g, tag);
-    const uint32_t v = team_poll(a, kTeamSplitWord, tag, members, clk, r);
+    const uint32_t v = team_poll(a, sm, kTeamSplitWord, tag, members, r);
     uint32_t c = 0;
 #pragma unroll
     for (int i = 0; i < kTeamPer; ++i) c += word_count(r.w[i]);
@@ -309,8 +316,7 @@ __device__ __forceinline__ void team_mark(TeamSmem<G>& sm, uint32_t i, uint32_t 
 // Loads the parents from c0 on of the member's part from the stage, as far as their slots fit a chunk, and marks them;
 // sm.np and sm.E tell how many parents and slots. Ends with a barrier. False when the launch is over.
 template <class G>
-__device__ __forceinline__ bool team_take(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, int32_t c0,
-                                          TeamClock& clk) {
+__device__ __forceinline__ bool team_take(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, int32_t c0) {
   constexpr int T = G::T, S = G::S, W = G::W;
   const int tid = threadIdx.x;
   const int32_t avail = min(lv.cnt - c0, (int32_t)T);
@@ -327,7 +333,7 @@ __device__ __forceinline__ bool team_take(const TeamArgs& a, TeamSmem<G>& sm, co
     const uint64_t* e = a.stage[lv.tag & 1u] + 2 * ((size_t)(lv.region + lo) * (size_t)a.cap + (size_t)((uint32_t)p - first));
     uint64_t e0 = ld_sync(e), e1 = ld_sync(e + 1);
     for (uint32_t spin = 0; (uint32_t)(e0 >> 32) != lv.tag || (uint32_t)(e1 >> 32) != lv.tag; ++spin) {
-      if (spin % 16u == 15u && (ld_sync(&a.ctl->done) || team_late(a, clk))) {
+      if (spin % 16u == 15u && (ld_sync(&a.ctl->done) || team_late(a, sm))) {
         sm.lost = 1;
         break;
       }
@@ -556,7 +562,7 @@ __device__ __forceinline__ bool team_place(const TeamArgs& a, TeamSmem<G>& sm, c
       __syncthreads();
     }
   } else {
-    nx.split = team_split(a, lv.members, width, most, here);
+    nx.split = team_split(a, lv, width, most, here);
   }
   const bool direct = only && !nx.split && cnt <= (uint32_t)T && dsum <= (uint32_t)S;
   if (!direct && nx.placed + cnt > (uint32_t)a.cap) {
@@ -634,19 +640,18 @@ __device__ __forceinline__ bool team_chunk_local(const TeamArgs& a, TeamSmem<G>&
   return team_place<G, KN, true>(a, sm, lv, 0, lv.cnt, lv.E, s, true, true, nx);
 }
 template <class G, int KN>
-__device__ __forceinline__ bool team_chunk(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
-                                           TeamClock& clk, TeamNext& nx) {
+__device__ __forceinline__ bool team_chunk(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here, TeamNext& nx) {
   TeamSlots<KN> s;
   team_expand<G, KN>(a, sm, 0, lv.E, s);
   team_claim<G, KN>(a, lv, lv.E, s);
-  if (!team_meet<G>(a, sm, lv, here, clk)) return false;
+  if (!team_meet<G>(a, sm, lv, here)) return false;
   return team_place<G, KN, false>(a, sm, lv, 0, lv.cnt, lv.E, s, true, true, nx);
 }
 
 // The part when it is more than one chunk: the claims of all of them, the meeting, then the children of each.
 template <class G>
 __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, int32_t np0,
-                                            uint32_t E0, uint32_t here, TeamClock& clk, TeamNext& nx) {
+                                            uint32_t E0, uint32_t here, TeamNext& nx) {
   constexpr int KN = G::EPT;
   TeamSlots<KN> s;
   int32_t np = np0;
@@ -657,14 +662,14 @@ __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, 
     c0 += np;
     if (c0 >= lv.cnt) break;
     __syncthreads();
-    if (!team_take<G>(a, sm, lv, c0, clk)) return false;
+    if (!team_take<G>(a, sm, lv, c0)) return false;
     np = (int32_t)sm.np;
     e = wave_uniform(sm.E);
   }
-  if (!team_meet<G>(a, sm, lv, here, clk)) return false;
+  if (!team_meet<G>(a, sm, lv, here)) return false;
   for (int32_t c0 = 0; c0 < lv.cnt;) {
     __syncthreads();
-    if (!team_take<G>(a, sm, lv, c0, clk)) return false;
+    if (!team_take<G>(a, sm, lv, c0)) return false;
     np = (int32_t)sm.np;
     e = wave_uniform(sm.E);
     team_expand<G, KN>(a, sm, c0, e, s);
@@ -690,8 +695,7 @@ __device__ __forceinline__ bool team_chunks(const TeamArgs& a, TeamSmem<G>& sm, 
 // One level as a member, and the state of the next one in lv. TEAM_PASSED: the pass is over (no parents in this level),
 // or this workgroup is not a member of the next level. here: thread 0 of the leader, the workgroups started.
 template <class G>
-__device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& sm, TeamLevel& lv, uint32_t here,
-                                               TeamClock& clk) {
+__device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& sm, TeamLevel& lv, uint32_t here) {
   TeamNext nx{0, 0, false, false};
   bool ok = true;
   if (lv.local && lv.cnt > 0 && !lv.marked) {  // too wide for one chunk: through the claim words from here on
@@ -706,19 +710,19 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
   } else if (lv.cnt > 0) {
     int32_t np = lv.cnt;
     if (!lv.marked) {
-      if (!team_take<G>(a, sm, lv, 0, clk)) return TEAM_STOP;
+      if (!team_take<G>(a, sm, lv, 0)) return TEAM_STOP;
       np = (int32_t)sm.np;
       lv.E = wave_uniform(sm.E);
     }
-    if (np < lv.cnt) ok = team_chunks<G>(a, sm, lv, np, lv.E, here, clk, nx);
-    else if (lv.E <= (uint32_t)G::T) ok = team_chunk<G, 1>(a, sm, lv, here, clk, nx);
-    else if (lv.E <= 2u * G::T) ok = team_chunk<G, 2>(a, sm, lv, here, clk, nx);
-    else ok = team_chunk<G, G::EPT>(a, sm, lv, here, clk, nx);
+    if (np < lv.cnt) ok = team_chunks<G>(a, sm, lv, np, lv.E, here, nx);
+    else if (lv.E <= (uint32_t)G::T) ok = team_chunk<G, 1>(a, sm, lv, here, nx);
+    else if (lv.E <= 2u * G::T) ok = team_chunk<G, 2>(a, sm, lv, here, nx);
+    else ok = team_chunk<G, G::EPT>(a, sm, lv, here, nx);
     if (!ok) return TEAM_STOP;
   } else {
-    if (!team_meet<G>(a, sm, lv, here, clk)) return sm.verdict == TEAM_PASSED ? TEAM_PASSED : TEAM_STOP;
+    if (!team_meet<G>(a, sm, lv, here)) return sm.verdict == TEAM_PASSED ? TEAM_PASSED : TEAM_STOP;
     __syncthreads();
-    nx.split = team_split(a, lv.members, sm.met[1], sm.met[2], sm.met[3]);
+    nx.split = team_split(a, lv, sm.met[1], sm.met[2], sm.met[3]);
     nx.marked = true;
     if (sm.met[3] == 0) return TEAM_STOP;
     if (wave_uniform((uint32_t)wave_id()) == 0u && nx.split)
@@ -731,7 +735,7 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
   const uint32_t tag = lv.tag++;
   lv.base += 1ull << 32;
   if (nx.split) {
-    const uint32_t v = team_counts<G>(a, sm, tag, lv.members, clk);
+    const uint32_t v = team_counts<G>(a, sm, tag, lv.members);
     if (v != TEAM_ON) return v;
     const int32_t m = (int32_t)sm.mnext, gn = (int32_t)sm.gnext;
     if (m == 0 || gn <= sm.g) return TEAM_PASSED;
@@ -751,7 +755,7 @@ __device__ __forceinline__ uint32_t team_level(const TeamArgs& a, TeamSmem<G>& s
 
 // A workgroup that does not lead: watches the leader's word and takes part in the levels it is counted in.
 template <class G>
-__device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, TeamClock& clk) {
+__device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm) {
   uint32_t seen = a.tag0;
   for (;;) {
     if (wave_id() == 0) {
@@ -761,7 +765,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, Te
         tag = wave_uniform((uint32_t)(w >> 32));
         gn = wave_uniform((uint32_t)w >> kTeamNodeBits);
         if (tag > seen && (int32_t)gn > sm.g) break;
-        if (team_stop(a, clk, spin)) {
+        if (team_stop(a, sm, spin)) {
           v = TEAM_STOP;
           break;
         }
@@ -787,14 +791,14 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, Te
     lv.base = r1;
     const int32_t regions = (int32_t)wave_uniform((uint32_t)(r0 >> 32));
     __syncthreads();
-    uint32_t v = team_counts<G>(a, sm, seen, regions, clk);
+    uint32_t v = team_counts<G>(a, sm, seen, regions);
     if (v == TEAM_ON) {
       const int32_t m = (int32_t)sm.mnext;
       if (m > 0) {
         team_even<G>(sm, lv, m, gn, regions);
         do {
           seen = lv.tag;
-          v = team_level<G>(a, sm, lv, 0u, clk);
+          v = team_level<G>(a, sm, lv, 0u);
         } while (v == TEAM_ON);
         // the leader's word of a redistribution after `seen` may count this workgroup again only later
       }
@@ -807,8 +811,7 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm, Te
 // The leader's pass from `start`: returns the nodes placed; *levels the index of the last level, *last its first queue
 // position. *stop when the launch is over.
 template <class G>
-__device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm, int32_t start, bool bfs, uint32_t epoch,
-                                             TeamClock& clk, uint32_t* tag, int32_t* levels, int32_t* last,
+__device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm, int32_t start, bool bfs, uint32_t epoch, uint32_t* tag, int32_t* levels, int32_t* last,
                                              bool* stop) {
   const int tid = threadIdx.x;
   const uint32_t rb = (uint32_t)a.row_ptr[start], d = (uint32_t)a.row_ptr[start + 1] - rb;
@@ -831,13 +834,13 @@ __device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm,
     // here = 0 when the watchdog fires (a leader on its own waits for nobody, so it looks at the clock here)
     if (tid == 0) {
       if (here < (uint32_t)a.members) here = min(ld_sync(&a.ctl->ticket), (uint32_t)a.members);
-      if (lv.tag % 64u == 0u && team_late(a, clk)) {
+      if (lv.tag % 64u == 0u && team_late(a, sm)) {
         team_fail(a, ERR_TIMEOUT);
         here = 0;
       }
     }
     const int32_t pos = lv.pos;
-    const uint32_t v = team_level<G>(a, sm, lv, here, clk);
+    const uint32_t v = team_level<G>(a, sm, lv, here);
     if (v == TEAM_STOP) {
       *stop = true;
       break;
@@ -855,16 +858,15 @@ __device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm,
 
 // The leader: the search and order of solo_matrix (engine_solo.hpp), a pass at a time.
 template <class G>
-__device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, TeamClock& clk) {
+__device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm) {
   const int tid = threadIdx.x, ln = lane_id();
   const int32_t n = a.n;
   constexpr uint32_t kEpochs = 255;  // passes until the claims must be cleared again
-  const uint64_t launch = clk.t0;
   bool searching = a.mode != SOLO_RUN && a.start < 0 && n > 1, redo = false, stop = false;
   int32_t cur = a.start >= 0 ? a.start : n > 1 ? n / 2 : 0;
   int32_t iters = a.start < 0 && n == 1 ? 1 : 0, passes = 0, placed = n, lev = 0, last = 0;
   uint32_t tag = a.tag0, lastdist = 0, left = kEpochs;
-  SearchPasses due;
+  if (tid == 0) sm.due = SearchPasses{1u, 0u};
   while (searching || a.mode != SOLO_SEARCH) {
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && a.mode == SOLO_ORDER && a.speculate > 0 && iters >= a.speculate;
@@ -873,22 +875,22 @@ __device__ __forceinline__ void team_lead(const TeamArgs& a, TeamSmem<G>& sm, Te
       left = kEpochs;
     }
     --left;
-    clk.deadline = min(launch + a.budget_ticks * due.count, wall_ticks() + a.budget_ticks);
-    clk.t0 = clk.deadline - a.budget_ticks * due.count;  // its own word moves the leader's deadline no further
     if (tid == 0) {
-      st_sync(&a.ctl->passes, (int32_t)due.count);
-      if (passes > 0) pass_beat(a.beat, launch);
+      st_sync(&a.ctl->passes, (int32_t)sm.due.count);
+      sm.deadline = min(sm.launch + a.budget_ticks * sm.due.count, wall_ticks() + a.budget_ticks);
+      sm.t0 = sm.deadline - a.budget_ticks * sm.due.count;  // its own word moves the leader's deadline no further
+      if (passes > 0) pass_beat(a.beat, sm.launch);
     }
-    placed = team_pass<G>(a, sm, cur, searching && !attempt, left, clk, &tag, &lev, &last, &stop);
+    placed = team_pass<G>(a, sm, cur, searching && !attempt, left, &tag, &lev, &last, &stop);
     ++passes;
     if (placed != n || stop || !searching) break;
     if ((uint32_t)lev == lastdist) {  // cur is the start
       if (attempt || a.mode == SOLO_SEARCH) break;
       searching = false;
-      ++due.count;
+      if (tid == 0) ++sm.due.count;
       continue;
     }
-    due.sweep((uint32_t)lev, attempt);
+    if (tid == 0) sm.due.sweep((uint32_t)lev, attempt);
     redo = attempt;  // a failed attempt is followed by the plain sweep from the same start
     if (redo) continue;
     lastdist = (uint32_t)lev;
@@ -927,9 +929,9 @@ __global__ __launch_bounds__(G::T) void k_team(TeamArgs a) {
   using SM = TeamSmem<G>;
   RCM_LDS(SM, sm);
   const int tid = threadIdx.x;
-  const uint64_t now = wall_ticks();
-  TeamClock clk{now, now + a.budget_ticks};
   if (tid == 0) {
+    sm.launch = sm.t0 = wall_ticks();
+    sm.deadline = sm.t0 + a.budget_ticks;
     sm.g = (int32_t)atomic_add_u32(&a.ctl->ticket, 1u);
     sm.ckey[0] = ~0u;
     sm.lost = 0;
@@ -941,9 +943,9 @@ __global__ __launch_bounds__(G::T) void k_team(TeamArgs a) {
   __syncthreads();
   if (sm.g >= a.members) return;
   if (sm.g == 0)
-    team_lead<G>(a, sm, clk);
+    team_lead<G>(a, sm);
   else
-    team_help<G>(a, sm, clk);
+    team_help<G>(a, sm);
 }
 
 // Clears what a launch starts from: claims, the members' words, the control block; with tag0 0 the stages too (fresh

@@ -153,6 +153,21 @@ def test_gpu_context(name):
 
 
 @pytest.mark.gpu
+def test_gpu_growing_levels():
+    """Levels that grow thirtyfold stay within the members' regions: spread before the first members have claimed most of
+    the next one."""
+    rp, ci = G.random_connected(200000, 3000000, seed=6)
+    assert np.diff(rp).max() <= 64
+    m = P.CSR(rp, ci)
+    print("[case]", m.rows, m.nnz, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        c.run(7)
+        assert c.timing().workers == 128
+        assert np.array_equal(c.perm(), O.cm(rp, ci, 7))
+
+
+@pytest.mark.gpu
 def test_gpu_memory_at_load():
     """A run allocates nothing: the team's memory is there when the matrix is loaded."""
     from hip_buffers import HipBuffers
