@@ -343,10 +343,16 @@ __device__ __forceinline__ bool solo_step(const SoloJob& J, SoloSmem<G>& sm, Sol
   return direct;
 }
 
-// One pass over the matrix from `start`: the CM order (or the plain BFS order) into perm. Returns the nodes placed;
-// *levels the index of the last level. sm.quit is set when the watchdog fired.
+// When a matrix is given up, for an engine of more workgroups: when more than `level` slots wait (about a level's; at least a
+// chunk's) with more than `spare` entries of the matrix still to expand -- `growing`, if they are four times those expanded.
+struct SoloGiveUp {
+  uint32_t level, spare, growing;
+};
+
+// One pass over the matrix from `start`: the CM order (or the plain BFS order) into perm. Returns the nodes placed, or -1
+// for a matrix given up; *levels the index of the last level. sm.quit is set when the watchdog fired.
 template <class G>
-__device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, int32_t start, bool bfs,
+__device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, int32_t start, bool bfs, SoloGiveUp give,
                                              uint64_t deadline, int32_t* levels, uint32_t* steps) {
   constexpr int T = G::T;
   const int tid = threadIdx.x;
@@ -372,6 +378,10 @@ __device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, 
       if (tid == 0) sm.levstart[q.lev & 63] = q.head;
     }
     if (!marked) {
+      const uint32_t waits = q.tdp - q.hdp;
+      if (waits > give.level &&
+          (uint32_t)J.row_ptr[J.n] - q.hdp > (waits / 4u > q.hdp ? give.growing : give.spare))
+        return -1;
       solo_take<G>(J, sm, q);
       __syncthreads();
       q.np = wave_uniform(sm.np);
@@ -416,11 +426,11 @@ struct SearchPasses {
 };
 
 // One matrix: the start search (SOLO_SEARCH), the order from `start` (SOLO_RUN), or both (SOLO_ORDER; `start` >= 0
-// skips the search). From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is first run as a CM pass: when its
+// skips the search), or ERR_CAPACITY when it is given up. From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is first run as a CM pass: when its
 // eccentricity equals the previous sweep's it is the confirming sweep and the result. The results go to *ctl.
 template <class G>
 __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, int32_t mode, int32_t start,
-                                            int32_t speculate, SoloClock& clk, Control* ctl) {
+                                            int32_t speculate, SoloGiveUp give, SoloClock& clk, Control* ctl) {
   const int tid = threadIdx.x, ln = lane_id();
   for (int i = tid; i < G::S; i += G::T) sm.tab[i] = kNoSlot;
   for (int i = tid; i < G::S; i += G::T) sm.mark[i] = 0;
@@ -446,7 +456,8 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && mode == SOLO_ORDER && speculate > 0 && iters >= speculate;
     if (passes > 0 && tid == 0) pass_beat(clk.beat, clk.t0);
-    placed = solo_pass<G>(J, sm, cur, searching && !attempt, min(clk.deadline(), wall_ticks() + clk.budget), &lev, &steps);
+    placed = solo_pass<G>(J, sm, cur, searching && !attempt, give, min(clk.deadline(), wall_ticks() + clk.budget), &lev,
+                          &steps);
     ++passes;
     expired = sm.quit != 0;
     if (placed != n || expired || !searching) break;
@@ -478,9 +489,9 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
     cur = sm.cur;
   }
   if (tid == 0) {
-    ctl->placed = (uint32_t)placed;
+    ctl->placed = (uint32_t)max(placed, 0);
     ctl->nbatches = steps ? steps : 1u;
-    ctl->error = expired ? ERR_TIMEOUT : ERR_NONE;
+    ctl->error = expired ? ERR_TIMEOUT : placed < 0 ? ERR_CAPACITY : ERR_NONE;
     ctl->start = cur;
     ctl->sweeps = iters;
     ctl->passes = passes;
@@ -493,11 +504,11 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
 // One matrix in one launch.
 template <class G>
 __global__ __launch_bounds__(G::T) void k_solo(SoloJob J, int32_t mode, int32_t start, int32_t speculate,
-                                               uint64_t budget_ticks, uint32_t* beat, Control* ctl) {
+                                               SoloGiveUp give, uint64_t budget_ticks, uint32_t* beat, Control* ctl) {
   using SM = SoloSmem<G>;
   RCM_LDS(SM, sm);
   SoloClock clk{wall_ticks(), budget_ticks, beat, 1u};
-  solo_matrix<G>(J, sm, mode, start, speculate, clk, ctl);
+  solo_matrix<G>(J, sm, mode, start, speculate, give, clk, ctl);
 }
 
 // Many matrices: workgroups take the jobs of the list in its order (largest first). A workgroup past the watchdog
@@ -511,6 +522,7 @@ struct SoloManyArgs {
   int32_t count;
   int32_t mode;
   int32_t speculate;
+  SoloGiveUp give;
   uint64_t budget_ticks;
   uint32_t* beat;
 };
@@ -534,7 +546,7 @@ __global__ __launch_bounds__(G::T) void k_solo_many(SoloManyArgs m) {
     if (j < 0) break;
     const JobDesc& D = m.jobs[j];
     const SoloJob J{D.row_ptr, D.col_idx, D.perm, D.qinfo, D.n};
-    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, clk, D.ctl);  // ends with a barrier
+    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, m.give, clk, D.ctl);  // ends with a barrier
   }
 }
 

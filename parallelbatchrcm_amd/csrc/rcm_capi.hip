@@ -112,6 +112,22 @@ bool solo_fits(int32_t n, uint32_t maxrow, int64_t total, int32_t alone) {
          maxrow <= (uint32_t)kSoloMaxRow;
 }
 
+// Levels of long rows, or of a random graph, outgrow one workgroup however few rows there are: it gives such a matrix up when
+// more than kSoloWide slots wait (7-point stencils and geometric graphs within the limits above stay below), unless what is
+// left, 1.3 us per 1000 entries, costs less than another engine's start, or a set's other entries would keep the batch
+// engine busy for longer: it takes 10 a ns of 27-point stencils, 25 of random graphs, whose levels grow tenfold. MI355X, us
+// an order by the batch engine alone, by one workgroup to its end, and as now: in a context, a 27-point stencil of 30^3
+// rows 450, 911, 223, a random graph of 30k rows of 31 entries 163, 1214, 118; in a set, one 27-point stencil of 40^3 rows
+// 767, 2345, 747, 20 of them 3263, 2379, 2401; a random graph of 60k rows 254, 2472, 219.
+constexpr uint32_t kSoloWide = 24576;
+constexpr int64_t kSoloSpare = 1 << 17;
+SoloGiveUp solo_give_up(int64_t total_nnz) {
+  const auto spare = [&](int64_t share) {
+    return (uint32_t)std::min<int64_t>(std::max<int64_t>(kSoloSpare, total_nnz / share), UINT32_MAX);
+  };
+  return SoloGiveUp{kSoloWide, spare(12), spare(32)};
+}
+
 // Whether a row holds so large a part of the matrix that its levels are few and wide: R-MAT graphs of 2^13 to 2^20 rows have
 // one of n / 27 entries or more.
 bool has_hub(int32_t n, uint32_t maxrow) { return maxrow > (uint32_t)kSoloMaxRow && (int64_t)maxrow * 32 >= n; }
@@ -370,6 +386,7 @@ struct rcm_ctx {
   int32_t team_cap = 0;
   uint32_t team_tag = 0;
   bool team_off = false;
+  bool solo_off = false;  // one workgroup gave the loaded matrix up: a team's
   // last result
   bool have_perm = false;
   bool reversed = false;
@@ -506,7 +523,7 @@ bool ctx_quick(const rcm_ctx* c) {
 int32_t sweep_number(int64_t speculate) { return (int32_t)std::min<int64_t>(speculate, INT32_MAX); }
 
 // Whether that is a team.
-bool ctx_team(const rcm_ctx* c) { return ctx_quick(c) && c->n > kCtxSolo; }
+bool ctx_team(const rcm_ctx* c) { return ctx_quick(c) && (c->n > kCtxSolo || c->solo_off); }
 
 // One launch of the level engine on the loaded matrix; the start used, sweeps and passes are in *c->h_ctl. False when
 // it takes the matrix no further (ctx_quick, no memory for a team, a stage region too small): the batch engine's.
@@ -549,7 +566,7 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
       const SoloJob J{c->rp, c->ci, c->perm, c->qinfo, c->n};
       // the result goes to pinned host memory as the kernel ends: no copy after it
       hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, c->stream, J, mode, start, sweep_number(c->speculate),
-                         budget, c->h_beat, c->h_ctl);
+                         solo_give_up(0), budget, c->h_beat, c->h_ctl);
     }
     RCM_HIP(hipGetLastError());
     RCM_HIP(hipEventRecord(c->ev[2], c->stream));
@@ -577,6 +594,10 @@ bool ctx_run_quick(rcm_ctx* c, int32_t mode, int32_t start, int* rc) {
     return RCM_OK;
   }();
   if (*rc != RCM_ECAPACITY) return true;
+  if (!team) {
+    c->solo_off = true;
+    return ctx_run_quick(c, mode, start, rc);
+  }
   c->team_off = true;
   return false;
 }
@@ -732,6 +753,7 @@ int load_common(rcm_ctx* c, int32_t n, int64_t nnz) {
   if (h[0] != 0) return RCM_EINVAL;
   c->maxdeg = h[1];
   c->team_off = false;
+  c->solo_off = false;
   c->n = n;
   c->nnz = nnz;
   c->have_perm = false;
@@ -790,6 +812,7 @@ struct rcm_batch {
   std::vector<int32_t> solo, rest;
   int32_t *d_solo = nullptr, *d_rest = nullptr, *blk_rest = nullptr;
   std::vector<int32_t> blk_rest_h;
+  std::vector<uint8_t> wide;  // one workgroup gave the matrix up
   int64_t rest_rows = 0;
   uint32_t* solo_next = nullptr;
   int solo_resident = 0;  // co-resident workgroups of the one-workgroup engine
@@ -965,14 +988,14 @@ bool batch_solo(const rcm_batch* b) {
 
 // Whether a set gains from its split. The engines run one after the other, and a matrix of the rest with many levels keeps
 // the batch engine busy for as long as its levels take, with the others or without: only beside kSoloShare times its rows,
-// or with a hub row (few levels), does the rest end early enough. MI355X, ms a run by the batch engine alone and by both:
+// or with few levels (a hub row, or given up by one workgroup), does the rest end early enough. MI355X, ms a run by the batch engine alone and by both:
 // 5, 30 and 60 matrices of up to 60k rows beside a 2D stencil of 152k rows 6.7 / 7.3, 6.8 / 7.9, 6.9 / 8.0; beside a
 // geometric graph of 150k 3.86 / 4.50, 3.86 / 4.96, 3.92 / 5.06; beside an R-MAT graph of 2^16 rows 1.27 / 1.09, 3.42 /
 // 1.58, 3.87 / 1.61, of 2^13 rows 1.27 / 0.87, 3.40 / 1.36, 3.83 / 1.42.
 bool solo_pays(const rcm_batch* b) {
   const int64_t company = (b->total_n - b->rest_rows) / kSoloShare;
   for (int32_t k : b->rest)
-    if (b->n[k] > company && !has_hub(b->n[k], b->maxrow[k])) return false;
+    if (b->n[k] > company && !has_hub(b->n[k], b->maxrow[k]) && !b->wide[k]) return false;
   return true;
 }
 
@@ -988,6 +1011,7 @@ void enqueue_solo(rcm_batch* b, int32_t mode) {
   m.speculate = sweep_number(b->speculate);
   m.budget_ticks = (uint64_t)b->timeout_ms * 100000ull;
   m.beat = b->h_beat;
+  m.give = solo_give_up(b->total_nnz);
   const int grid = std::max(1, std::min(m.count, b->workers > 0 ? std::min((int)b->workers, b->solo_resident)
                                                                 : b->solo_resident));
   hipLaunchKernelGGL(k_solo_reset, dim3(1), dim3(64), 0, b->stream, m.next);
@@ -2003,6 +2027,54 @@ int rcm_batch_set_param(rcm_batch* b, int param, int64_t v) {
   }
 }
 
+// Splits the loaded set by engine, and its lists to the device.
+static int batch_split(rcm_batch* b) {
+  b->solo.clear();
+  b->rest.clear();
+  b->rest_rows = 0;
+  for (int32_t k : b->order) {
+    if (solo_fits(b->n[k], b->maxrow[k], b->total_n, b->lane ? kSoloLane : kSoloAlone) && !b->wide[k]) {
+      b->solo.push_back(k);
+    } else {
+      b->rest.push_back(k);
+      b->rest_rows += b->n[k];
+    }
+  }
+  if (!b->lane && !solo_pays(b)) {
+    b->solo.clear();
+    b->rest = b->order;
+    b->rest_rows = b->total_n;
+  }
+  (void)build_blk(b, b->rest.data(), (int32_t)b->rest.size(), b->blk_rest_h);
+  if (!b->solo.empty())
+    RCM_HIP(hipMemcpyAsync(b->d_solo, b->solo.data(), b->solo.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                           b->stream));
+  if (!b->rest.empty()) {
+    RCM_HIP(hipMemcpyAsync(b->d_rest, b->rest.data(), b->rest.size() * sizeof(int32_t), hipMemcpyHostToDevice,
+                           b->stream));
+    RCM_HIP(hipMemcpyAsync(b->blk_rest, b->blk_rest_h.data(), b->blk_rest_h.size() * sizeof(int32_t),
+                           hipMemcpyHostToDevice, b->stream));
+  }
+  RCM_HIP(hipStreamSynchronize(b->stream));
+  return RCM_OK;
+}
+
+// The matrices that the one-workgroup engine has given up are the batch engine's from here on: split again, their status
+// (RCM_ECAPACITY) taken back. `gave`, if there, receives them.
+static int batch_take_back(rcm_batch* b, int32_t* status, std::vector<int32_t>* gave) {
+  bool any = false;
+  for (int32_t k : b->solo)
+    if (status[k] == RCM_ECAPACITY) {
+      any = true;
+      b->wide[k] = 1;
+      status[k] = RCM_OK;
+      if (gave) gave->push_back(k);
+    }
+  if (!any) return RCM_OK;
+  batch_drop_graphs(b);
+  return batch_split(b);
+}
+
 int rcm_batch_load(rcm_batch* b, int32_t count, const int32_t* n, const int64_t* nnz, const int64_t* rp_off,
                    const int64_t* ci_off, const int32_t* row_ptr_cat, const int32_t* col_idx_cat, int32_t* status_out) {
   if (!b || count < 1 || !n || !nnz || !rp_off || !ci_off || !row_ptr_cat || !col_idx_cat) return RCM_EINVAL;
@@ -2120,31 +2192,8 @@ int rcm_batch_load(rcm_batch* b, int32_t count, const int32_t* n, const int64_t*
     batch_reset(b);
     return rc;
   }
-  b->rest_rows = 0;
-  for (int32_t k : b->order) {
-    if (solo_fits(n[k], b->maxrow[k], tot, b->lane ? kSoloLane : kSoloAlone)) {
-      b->solo.push_back(k);
-    } else {
-      b->rest.push_back(k);
-      b->rest_rows += n[k];
-    }
-  }
-  if (!b->lane && !solo_pays(b)) {
-    b->solo.clear();
-    b->rest = b->order;
-    b->rest_rows = tot;
-  }
-  (void)build_blk(b, b->rest.data(), (int32_t)b->rest.size(), b->blk_rest_h);
-  if (!b->solo.empty())
-    RCM_HIP(hipMemcpyAsync(b->d_solo, b->solo.data(), b->solo.size() * sizeof(int32_t), hipMemcpyHostToDevice,
-                           b->stream));
-  if (!b->rest.empty()) {
-    RCM_HIP(hipMemcpyAsync(b->d_rest, b->rest.data(), b->rest.size() * sizeof(int32_t), hipMemcpyHostToDevice,
-                           b->stream));
-    RCM_HIP(hipMemcpyAsync(b->blk_rest, b->blk_rest_h.data(), b->blk_rest_h.size() * sizeof(int32_t),
-                           hipMemcpyHostToDevice, b->stream));
-  }
-  RCM_HIP(hipStreamSynchronize(b->stream));
+  b->wide.assign(C, 0);
+  if (const int sp = batch_split(b)) return sp;
   b->timing.load_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return RCM_OK;
 }
@@ -2165,10 +2214,11 @@ int batch_solo_pass(rcm_batch* b, int32_t mode, const std::vector<int32_t>& give
   if (wr) return wr;
   *b->h_g = ManyControl{};  // the batch engine's abort word: not this launch's
   (void)collect_status(b, b->solo.data(), (int32_t)b->solo.size(), status, nullptr);
-  for (int32_t k : b->solo) {
-    cur[k] = b->h_ctl[k].start;
-    iters[k] = b->h_ctl[k].sweeps;
-  }
+  for (int32_t k : b->solo)
+    if (status[k] != RCM_ECAPACITY) {
+      cur[k] = b->h_ctl[k].start;
+      iters[k] = b->h_ctl[k].sweeps;
+    }
   return RCM_OK;
 }
 
@@ -2213,13 +2263,16 @@ int rcm_batch_find_start(rcm_batch* b, int32_t* start_out, int32_t* iterations_o
   std::vector<uint32_t> lastdist(C, 0);
   int sweeps = 0;
   const bool solo = batch_solo(b);
+  std::vector<int32_t> gave, todo = solo ? b->rest : b->order;
   if (solo) {
     ++sweeps;
     const int r = batch_solo_pass(b, SOLO_SEARCH, std::vector<int32_t>((size_t)C, -1), cur.data(), iters.data(),
                                   status.data());
     if (r) return r;
+    if (const int t = batch_take_back(b, status.data(), &gave)) return t;
   }
-  for (int32_t k : solo ? b->rest : b->order) {
+  todo.insert(todo.end(), gave.begin(), gave.end());
+  for (int32_t k : todo) {
     if (b->n[k] == 1) {
       cur[k] = 0;
       iters[k] = 1;
@@ -2295,7 +2348,9 @@ int rcm_batch_order(rcm_batch* b, const int32_t* start_in, uint32_t flags, int32
     ++launches;
     const int r = batch_solo_pass(b, SOLO_ORDER, given, cur.data(), iters.data(), status.data());
     if (r) return r;
-    for (int32_t k : b->solo) need[k] = kDone;
+    for (int32_t k : b->solo)
+      if (status[k] != RCM_ECAPACITY) need[k] = kDone;
+    if (const int t = batch_take_back(b, status.data(), nullptr)) return t;
   }
   std::vector<int32_t> plain, cm;
   for (;;) {
@@ -2413,7 +2468,26 @@ int rcm_batch_run(rcm_batch* b, const int32_t* start, uint32_t flags, int32_t* s
   if (solo && b->rest.empty()) *b->h_g = ManyControl{};  // the batch engine did not run: no abort word of its own
   int64_t nb = 0;
   std::vector<int32_t> st((size_t)C, RCM_OK);
-  const int rc = collect_status(b, b->order.data(), C, st.data(), &nb);
+  (void)collect_status(b, b->order.data(), C, st.data(), &nb);
+  std::vector<int32_t> gave;
+  if (solo)
+    if (const int t = batch_take_back(b, st.data(), &gave)) return t;
+  if (!gave.empty()) {  // this once; the next run has them in its one launch
+    const int r = batch_pass(b, gave, std::vector<int32_t>(start, start + C), false, false, st.data());
+    if (r) return r;
+    for (int32_t k : gave) nb += b->h_ctl[k].nbatches;
+    if (rev)
+      hipLaunchKernelGGL(k_reverse_many, dim3((unsigned)b->nblk_order), dim3(256), 0, b->stream, b->jobs, b->d_order,
+                         C, b->blk_order);
+    RCM_HIP(hipEventRecord(b->ev[1], b->stream));
+    RCM_HIP(hipStreamSynchronize(b->stream));
+    RCM_HIP(hipEventElapsedTime(&ms, b->ev[0], b->ev[1]));
+    b->timing.run_ms = ms;
+    b->timing.workers = batch_workers(b);
+  }
+  int rc = RCM_OK;
+  for (int32_t k : b->order)
+    if (st[k] != RCM_OK && rc == RCM_OK) rc = st[k];
   if (status_out) std::copy(st.begin(), st.end(), status_out);
   b->ok_jobs.clear();  // matrices with a complete order (the bandwidth reads only these)
   for (int32_t k : b->order)
@@ -2989,18 +3063,20 @@ int rcm_gpu_batch_noalloc(int32_t n, int64_t nnz, const int32_t* d_row_ptr, cons
   a.claim_filter = kDefaultClaimFilter;
 
   int32_t start = start_node;
-  const bool solo = solo_fits(n, vflags[1], n, kSoloNoAlloc);
+  bool solo = solo_fits(n, vflags[1], n, kSoloNoAlloc);
   if (solo) {  // start search and order in one launch of one workgroup
     const SoloJob J{d_row_ptr, d_col_idx, d_perm_out, a.qinfo, n};
     hipLaunchKernelGGL(k_solo<SoloG>, dim3(1), dim3(SoloG::T), 0, nullptr, J, (int32_t)SOLO_ORDER, start,
-                       (int32_t)kDefaultSpeculate, a.budget_ticks, nullptr, a.ctl);
+                       (int32_t)kDefaultSpeculate, solo_give_up(0), a.budget_ticks, nullptr, a.ctl);
     RCM_HIP(hipGetLastError());
     Control h{};
     RCM_HIP(hipMemcpy(&h, a.ctl, sizeof(Control), hipMemcpyDeviceToHost));
     if (h.error == ERR_TIMEOUT) return RCM_ETIMEOUT;
-    if ((int32_t)h.placed != n) return RCM_ENOTCONNECTED;
-    start = h.start;
-  } else if (start < 0) {  // SimplePeripheral::findPeripheral (src/simple_peripheral.cpp:92-141)
+    solo = h.error == ERR_NONE;
+    if (solo && (int32_t)h.placed != n) return RCM_ENOTCONNECTED;
+    if (solo) start = h.start;
+  }
+  if (!solo && start < 0) {  // SimplePeripheral::findPeripheral (src/simple_peripheral.cpp:92-141)
     int32_t* level = reinterpret_cast<int32_t*>(base + L.level);
     start = n / 2;
     if (n == 1) {

@@ -25,8 +25,8 @@ using namespace rcm;
 namespace {
 template <class G>
 int run(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* ci_off, const int32_t* rpc,
-        const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate, int32_t* perm_cat,
-        int32_t* info, double timeout_s) {
+        const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate, SoloGiveUp give,
+        int32_t* perm_cat, int32_t* info, double timeout_s) {
   int64_t tot = 0;
   for (int k = 0; k < count; ++k) tot += n[k];
   std::vector<int32_t> perm(tot, -1);
@@ -59,6 +59,7 @@ int run(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* c
   m.count = count;
   m.mode = mode;
   m.speculate = speculate;
+  m.give = give;
   m.budget_ticks = (uint64_t)(timeout_s * 1e8);
   emu::launch(1, 64, false, k_solo_reset, &next);
   emu::emu_lds_bytes = sizeof(SoloSmem<G>);
@@ -119,15 +120,17 @@ int team(int32_t n, const int32_t* rp, const int32_t* ci, int32_t start, int32_t
 extern "C" {
 // Orders `count` concatenated matrices, one workgroup each. geo: 0 = the geometry of small chunks (128 threads, 256
 // slots, a ring of 64 entries: chunks, their remainders and the ring's overflow at small sizes), 1 = the library's.
-// perm_cat: matrix k's order at sum_{i<k} n[i]; info[6 k ..] = error, placed, steps, start, sweeps, passes.
+// wide_level, spare: when a matrix is given up. perm_cat: matrix k's order at sum_{i<k} n[i]; info[6 k ..] = error, placed,
+// steps, start, sweeps, passes.
 int emu_run_solo(int32_t count, const int32_t* n, const int64_t* rp_off, const int64_t* ci_off, const int32_t* rpc,
                  const int32_t* cic, const int32_t* start, int32_t workers, int32_t mode, int32_t speculate,
-                 int32_t geo, int32_t* perm_cat, int32_t* info, double timeout_s) {
+                 int32_t geo, uint32_t wide_level, uint32_t spare, int32_t* perm_cat, int32_t* info, double timeout_s) {
   if (count <= 0 || workers <= 0) return -1;
+  const SoloGiveUp give{wide_level, spare, spare};
   return geo ? run<SoloGeo<1024, 4096, kSoloMaxN>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode, speculate,
-                                                 perm_cat, info, timeout_s)
+                                                 give, perm_cat, info, timeout_s)
              : run<SoloGeo<128, 256, 1 << 16, 64>>(count, n, rp_off, ci_off, rpc, cic, start, workers, mode,
-                                                   speculate, perm_cat, info, timeout_s);
+                                                   speculate, give, perm_cat, info, timeout_s);
 }
 
 void emu_team_linger(int where, int member, int phase) {

@@ -204,16 +204,16 @@ def run_wg(mats, starts, workers=3, bfs=False):
     return rc, [perm[off[k]:off[k + 1]] for k in range(len(mats))], [lev[off[k]:off[k + 1]] for k in range(len(mats))], info
 
 
-def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.0):
+def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.0, give_up=(2**32 - 1, 2**32 - 1)):
     """One workgroup per matrix (engine_solo.hpp). mats: list of (rp, ci); mode 0 = order from starts[k], 1 = start
     search, 2 = start search (where starts[k] < 0) and order. Returns ([perm], info[count, 6]) with info = error,
-    placed, steps, start, sweeps, passes."""
+    placed, steps, start, sweeps, passes. give_up: a level's slots, and entries left, from which a matrix is given up."""
     L = lib("solo")
     if not hasattr(L, "_solo_ready"):
         I64P = C.POINTER(C.c_int64)
         L.emu_run_solo.restype = C.c_int
         L.emu_run_solo.argtypes = [C.c_int32, I32P, I64P, I64P, I32P, I32P, I32P, C.c_int32, C.c_int32, C.c_int32,
-                                   C.c_int32, I32P, I32P, C.c_double]
+                                   C.c_int32, C.c_uint32, C.c_uint32, I32P, I32P, C.c_double]
         L._solo_ready = True
     n = np.array([len(rp) - 1 for rp, _ in mats], np.int32)
     rp_off = np.concatenate([[0], np.cumsum([len(rp) for rp, _ in mats])[:-1]]).astype(np.int64)
@@ -226,7 +226,7 @@ def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.
     I64 = C.POINTER(C.c_int64)
     rc = L.emu_run_solo(len(mats), n.ctypes.data_as(I32P), rp_off.ctypes.data_as(I64), ci_off.ctypes.data_as(I64),
                         rpc.ctypes.data_as(I32P), cic.ctypes.data_as(I32P), st.ctypes.data_as(I32P), workers, mode,
-                        speculate, geo, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
+                        speculate, geo, *give_up, perm.ctypes.data_as(I32P), info.ctypes.data_as(I32P), timeout_s)
     assert rc == 0, "emulator rejected the arguments"
     off = np.concatenate([[0], np.cumsum(n)])
     return [perm[off[k]:off[k + 1]] for k in range(len(mats))], info

@@ -95,6 +95,24 @@ def test_emulated_watchdog():
     assert (info[:, 0] == 1).all()
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_emulated_give_up(mode):
+    """A matrix is given up at a level too wide with too much left, in whatever pass; the others of the launch are not."""
+    pytest.importorskip("emu_lib")
+    import emu_lib as E
+
+    mats = [CASES["random1500"](), CASES["path300"](), CASES["star64"]()]
+    nnz = [len(ci) for _, ci in mats]
+    for level, spare, gave in ((2000, 1000, [True, False, False]), (2000, nnz[0], [False] * 3), (300, 60, [True, False, False])):
+        perms, info = E.run_solo(mats, [0] * 3 if mode == 0 else [-1] * 3, workers=2, mode=mode, give_up=(level, spare))
+        assert (info[:, 0] == 2).tolist() == gave, (level, spare)
+        for k, (rp, ci) in enumerate(mats):
+            if not gave[k]:
+                s = 0 if mode == 0 else O.peripheral(rp, ci)[1]
+                assert info[k, 0] == 0 and info[k, 3] == s, k
+                assert mode == 1 or np.array_equal(perms[k], O.cm(rp, ci, s)), k
+
+
 # unsymmetric: the sweeps from nodes 2 and 3 find eccentricities 1 and 2 in turn, and no start is ever confirmed
 ENDLESS = (np.array([0, 3, 6, 9, 12], np.int32), np.array([1, 2, 3, 1, 2, 3, 0, 1, 3, 0, 1, 3], np.int32))
 
@@ -248,6 +266,73 @@ def test_gpu_set_split(name):
                     assert np.array_equal(p, want[k][2][::-1] if flags == P.RCM_FLAG_REVERSE else want[k][2]), (rep, k)
         assert b.timing().graph_replays >= 4
         assert b.timing().workers == workgroups if workgroups else b.timing().workers > len(mats)
+
+
+def _box27(a, b, c):
+    """The 27-point stencil on a x b x c nodes, relabelled."""
+    at = np.stack(np.meshgrid(np.arange(a), np.arange(b), np.arange(c), indexing="ij"), -1).reshape(-1, 3)
+    off = np.stack(np.meshgrid(*[np.arange(-1, 2)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    to = at[:, None] + off[None]
+    inside = ((to >= 0) & (to < (a, b, c))).all(-1)
+    rp = np.concatenate([[0], np.cumsum(inside.sum(1))]).astype(np.int32)
+    m, _ = P.workloads.permute_symmetric(P.CSR(rp, ((to[..., 0] * b + to[..., 1]) * c + to[..., 2])[inside].astype(np.int32)), 3)
+    return m.row_offsets, m.col_ids
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["random", "box27", "bar27"])
+def test_gpu_wide_levels(name):
+    """Matrices that one workgroup gives up (levels of a random graph, of a 27-point stencil) and one that it does not (the
+    same stencil on a bar), alone, in a set with others, in one call, and in a serving lane."""
+    from hip_buffers import HipBuffers
+    from test_zz_no_alloc import _noalloc
+
+    rp, ci = {"random": lambda: G.random_connected(20000, 300000, seed=3), "box27": lambda: _box27(30, 30, 30),
+              "bar27": lambda: _box27(8, 8, 400)}[name]()
+    m = P.CSR(rp, ci)
+    _, s, it, _ = O.peripheral(rp, ci)
+    want = O.cm(rp, ci, s)
+    wide = name != "bar27"
+    print("[case]", name, m.rows, m.nnz, flush=True)
+    with P.RcmContext(timeout_ms=20000) as c:
+        c.load(m)
+        assert c.order() == (s, it) and np.array_equal(c.perm(), want)
+        c.run(s, P.RCM_FLAG_REVERSE)
+        assert np.array_equal(c.perm(), want[::-1]) and c.timing().workers == (128 if wide else 1)
+        assert c.find_start() == s
+        c.load(m)  # a new matrix: one workgroup is tried again
+        c.run(s)
+        assert np.array_equal(c.perm(), want)
+    others = [P.CSR(*CASES["grid24x20"]()), P.CSR(*CASES["path300"]())]
+    mats = [others[0], m, others[1]]
+    starts = [O.peripheral(x.row_offsets, x.col_ids)[1] for x in mats]
+    orders = [O.cm(x.row_offsets, x.col_ids, k) for x, k in zip(mats, starts)]
+    for first in ("run", "reverse", "order", "find"):
+        with P.RcmBatch(timeout_ms=20000, graph=True) as b:
+            b.load(P.BatchSet.from_matrices(mats))
+            for rep in range(3):
+                if first == "order":
+                    got, iters, st = b.order()
+                    assert not st.any() and got.tolist() == starts and iters[1] == it
+                elif first == "find":
+                    got, iters, st = b.find_start()
+                    assert not st.any() and got.tolist() == starts and iters[1] == it
+                    assert not b.run(got).any()
+                else:
+                    assert not b.run(starts, P.RCM_FLAG_REVERSE if first == "reverse" else P.RCM_FLAG_STABLE).any()
+                for k, p in enumerate(b.perms()):
+                    assert np.array_equal(p, orders[k][::-1] if first == "reverse" else orders[k]), (first, rep, k)
+            assert not b.run(starts).any() and (b.timing().workers > 3) == wide
+    perm, bw, used = P.rcm_gpu_batch(m, -1, P.RCM_FLAG_BANDWIDTH)
+    assert used == s and np.array_equal(perm, want) and bw == O.bandwidth(rp, ci, want)
+    with HipBuffers() as hip:
+        rc, perm, bw, used = _noalloc(hip, m, -1, P.RCM_FLAG_BANDWIDTH)
+        assert rc == 0 and used == s and np.array_equal(perm, want) and bw == O.bandwidth(rp, ci, want)
+    with P.RcmServer(lanes=2, arena_bytes=1 << 28) as srv:
+        jobs = [srv.submit(x) for x in mats]
+        for j, o in zip(jobs, orders):
+            rc, perm, _ = srv.wait(j)
+            assert rc == 0 and np.array_equal(perm, o)
 
 
 @pytest.mark.gpu
