@@ -577,15 +577,18 @@ __device__ __forceinline__ bool team_place(const TeamArgs& a, TeamSmem<G>& sm, c
   // Readers of a redistribution's children look at their tags, so its word goes out first. A part without children, though,
   // may be of the pass's last level: then the leader reads the queue as soon as it has the members' words, with no meeting
   // before, and the word waits for the part's queue entries (of all its chunks).
-  const bool word = last && nx.split, barren = nx.placed + cnt == 0;
-  if (wv == 0 && word && !barren) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), nx.placed + cnt);
-  RCM_TEAM_LINGER(3, sm.g, lv.tag);
-  if (tid < np) st_sync(&a.perm[q0 + tid], (int32_t)sm.node[tid]);
-  if (word && barren) {
+  const bool word = last && nx.split, barren = word && nx.placed + cnt == 0;
+  const auto store_queue = [&]() {
+    RCM_TEAM_LINGER(3, sm.g, lv.tag);
+    if (tid < np) st_sync(&a.perm[q0 + tid], (int32_t)sm.node[tid]);
+  };
+  if (barren) {
+    store_queue();
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (wv == 0) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), 0u);
   }
+  if (wv == 0 && word) team_publish<G>(a, sm, lv, width, team_wanted(a, share, here), nx.placed + cnt);
+  if (!barren) store_queue();
   if (active) {
     const uint32_t xc = ic - vc, xd = id - vd;
 #pragma unroll
