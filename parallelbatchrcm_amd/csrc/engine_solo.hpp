@@ -44,6 +44,40 @@ struct SoloGeo {
   static_assert(S >= kSoloMaxRow && S <= 65536, "any one parent fits a chunk");
 };
 
+// Which passes of a search the watchdog counts. In a symmetric matrix every sweep is longer than the one before or confirms
+// it; in others the sweeps may repeat for ever, so one that does neither moves the deadline no further.
+struct SearchPasses {
+  uint32_t count, longest;  // 1 and 0 at first
+  __device__ __forceinline__ void sweep(uint32_t lev, bool attempt) {  // the sweep after it is due, and an attempt's repeat
+    if (lev <= longest) return;
+    longest = lev;
+    count += attempt ? 2u : 1u;
+  }
+};
+
+// The watchdog of a workgroup, kept by thread 0. Its budget is for one pass over each matrix, as where every sweep is a
+// launch of its own: a pass is to end within one budget, and the pass numbered p (from 1) of any matrix within p budgets of
+// the launch.
+struct SoloClock {
+  uint64_t t0, budget, deadline;
+  uint32_t* beat;      // pinned, or null: changes as passes begin, so that the host does not give a long search up
+  uint32_t most;       // the largest p yet
+  SearchPasses due;
+  __device__ __forceinline__ void begin(uint64_t ticks, uint32_t* b) {
+    t0 = wall_ticks();
+    budget = ticks;
+    deadline = t0 + ticks;
+    beat = b;
+    most = 1u;
+  }
+  __device__ __forceinline__ bool pass() {  // before one: whether it is too late for it
+    most = max(most, due.count);
+    const uint64_t now = wall_ticks(), end = t0 + budget * most;
+    deadline = min(end, now + budget);
+    return now > end;
+  }
+};
+
 template <class G>
 struct SoloSmem {
   uint32_t tab[G::S];            // hash: the smallest slot claiming a child, kNoSlot when free
@@ -60,6 +94,7 @@ struct SoloSmem {
   int32_t levstart[64];          // first queue position of the last 64 levels
   uint32_t np, E, quit;          // of the chunk: parents, slots; the watchdog fired in the pass
   uint32_t late;                 // it fired between two passes
+  SoloClock clk;
   int32_t job, cur;
 };
 constexpr uint32_t kNoSlot = ~0u;
@@ -353,7 +388,7 @@ struct SoloGiveUp {
 // for a matrix given up; *levels the index of the last level. sm.quit is set when the watchdog fired.
 template <class G>
 __device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, int32_t start, bool bfs, SoloGiveUp give,
-                                             uint64_t deadline, int32_t* levels, uint32_t* steps) {
+                                             int32_t* levels, uint32_t* steps) {
   constexpr int T = G::T;
   const int tid = threadIdx.x;
   for (int32_t i = tid; i < (J.n + 31) / 32; i += T) sm.vis[i] = 0u;
@@ -388,7 +423,7 @@ __device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, 
       q.E = wave_uniform(sm.E);
     }
     if ((++step & 63u) == 0u) {
-      if (tid == 0) sm.quit = wall_ticks() > deadline ? 1u : 0u;
+      if (tid == 0) sm.quit = wall_ticks() > sm.clk.deadline ? 1u : 0u;
       __syncthreads();
       if (sm.quit) break;
     }
@@ -399,14 +434,6 @@ __device__ __forceinline__ int32_t solo_pass(const SoloJob& J, SoloSmem<G>& sm, 
   return q.tail;
 }
 
-// The watchdog of a workgroup. Its budget is for one pass over each matrix, as where every sweep is a launch of its own: a
-// pass is to end within one budget, and the pass numbered p (from 1) of any matrix within p budgets of the launch.
-struct SoloClock {
-  uint64_t t0, budget;
-  uint32_t* beat;  // pinned, or null: changes as passes begin, so that the host does not give a long search up
-  uint32_t due;    // the largest p yet
-  __device__ __forceinline__ uint64_t deadline() const { return t0 + budget * due; }
-};
 // One thread, as a pass after the first begins. The host allows 10 s beyond the budget; before 10 ms it need not know (the
 // store to its memory takes 3 us, of a pass over a 100 x 100 grid's 290).
 __device__ __forceinline__ void pass_beat(uint32_t* beat, uint64_t t0) {
@@ -414,23 +441,12 @@ __device__ __forceinline__ void pass_beat(uint32_t* beat, uint64_t t0) {
   if (beat && now - t0 > 1000000u) st_host(beat, (uint32_t)now);
 }
 
-// Which passes of a search the watchdog counts. In a symmetric matrix every sweep is longer than the one before or confirms
-// it; in others the sweeps may repeat for ever, so one that does neither moves the deadline no further.
-struct SearchPasses {
-  uint32_t count, longest;  // 1 and 0 at first
-  __device__ __forceinline__ void sweep(uint32_t lev, bool attempt) {  // the sweep after it is due, and an attempt's repeat
-    if (lev <= longest) return;
-    longest = lev;
-    count += attempt ? 2u : 1u;
-  }
-};
-
 // One matrix: the start search (SOLO_SEARCH), the order from `start` (SOLO_RUN), or both (SOLO_ORDER; `start` >= 0
 // skips the search), or ERR_CAPACITY when it is given up. From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is first run as a CM pass: when its
 // eccentricity equals the previous sweep's it is the confirming sweep and the result. The results go to *ctl.
 template <class G>
 __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, int32_t mode, int32_t start,
-                                            int32_t speculate, SoloGiveUp give, SoloClock& clk, Control* ctl) {
+                                            int32_t speculate, SoloGiveUp give, Control* ctl) {
   const int tid = threadIdx.x, ln = lane_id();
   for (int i = tid; i < G::S; i += G::T) sm.tab[i] = kNoSlot;
   for (int i = tid; i < G::S; i += G::T) sm.mark[i] = 0;
@@ -440,34 +456,29 @@ __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, i
   int32_t cur = start >= 0 ? start : n > 1 ? n / 2 : 0;
   int32_t iters = start < 0 && n == 1 ? 1 : 0, passes = 0, placed = n, lev = 0;
   uint32_t steps = 0, lastdist = 0;
-  SearchPasses due{1u, 0u};
-  bool expired = wall_ticks() > clk.deadline();  // thread 0's word counts, below
-  if (tid == 0) sm.quit = expired ? 1u : 0u;
-  __syncthreads();
-  expired = sm.quit != 0;
-  while (!expired && (searching || mode != SOLO_SEARCH)) {
-    clk.due = max(clk.due, due.count);
-    if (passes > 0) {  // a pass looks at the clock on every 64th step, and may have fewer
-      if (tid == 0) sm.late = wall_ticks() > clk.deadline() ? 1u : 0u;
-      __syncthreads();
-      expired = sm.late != 0;
-      if (expired) break;
+  bool expired = false;
+  if (tid == 0) sm.clk.due = SearchPasses{1u, 0u};
+  while (searching || mode != SOLO_SEARCH) {
+    if (tid == 0) {  // a pass looks at the clock on every 64th step, and may have fewer
+      sm.late = sm.clk.pass() ? 1u : 0u;
+      if (passes > 0) pass_beat(sm.clk.beat, sm.clk.t0);
     }
+    __syncthreads();
+    expired = sm.late != 0;
+    if (expired) break;
     if (searching && !redo) ++iters;
     const bool attempt = searching && !redo && mode == SOLO_ORDER && speculate > 0 && iters >= speculate;
-    if (passes > 0 && tid == 0) pass_beat(clk.beat, clk.t0);
-    placed = solo_pass<G>(J, sm, cur, searching && !attempt, give, min(clk.deadline(), wall_ticks() + clk.budget), &lev,
-                          &steps);
+    placed = solo_pass<G>(J, sm, cur, searching && !attempt, give, &lev, &steps);
     ++passes;
     expired = sm.quit != 0;
     if (placed != n || expired || !searching) break;
     if ((uint32_t)lev == lastdist) {  // cur is the start
       if (attempt || mode == SOLO_SEARCH) break;
       searching = false;
-      ++due.count;
+      if (tid == 0) ++sm.clk.due.count;
       continue;
     }
-    due.sweep((uint32_t)lev, attempt);
+    if (tid == 0) sm.clk.due.sweep((uint32_t)lev, attempt);
     redo = attempt;  // a failed attempt is followed by the plain sweep from the same start
     if (redo) continue;
     lastdist = (uint32_t)lev;
@@ -507,8 +518,8 @@ __global__ __launch_bounds__(G::T) void k_solo(SoloJob J, int32_t mode, int32_t 
                                                SoloGiveUp give, uint64_t budget_ticks, uint32_t* beat, Control* ctl) {
   using SM = SoloSmem<G>;
   RCM_LDS(SM, sm);
-  SoloClock clk{wall_ticks(), budget_ticks, beat, 1u};
-  solo_matrix<G>(J, sm, mode, start, speculate, give, clk, ctl);
+  if (threadIdx.x == 0) sm.clk.begin(budget_ticks, beat);
+  solo_matrix<G>(J, sm, mode, start, speculate, give, ctl);
 }
 
 // Many matrices: workgroups take the jobs of the list in its order (largest first). A workgroup past the watchdog
@@ -535,7 +546,7 @@ template <class G>
 __global__ __launch_bounds__(G::T) void k_solo_many(SoloManyArgs m) {
   using SM = SoloSmem<G>;
   RCM_LDS(SM, sm);
-  SoloClock clk{wall_ticks(), m.budget_ticks, m.beat, 1u};
+  if (threadIdx.x == 0) sm.clk.begin(m.budget_ticks, m.beat);
   for (;;) {
     if (threadIdx.x == 0) {
       const uint32_t x = atomic_add_u32(m.next, 1u);
@@ -546,7 +557,7 @@ __global__ __launch_bounds__(G::T) void k_solo_many(SoloManyArgs m) {
     if (j < 0) break;
     const JobDesc& D = m.jobs[j];
     const SoloJob J{D.row_ptr, D.col_idx, D.perm, D.qinfo, D.n};
-    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, m.give, clk, D.ctl);  // ends with a barrier
+    solo_matrix<G>(J, sm, m.mode, m.starts[j], m.speculate, m.give, D.ctl);  // ends with a barrier
   }
 }
 
