@@ -2871,7 +2871,9 @@ int rcm_ctx_autotune(rcm_ctx* c, int32_t start, int32_t repeats, rcm_tune_result
   c->variant = kDefaultCtxVariant;
   c->workers = 0;
   c->engine_set = false;
+  if (const int rc = timed()) return rc;  // once for nothing: first launches take longer
   if (const int rc = timed()) return rc;
+  count = 1;
   bool automatic = ctx_quick(c);
   best.default_ms = best.best_ms = median_of(t);
   best.variant = (int32_t)(automatic ? c->variant : ctx_variant(c));
@@ -2949,7 +2951,9 @@ int rcm_batch_autotune(rcm_batch* b, const int32_t* start, int32_t repeats, rcm_
   // the default: matrices that fit it by the one-workgroup engine
   rcm_batch_set_param(b, RCM_PARAM_VARIANT, kDefaultBatchVariant);
   rcm_batch_set_param(b, RCM_PARAM_WORKERS, 0);
+  if (const int rc = timed()) return rc;  // once for nothing: first launches take longer
   if (const int rc = timed()) return rc;
+  count = 1;
   bool automatic = batch_solo(b);
   best.default_ms = best.best_ms = median_of(t);
   best.variant = (int32_t)b->variant;
