@@ -19,6 +19,8 @@
 //   Order. The owned children are packed in slot order, so siblings are neighbours (one child per parent on average);
 //   each counts the earlier ones of larger and the later ones of smaller degree, which gives its place in the stable
 //   valence sort (src/rcm_cpu.cpp:94-96).
+//   Wide levels. Above 24,576 slots or so a level is work for the whole GPU, and a matrix with enough left is given up
+//   (SoloGiveUp).
 //   Start search. The sweeps of SimplePeripheral::findPeripheral (src/simple_peripheral.cpp:44-141) and the order run
 //   in the same launch: the rule on the last 32 discovered nodes needs only the queue and the level boundaries.
 #pragma once
@@ -442,8 +444,9 @@ __device__ __forceinline__ void pass_beat(uint32_t* beat, uint64_t t0) {
 }
 
 // One matrix: the start search (SOLO_SEARCH), the order from `start` (SOLO_RUN), or both (SOLO_ORDER; `start` >= 0
-// skips the search), or ERR_CAPACITY when it is given up. From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is first run as a CM pass: when its
-// eccentricity equals the previous sweep's it is the confirming sweep and the result. The results go to *ctl.
+// skips the search), or ERR_CAPACITY when it is given up. From sweep `speculate` on (0: never) a sweep of SOLO_ORDER is
+// first run as a CM pass: when its eccentricity equals the previous sweep's it is the confirming sweep and the result. The
+// results go to *ctl.
 template <class G>
 __device__ __forceinline__ void solo_matrix(const SoloJob& J, SoloSmem<G>& sm, int32_t mode, int32_t start,
                                             int32_t speculate, SoloGiveUp give, Control* ctl) {

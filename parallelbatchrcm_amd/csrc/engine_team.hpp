@@ -15,25 +15,27 @@
 //   word holds owns c -- the serial rule (src/rcm_cpu.cpp:83-92). The codes of a later pass are below those of an
 //   earlier one, so a pass needs no clearing.
 //   Order. As in engine_solo.hpp: the owned children packed in slot order, siblings placed by (degree, slot).
-//   Redistribution. When the level has outgrown its members, or left most of them idle, or grown lopsided, every member
-//   writes its children to its region of a double-buffered stage and their count to its word, and the next level's
-//   parents are split evenly. Stage entries carry the tag of the level they are parents of, so a reader that comes
-//   first polls the entry, and no writer waits for its stores before it publishes. A part that exceeds one chunk
-//   (T parents, S slots) also lives in the member's region, and is expanded chunk by chunk.
+//   Redistribution. When the level has outgrown its members or all levels before it, or left most members idle, or grown
+//   lopsided, every member writes its children to its region of a double-buffered stage and their count to its word, and
+//   the next level's parents are split evenly. Stage entries carry the tag of the level they are parents of, so a reader
+//   that comes first polls the entry, and a writer publishes before it stores -- but for a part without children, whose
+//   word may end the pass. A part that exceeds one chunk (T parents, S slots) also lives in the member's region, and is
+//   expanded chunk by chunk.
 //   Alone. Until the first redistribution of a pass its leader is the only member, and meets nobody: while the level is
 //   narrow and the matrix has at most kTeamLocalN rows it claims in LDS, as engine_solo.hpp does (1.4 us a level against
 //   3.2 through the claim words), and only stores the claims of what it places.
 //   Membership. The workgroups that have started, in order of arrival; the first leads. Nobody waits for a workgroup
 //   that has not started, so a launch ends whatever else runs on the GPU; the workgroups a level does without watch
 //   the leader's word for the next redistribution.
-// Measured on MI355X, whole calls, the batch engine before and a team after: one order of the 128^3 stencil 4.09 and 2.29
-// ms (379 levels), start search and order of a geometric graph of 1M points 22.9 and 13.3 to 14.2 ms, of a 48^3 stencil 3.4 and
-// 1.9 ms.
+// Measured on MI355X, whole calls, the batch engine before and a team after: one order of the 128^3 stencil 4.09 and 2.31 to
+// 2.38 ms (379 levels), start search and order of a geometric graph of 1M points 23.0 and 14.2 to 14.8 ms, of a 48^3 stencil
+// 3.4 and 1.9 ms.
 #pragma once
 #include "engine_solo.hpp"
 
 // Where the tests hold a member up: between its word and its look at the others' (0 a meeting, 1 a redistribution),
-// before a workgroup that joins reads the leader's record (2), and before a level's queue entries are stored (3). Nothing here relies on members keeping pace.
+// before a workgroup that joins reads the leader's record (2), and before a level's queue entries are stored (3).
+// Nothing here relies on members keeping pace.
 #ifndef RCM_TEAM_LINGER
 #define RCM_TEAM_LINGER(where, member, tag)
 #endif
@@ -226,7 +228,8 @@ __device__ __forceinline__ bool team_meet(const TeamArgs& a, TeamSmem<G>& sm, co
   TeamWords r;
   if (wave_id() == 0) {
     if (lane_id() == 0)
-      st_sync(team_word(a, sm.g, (int)(lv.tag & 1u)), ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
+      st_sync(team_word(a, sm.g, (int)(lv.tag & 1u)),
+              ((uint64_t)lv.tag << 32) | (uint64_t)((here << kTeamNodeBits) | (uint32_t)lv.cnt));
     RCM_TEAM_LINGER(0, sm.g, lv.tag);
     const uint32_t v = team_poll(a, sm, (int)(lv.tag & 1u), lv.tag, lv.members, r);
     if (lane_id() == 0) sm.verdict = v;
@@ -643,7 +646,8 @@ __device__ __forceinline__ bool team_chunk_local(const TeamArgs& a, TeamSmem<G>&
   return team_place<G, KN, true>(a, sm, lv, 0, lv.cnt, lv.E, s, true, true, nx);
 }
 template <class G, int KN>
-__device__ __forceinline__ bool team_chunk(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here, TeamNext& nx) {
+__device__ __forceinline__ bool team_chunk(const TeamArgs& a, TeamSmem<G>& sm, const TeamLevel& lv, uint32_t here,
+                                           TeamNext& nx) {
   TeamSlots<KN> s;
   team_expand<G, KN>(a, sm, 0, lv.E, s);
   team_claim<G, KN>(a, lv, lv.E, s);
@@ -814,8 +818,8 @@ __device__ __forceinline__ void team_help(const TeamArgs& a, TeamSmem<G>& sm) {
 // The leader's pass from `start`: returns the nodes placed; *levels the index of the last level, *last its first queue
 // position. *stop when the launch is over.
 template <class G>
-__device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm, int32_t start, bool bfs, uint32_t epoch, uint32_t* tag, int32_t* levels, int32_t* last,
-                                             bool* stop) {
+__device__ __forceinline__ int32_t team_pass(const TeamArgs& a, TeamSmem<G>& sm, int32_t start, bool bfs, uint32_t epoch,
+                                             uint32_t* tag, int32_t* levels, int32_t* last, bool* stop) {
   const int tid = threadIdx.x;
   const uint32_t rb = (uint32_t)a.row_ptr[start], d = (uint32_t)a.row_ptr[start + 1] - rb;
   const uint64_t base = (uint64_t)epoch << 56;

@@ -134,6 +134,9 @@ bool has_hub(int32_t n, uint32_t maxrow) { return maxrow > (uint32_t)kSoloMaxRow
 
 // The team engine (engine_team.hpp): up to kTeamMax workgroups on the matrix of a context, beyond kCtxSolo rows.
 using TeamG = TeamGeo<1024, 4096>;
+// Against the batch engine a team gains on all of them: one order of 2D stencils of 1000 x 1000, 300 x 1000, 60 x 6000 and
+// 12 x 60000 rows 32.2, 11.4, 35.3 and 335 ms by the batch engine, 9.7, 6.4, 28.6 and 221 by a team (beyond kTeamLocalN rows
+// too, where its leader has no bitmap), of a geometric graph of 300k rows of 7 entries 6.3 and 4.3.
 // Start search and order in ms, one workgroup against the team: 32k rows, 2D 1.67 / 2.56, 3D 1.25 / 1.16, geometric of
 // mean degree 13 2.19 / 2.00; 64k, 2.95 / 4.25, 2.42 / 1.46, 4.16 / 2.96; 128k, 5.09 / 6.9, 4.6 / 2.09, 8.2 / 4.3. The
 // wider the levels the more a team gives, the narrow ones its leader takes on its own at 1.5 times one workgroup's time.
@@ -988,10 +991,10 @@ bool batch_solo(const rcm_batch* b) {
 
 // Whether a set gains from its split. The engines run one after the other, and a matrix of the rest with many levels keeps
 // the batch engine busy for as long as its levels take, with the others or without: only beside kSoloShare times its rows,
-// or with few levels (a hub row, or given up by one workgroup), does the rest end early enough. MI355X, ms a run by the batch engine alone and by both:
-// 5, 30 and 60 matrices of up to 60k rows beside a 2D stencil of 152k rows 6.7 / 7.3, 6.8 / 7.9, 6.9 / 8.0; beside a
-// geometric graph of 150k 3.86 / 4.50, 3.86 / 4.96, 3.92 / 5.06; beside an R-MAT graph of 2^16 rows 1.27 / 1.09, 3.42 /
-// 1.58, 3.87 / 1.61, of 2^13 rows 1.27 / 0.87, 3.40 / 1.36, 3.83 / 1.42.
+// or with few levels (a hub row, or given up by one workgroup), does the rest end early enough. MI355X, ms a run
+// by the batch engine alone and by both: 5, 30 and 60 matrices of up to 60k rows beside a 2D stencil of 152k rows 6.7 / 7.3,
+// 6.8 / 7.9, 6.9 / 8.0; beside a geometric graph of 150k 3.86 / 4.50, 3.86 / 4.96, 3.92 / 5.06; beside an R-MAT graph of
+// 2^16 rows 1.27 / 1.09, 3.42 / 1.58, 3.87 / 1.61, of 2^13 rows 1.27 / 0.87, 3.40 / 1.36, 3.83 / 1.42.
 bool solo_pays(const rcm_batch* b) {
   const int64_t company = (b->total_n - b->rest_rows) / kSoloShare;
   for (int32_t k : b->rest)

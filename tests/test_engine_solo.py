@@ -103,7 +103,8 @@ def test_emulated_give_up(mode):
 
     mats = [CASES["random1500"](), CASES["path300"](), CASES["star64"]()]
     nnz = [len(ci) for _, ci in mats]
-    for level, spare, gave in ((2000, 1000, [True, False, False]), (2000, nnz[0], [False] * 3), (300, 60, [True, False, False])):
+    for level, spare, wide in ((2000, 1000, True), (2000, nnz[0], False), (300, 60, True)):
+        gave = [wide, False, False]
         perms, info = E.run_solo(mats, [0] * 3 if mode == 0 else [-1] * 3, workers=2, mode=mode, give_up=(level, spare))
         assert (info[:, 0] == 2).tolist() == gave, (level, spare)
         for k, (rp, ci) in enumerate(mats):
