@@ -139,6 +139,12 @@ void emu_team_linger(int where, int member, int phase) {
   emu_linger[2] = phase;
 }
 
+// A clock that every look moves on by `step` ticks, from 0 (step 0: the time again). Returns what the one before came to.
+uint64_t emu_clock(uint64_t step) {
+  emu::clock_step = step;
+  return emu::clock_ticks.exchange(0);
+}
+
 // Orders one matrix with a team of `workers` workgroups (engine_team.hpp). wide: parents per member wanted, as a power of
 // two. alone: slots of a level its leader takes on its own. cap: entries of a stage region. tag0 0 starts from memory that
 // holds anything. geo: 0 = workgroups of one wave (256 slots), 1 = of two waves (512 slots). info = error, placed, levels,

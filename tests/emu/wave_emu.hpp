@@ -260,7 +260,12 @@ inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int row_mask,
 #define __builtin_amdgcn_fence(order, scope) \
   (std::atomic_thread_fence(std::memory_order_seq_cst), emu::ctx.wave->barrier())
 inline void __builtin_amdgcn_s_sleep(int) { std::this_thread::yield(); }
+// The clock, in ticks of 10 ns; while emu::clock_step is not 0, one that every look moves on by so many.
+namespace emu {
+inline std::atomic<uint64_t> clock_step{0}, clock_ticks{0};
+}
 inline uint64_t __builtin_amdgcn_s_memrealtime() {
+  if (const uint64_t step = emu::clock_step) return emu::clock_ticks += step;
   return (uint64_t)std::chrono::duration_cast<std::chrono::nanoseconds>(
              std::chrono::steady_clock::now().time_since_epoch()).count() / 10ull;
 }

@@ -232,6 +232,15 @@ def run_solo(mats, starts, workers=2, mode=0, speculate=3, geo=0, timeout_s=120.
     return [perm[off[k]:off[k + 1]] for k in range(len(mats))], info
 
 
+def clock(step):
+    """The emulated engines' clock for run_solo and run_team: every look moves it on by `step` s, from 0 (0: the time
+    again). Returns the seconds that the one before came to."""
+    L = lib("solo")
+    L.emu_clock.restype = C.c_uint64
+    L.emu_clock.argtypes = [C.c_uint64]
+    return L.emu_clock(round(step * 1e8)) / 1e8
+
+
 def run_team(rp, ci, start, workers=3, mode=0, speculate=3, wide=2, alone=0, cap=4096, tag0=1000,
              linger=(-1, -1, -1), timeout_s=120.0, geo=0):
     """A team of workgroups on one matrix (engine_team.hpp). Returns (perm, info) with info as run_solo's. linger: where,
